@@ -420,6 +420,251 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE))) 
   }
 }
 
+// ---------------------------------------------------------------------------
+// The scan of few lanes.  With a wave lane per channel and 16 or 32 states in
+// its registers, one 105M lane is 192 waves: most SIMDs idle while each step
+// of the busy ones takes 16 states' arithmetic.  Here a wave lane owns one
+// channel and one of the four partial sums of a readout group (states
+// p, p + 4, ... of the group's 4 * M), so one lane is 768 waves (d_state 256,
+// M = 4) or 64 (the small model, M = 2) with M states' arithmetic per step.
+// The partial sums meet inside the quad of neighbouring wave lanes by DPP,
+// the groups of a state block in LDS, in the same order as above
+// ((p0 + p1) + (p2 + p3), then group after group): the same operations on
+// the same operands, so the same bits.
+//
+// Bound: one wave per SIMD issues a step's chain of about 28 instructions
+// every ~245 cycles (105M, one lane; ~150 at the rate one wave can issue
+// them), against 6 issue slots per state and step at full occupancy.  A
+// workgroup's four waves own CH channels and NG = 64 / CH groups, so 192
+// workgroups spread a 105M lane over the CUs.  delta and u = delta * x are
+// staged as pairs; B and C as four planes (states j with j mod 4 = p), so a
+// lane's M values are one LDS read and the staging stores of consecutive
+// threads are consecutive; the plane pitch puts the planes' and groups'
+// reads of a wave in distinct banks.  Each lane of a quad keeps the sum of
+// one of four steps, so four steps are stored by one LDS write.  Measured
+// against the scan above, prefill of T = 512: 105M bf16 one lane 3.95 -> 1.39
+// ms (scan 265 -> 52 us per layer), four lanes 5.86 -> 2.68, eight 6.64 ->
+// 4.42; small fp32 model one lane 0.387 -> 0.244 (scan 110 -> 40 us).
+template <int M>
+constexpr int quad_block_groups() { return M == 4 ? 8 : 4; }  // readout groups per state block (ssm_state_blocks)
+
+template <int M, int CH, bool VEC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void ssm_quad_kernel(SsmArgs a) {
+  constexpr int NW = 4, NT = NW * 64, TC = 16;
+  constexpr int GS = 4 * M, GW = 16 / CH, NG = NW * GW, SB = NG * GS;
+  constexpr int NGB = quad_block_groups<M>(), NB = NG / NGB;  // state blocks per workgroup
+  static_assert(NB * NGB == NG, "a workgroup covers whole state blocks");
+  constexpr int PL = SB / 4 + (M == 4 ? 8 : 4);   // plane pitch (floats)
+  constexpr int NBC = TC * SB / 4 / NT;           // float4s of B (and C) staged per thread
+  static_assert(TC % 8 == 0 && NBC * NT * 4 == TC * SB && TC * CH <= NT, "whole staging rounds");
+  typedef float vm_t __attribute__((ext_vector_type(M)));
+  __shared__ __attribute__((aligned(16))) float2 sU[2][TC][CH];
+  __shared__ __attribute__((aligned(16))) float sB[2][TC][4 * PL];
+  __shared__ __attribute__((aligned(16))) float sC[2][TC][4 * PL];
+  __shared__ float sY[2][NG][TC][CH];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int p = lane & 3, ch = (lane >> 2) & (CH - 1), g = wave * GW + lane / (4 * CH);
+  const int i0 = blockIdx.x * CH, b = blockIdx.y, jb = blockIdx.z * SB;
+  const int i = i0 + ch, jw = jb + g * GS + p;
+  const bool ivalid = i < a.d;
+  const int T = a.T, d = a.d, s = a.s;
+  const size_t row0 = (size_t)b * T;
+
+  float h[M], r2[M];
+  float* carry = a.carry + (size_t)b * a.carry_stride;
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    const int j = jw + 4 * m;
+    const bool ok = ivalid && j < s;
+    h[m] = ok ? carry[carry_at(j, i, d, s)] : 0.0f;
+    r2[m] = ok ? a.rates2[(size_t)j * d + i] : 0.0f;
+  }
+
+  // This thread's step and channel of a chunk (threads past TC * CH repeat
+  // the first ones' loads and store nothing).
+  const int ett = tid / CH % TC, eci = tid % CH;
+  // Offset of row t of this lane in a matrix of leading dimension ld.
+  const uint32_t r0 = (uint32_t)row0;
+  auto row = [&](int t, int ld) { return (size_t)(r0 + (uint32_t)t) * (uint32_t)ld; };
+  // The staged loads are unguarded (a guarded load's zero fill waits for the
+  // load before it): a chunk whose channels, states and steps are all in
+  // range reads at running pointers, any other at clamped addresses, masked
+  // on the way to LDS.
+  const bool whole = VEC && i0 + CH <= d && jb + SB <= s;  // uniform
+  const float* pdp = a.delta + row(min(ett, T - 1), a.ld_delta) + min(i0 + eci, d - 1);
+  const float* pxp = a.xn + row(min(ett, T - 1), a.ld_x) + min(i0 + eci, d - 1);
+  const float *pbp[NBC], *pcp[NBC];
+#pragma unroll
+  for (int k = 0; k < NBC; ++k) {
+    const int e = tid + NT * k, t = e / (SB / 4), j = jb + 4 * (e % (SB / 4));
+    pbp[k] = a.bproj + row(t, a.ld_b) + j;
+    pcp[k] = a.cproj + row(t, a.ld_c) + j;
+  }
+  const size_t sd = (size_t)TC * (uint32_t)a.ld_delta, sx = (size_t)TC * (uint32_t)a.ld_x,
+               sb = (size_t)TC * (uint32_t)a.ld_b, sc = (size_t)TC * (uint32_t)a.ld_c;
+  float pd, px;
+  float4 pb[NBC], pc[NBC];
+  // The chunk at t0; called for t0 = 0, TC, 2 TC, ... in order.
+  auto load = [&](int t0) {
+    if (whole && t0 + TC <= T) {
+      pd = *pdp;
+      px = *pxp;
+      pdp += sd;
+      pxp += sx;
+#pragma unroll
+      for (int k = 0; k < NBC; ++k) {
+        pb[k] = *reinterpret_cast<const float4*>(pbp[k]);
+        pc[k] = *reinterpret_cast<const float4*>(pcp[k]);
+        pbp[k] += sb;
+        pcp[k] += sc;
+      }
+      return;
+    }
+    {
+      const int t = min(t0 + ett, T - 1), gi = min(i0 + eci, d - 1);
+      pd = a.delta[row(t, a.ld_delta) + gi];
+      px = a.xn[row(t, a.ld_x) + gi];
+    }
+#pragma unroll
+    for (int k = 0; k < NBC; ++k) {
+      const int e = tid + NT * k, t = min(t0 + e / (SB / 4), T - 1), j = jb + 4 * (e % (SB / 4));
+      const float* br = a.bproj + row(t, a.ld_b);
+      const float* cr = a.cproj + row(t, a.ld_c);
+      if constexpr (VEC) {
+        pb[k] = *reinterpret_cast<const float4*>(br + min(j, s - 4));
+        pc[k] = *reinterpret_cast<const float4*>(cr + min(j, s - 4));
+      } else {
+        const int j0 = min(j, s - 1), j1 = min(j + 1, s - 1), j2 = min(j + 2, s - 1), j3 = min(j + 3, s - 1);
+        pb[k] = make_float4(br[j0], br[j1], br[j2], br[j3]);
+        pc[k] = make_float4(cr[j0], cr[j1], cr[j2], cr[j3]);
+      }
+    }
+  };
+  auto store = [&](int t0, int buf) {
+    if (!(whole && t0 + TC <= T)) {
+      const bool oku = t0 + ett < T && i0 + eci < d;
+      pd = oku ? pd : 0.0f;
+      px = oku ? px : 0.0f;
+#pragma unroll
+      for (int k = 0; k < NBC; ++k) {
+        const int e = tid + NT * k, j = jb + 4 * (e % (SB / 4));
+        const int n = t0 + e / (SB / 4) < T ? s - j : 0;  // states of this piece in range
+        pb[k].x = n > 0 ? pb[k].x : 0.0f, pc[k].x = n > 0 ? pc[k].x : 0.0f;
+        pb[k].y = n > 1 ? pb[k].y : 0.0f, pc[k].y = n > 1 ? pc[k].y : 0.0f;
+        pb[k].z = n > 2 ? pb[k].z : 0.0f, pc[k].z = n > 2 ? pc[k].z : 0.0f;
+        pb[k].w = n > 3 ? pb[k].w : 0.0f, pc[k].w = n > 3 ? pc[k].w : 0.0f;
+      }
+    }
+    if (tid < TC * CH) sU[buf][ett][eci] = make_float2(pd, pd * px);
+#pragma unroll
+    for (int k = 0; k < NBC; ++k) {
+      const int e = tid + NT * k, tt = e / (SB / 4), q = e % (SB / 4);
+      float* pB = &sB[buf][tt][q];
+      float* pC = &sC[buf][tt][q];
+      pB[0] = pb[k].x, pB[PL] = pb[k].y, pB[2 * PL] = pb[k].z, pB[3 * PL] = pb[k].w;
+      pC[0] = pc[k].x, pC[PL] = pc[k].y, pC[2 * PL] = pc[k].z, pC[3 * PL] = pc[k].w;
+    }
+  };
+  const int nz = (s + NGB * GS - 1) / (NGB * GS);  // ssm_state_blocks(s)
+  // The readout of the chunk at t0 from its groups' sums.
+  auto finish = [&](int t0, int buf) {
+    const int t = t0 + ett, gi = i0 + eci;
+    if (tid < TC * CH && t < T && gi < d) {
+      float v = 0.0f;
+#pragma unroll
+      for (int blk = 0; blk < NB; ++blk) {
+        const int z = blockIdx.z * NB + blk;
+        if (blk > 0 && z >= nz) break;
+        float bv = sY[buf][blk * NGB][ett][eci];
+#pragma unroll
+        for (int q = 1; q < NGB; ++q) bv += sY[buf][blk * NGB + q][ett][eci];
+        if (a.y_part) a.y_part[(size_t)z * a.rows * d + row(t, d) + gi] = bv;
+        v = blk == 0 ? bv : v + bv;
+      }
+      if (!a.y_part) {
+        if (gridDim.z > 1)
+          atomicAdd(a.y + row(t, a.ld_y) + gi, v);
+        else
+          a.y[row(t, a.ld_y) + gi] = v;
+      }
+    }
+  };
+  // Four steps' inputs in registers, read from LDS a group ahead of their use.
+  struct Quad {
+    float2 u[4];
+    vm_t b[4], c[4];
+  };
+  auto read = [&](Quad& q, int buf, int t4) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      q.u[k] = sU[buf][t4 + k][ch];
+      q.b[k] = *reinterpret_cast<const vm_t*>(&sB[buf][t4 + k][p * PL + g * M]);
+      q.c[k] = *reinterpret_cast<const vm_t*>(&sC[buf][t4 + k][p * PL + g * M]);
+    }
+  };
+  auto steps = [&](const Quad& q, int buf, int t4) {
+    float ab[4][M], ub[4][M], sum[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        ab[k][m] = __builtin_amdgcn_exp2f(q.u[k].x * r2[m]);
+        ub[k][m] = q.u[k].y * q.b[k][m];
+      }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      float yp = 0.0f;
+#pragma unroll
+      for (int m = 0; m < M; ++m) h[m] = fmaf(ab[k][m], h[m], ub[k][m]);
+#pragma unroll
+      for (int m = 0; m < M; ++m) yp = fmaf(h[m], q.c[k][m], yp);
+      sum[k] = yp;
+    }
+    // (p0 + p1) + (p2 + p3) over the quad: quad_perm [1,0,3,2], [2,3,0,1].
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      sum[k] += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(sum[k]), 0xB1, 0xF, 0xF, true));
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      sum[k] += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(sum[k]), 0x4E, 0xF, 0xF, true));
+    sY[buf][g][t4 + p][ch] = p < 2 ? (p == 0 ? sum[0] : sum[1]) : (p == 2 ? sum[2] : sum[3]);
+  };
+
+  // Chunk c computes from buffer c & 1 while the next chunk's inputs move
+  // from registers to the other buffer, the one after that is loaded, and the
+  // previous chunk's readout is finished: one barrier per chunk.
+  load(0);
+  store(0, 0);
+  load(TC);
+  __syncthreads();
+  int buf = 0;
+  for (int t0 = 0; t0 < T; t0 += TC, buf ^= 1) {
+    Quad qa, qb;
+    read(qa, buf, 0);
+    store(t0 + TC, buf ^ 1);
+    if (t0 > 0) finish(t0 - TC, buf ^ 1);  // before the loads: their waits count what was issued after them
+    load(t0 + 2 * TC);
+    // Steps past T have delta = u = 0 and leave h as it is.
+    const int n = min(TC, T - t0);
+    for (int t8 = 0; t8 < n; t8 += 8) {
+      read(qb, buf, t8 + 4);
+      __builtin_amdgcn_sched_barrier(0);
+      steps(qa, buf, t8);
+      read(qa, buf, (t8 + 8) & (TC - 1));
+      __builtin_amdgcn_sched_barrier(0);
+      steps(qb, buf, t8 + 4);
+    }
+    __syncthreads();
+  }
+  finish((T - 1) / TC * TC, buf ^ 1);
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    const int j = jw + 4 * m;
+    if (ivalid && j < s) carry[carry_at(j, i, d, s)] = h[m];
+  }
+}
+
 // y = sum over state blocks of the partial readouts, in block order.
 __global__ void ssm_reduce_kernel(const float* __restrict__ part, int nz, size_t rows, int d,
                                   float* __restrict__ y, int ld_y) {
@@ -447,14 +692,33 @@ bool ssm_needs_zeroed_y(int s) { return ssm_state_blocks(s) == 2; }
 // twice the waves, half the registers per lane) keeps the SIMDs fed.
 constexpr long kScanFullGrid = 768;
 
+// The few-lane scan (ssm_quad_kernel) up to this many of its workgroups
+// beside another lane group, twice as many alone with M = 4.  Prefill of the
+// 105M model, T = 512, old / quad scan: in two groups, 16 lanes (1536
+// workgroups a group) 7.65 / 7.37 ms, 18 lanes 7.83 / 8.17, 24 lanes 9.28 /
+// 9.93; serialised scan stage, 16 lanes (3072) 4.71 / 4.20 ms, 18 lanes
+// 4.73 / 4.82.  Small model, scan stage: 64 lanes x 256 (1024) 0.120 / 0.098
+// ms, 128 x 128 (2048) 0.082 / 0.098.
+constexpr int kQuadChannels = 8;
+constexpr long kQuadMax = 1536;
+
 // Lanes per decode-step workgroup (they share the rate loads).
 #ifndef PSSA_SSM_STEP_LPB
 #define PSSA_SSM_STEP_LPB 4
 #endif
 
+// The few-lane scan's grid: kQuadChannels channels and 128 (J = 32) or 64
+// (J = 8) states per workgroup.
+template <int J>
+static long quad_workgroups(const SsmArgs& a, dim3& grid) {
+  constexpr int SB = J == 32 ? 128 : 64;
+  grid = dim3((a.d + kQuadChannels - 1) / kQuadChannels, a.lanes, (a.s + SB - 1) / SB);
+  return (long)grid.x * grid.y * grid.z;
+}
+
 template <int J>
 static void launch_j(hipStream_t stream, const SsmArgs& a, bool mat) {
-  dim3 grid((a.d + 63) / 64, a.lanes, (a.s + 4 * J - 1) / (4 * J));
+  dim3 grid((a.d + 63) / 64, a.lanes, (a.s + 4 * J - 1) / (4 * J)), qgrid;
   if (mat) {
     ssm_materialize_kernel<J, true><<<grid, 256, 0, stream>>>(a);
   } else if (a.T == 1) {
@@ -471,6 +735,14 @@ static void launch_j(hipStream_t stream, const SsmArgs& a, bool mat) {
     }
   } else if (a.T < SSM_TC) {
     ssm_materialize_kernel<J, false><<<grid, 256, 0, stream>>>(a);
+  } else if (J >= 8 && quad_workgroups<J>(a, qgrid) <= (J == 32 && !a.concurrent ? 2 : 1) * kQuadMax) {
+    constexpr int M = J == 32 ? 4 : 2;
+    const bool vec = a.s % 4 == 0 && a.ld_b % 4 == 0 && a.ld_c % 4 == 0 && ((uintptr_t)a.bproj & 15) == 0 &&
+                     ((uintptr_t)a.cproj & 15) == 0;
+    if (vec)
+      ssm_quad_kernel<M, kQuadChannels, true><<<qgrid, 256, 0, stream>>>(a);
+    else
+      ssm_quad_kernel<M, kQuadChannels, false><<<qgrid, 256, 0, stream>>>(a);
   } else if constexpr (J == 32) {
     if ((long)grid.x * grid.y * grid.z < kScanFullGrid && !a.concurrent)
       ssm_scan_kernel<16, 8, 4><<<grid, 512, 0, stream>>>(a);

@@ -220,6 +220,26 @@ def test_ssm_random_shapes(hip, L, dm, ds):
     assert rel_err(fin, rs[L * dm * ds:]) < 1e-5
 
 
+@pytest.mark.parametrize("dm,ds", [(24, 256), (70, 130), (8, 128), (24, 64), (9, 33), (17, 40)])
+def test_ssm_few_lane_scan_equals_general_kernel_bitwise(hip, dm, ds):
+    """The few-lane scan around its chunk (16 steps) and channel-block (8)
+    edges against the step-by-step kernel that also writes the tape: the same
+    operations in the same order, so every readout and final state bit."""
+    for L in (4, 5, 8, 15, 16, 17, 31, 32, 33, 50):
+        say("ssm few-lane", L, dm, ds)
+        rng = np.random.default_rng(L + dm + ds)
+        delta = np.float32(np.log1p(np.exp(rng.standard_normal(L * dm))))
+        b = rng.standard_normal(L * ds).astype(np.float32) * 0.3
+        x = rng.standard_normal(L * dm).astype(np.float32)
+        rates = -np.float32(np.log1p(np.exp(rng.standard_normal(dm * ds))))
+        c = rng.standard_normal(L * ds).astype(np.float32) * 0.3
+        init = rng.standard_normal(dm * ds).astype(np.float32) * 0.1
+        _, _, _, y, fin = hip.ssm_forward(delta, b, x, rates, c, init, L, dm, ds, materialize=False)
+        _, _, _, y_ref, fin_ref = hip.ssm_forward(delta, b, x, rates, c, init, L, dm, ds)
+        np.testing.assert_array_equal(y, y_ref)
+        np.testing.assert_array_equal(fin, fin_ref)
+
+
 def test_ssm_softplus_and_rate_tails(hip):
     """tests/numeric_recurrence.rs:48-137: tiny delta from the softplus tail and a
     huge delta against a tiny rate keep the state finite and exact to ~1e-6."""
