@@ -1242,75 +1242,93 @@ int pssa_hip_forward_inference(pssa_hip_lanes* L, const uint32_t* ids, size_t n_
   return pssa_hip_prefill(L, ids, n_lanes, 1, logits, logits_len, err, err_len);
 }
 
+// Lanes of their own lengths as the device runs them: one pass over all
+// rows, lane after lane, each stage once per layer (time segments of the lanes
+// still running cost a pass of small launches per distinct length).  Longest
+// lanes first, dealt to the concurrent lane groups of a prefill.
+struct RaggedPlan {
+  std::vector<size_t> order;  // launch lane -> index into the caller's lengths
+  std::vector<size_t> row;    // first row of each launch lane in the packed rows
+  std::vector<uint32_t> meta; // spans, last rows, positions: the upload
+  pssa::RaggedRows rows;
+};
+
+// lens[i] tokens on lane lane_of[i] (0: does not run); tokens > 0.
+static void plan_ragged(const pssa_hip_lanes* L, const std::vector<uint64_t>& lens, const std::vector<uint64_t>& lane_of,
+                        RaggedPlan& p) {
+  std::vector<size_t> sorted;
+  for (size_t i = 0; i < lens.size(); ++i)
+    if (lens[i] > 0) sorted.push_back(i);
+  std::stable_sort(sorted.begin(), sorted.end(), [&](size_t a, size_t b) { return lens[a] > lens[b]; });
+  pssa::RaggedRows& r = p.rows;
+  r.max_len = lens[sorted[0]];
+  r.groups = pssa::prefill_lane_groups(L, sorted.size(), r.max_len);
+  for (int g = 0; g < r.groups; ++g) {
+    r.lane0[g] = p.order.size();
+    for (size_t i = 0; i < sorted.size(); ++i)
+      if (r.groups == 1 || ((i & 3) == 0 || (i & 3) == 3) == (g == 0)) p.order.push_back(sorted[i]);
+  }
+  r.lane0[r.groups] = p.order.size();
+  size_t row = 0;
+  for (int g = 0; g < r.groups; ++g) {
+    r.row0[g] = row;
+    for (size_t l = r.lane0[g]; l < r.lane0[g + 1]; ++l) {
+      p.row.push_back(row);
+      p.meta.push_back((uint32_t)(row - r.row0[g]));
+      p.meta.push_back((uint32_t)lens[p.order[l]]);
+      p.meta.push_back((uint32_t)lane_of[p.order[l]]);
+      row += lens[p.order[l]];
+    }
+  }
+  r.row0[r.groups] = row;
+}
+
+// Copies the plan's metadata to the device (p.meta must stay until the
+// stream is synchronised) and points the rows at it.
+static Status upload_plan(pssa_hip_lanes* L, RaggedPlan& p, size_t n_last, size_t n_pos) {
+  if (!L->row_meta.p) PSSA_RETURN_IF(L->row_meta.alloc((4 * L->lanes + L->max_tokens) * 4));
+  const size_t n_span = 3 * p.order.size();
+  PSSA_HIP_TRY(hipMemcpyAsync(L->row_meta.p, p.meta.data(), p.meta.size() * 4, hipMemcpyHostToDevice, L->ctx->stream));
+  p.rows.spans = L->row_meta.as<int>();
+  if (n_last) p.rows.last = L->row_meta.as<uint32_t>() + n_span;
+  if (n_pos) p.rows.pos = L->row_meta.as<uint32_t>() + n_span + n_last;
+  p.rows.n_lanes = n_last;
+  return Status::Ok();
+}
+
 // Ragged prefill with L->ctx->mu held: lane i consumes lens[i] ids (0 leaves
 // the lane untouched), packed in lane order.  Each lane's last-token logits
 // end in row i of lanes->logits (lanes of length 0: undefined).
 static Status ragged_locked(pssa_hip_lanes* L, const uint32_t* ids, const uint64_t* lens, size_t n_lanes) {
-  const pssa_hip_config& c = L->model->cfg;
-  const size_t V = c.d_vocab;
-  const hipStream_t st = L->ctx->stream;
-  const size_t cw = c.depth * L->loops * c.d_latent * c.d_state;
   size_t tokens = 0;
-  for (size_t i = 0; i < n_lanes; ++i) tokens += lens[i];
+  std::vector<size_t> offset(n_lanes);
+  std::vector<uint64_t> lens_v(lens, lens + n_lanes), lane_of(n_lanes);
+  for (size_t i = 0; i < n_lanes; ++i) {
+    offset[i] = tokens;
+    tokens += lens[i];
+    lane_of[i] = i;
+  }
   if (tokens == 0) return Status::Ok();
-  // Lanes in order of decreasing length, so that the lanes still running
-  // are always a prefix (the segments of pssa_hip_batch_forward).
-  std::vector<size_t> offset(n_lanes), order(n_lanes);
-  for (size_t i = 0, o = 0; i < n_lanes; o += lens[i], ++i) offset[i] = o;
-  for (size_t i = 0; i < n_lanes; ++i) order[i] = i;
-  std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return lens[a] > lens[b]; });
-  size_t n_active = 0;
-  while (n_active < n_lanes && lens[order[n_active]] > 0) ++n_active;
-  bool identity = true;
-  for (size_t i = 0; i < n_active; ++i) identity &= order[i] == i;
-  float* carry = L->carry.as<float>();
-  float* work = carry;
-  if (!identity) {
-    if (!L->carry_work.p) PSSA_RETURN_IF(L->carry_work.alloc(L->lanes * cw * 4));
-    work = L->carry_work.as<float>();
-    for (size_t i = 0; i < n_active; ++i)
-      PSSA_HIP_TRY(hipMemcpyAsync(work + i * cw, carry + order[i] * cw, cw * 4, hipMemcpyDeviceToDevice, st));
-  }
+  RaggedPlan p;
+  plan_ragged(L, lens_v, lane_of, p);
   std::vector<uint32_t> ids_h(tokens);
-  struct Segment {
-    size_t T, n_active, row;
-  };
-  std::vector<Segment> segs;
-  size_t t0 = 0, row = 0;
-  while (n_active > 0) {
-    const size_t t1 = lens[order[n_active - 1]], T = t1 - t0;
-    for (size_t i = 0; i < n_active; ++i)
-      for (size_t t = 0; t < T; ++t) ids_h[row + i * T + t] = ids[offset[order[i]] + t0 + t];
-    segs.push_back({T, n_active, row});
-    row += n_active * T;
-    t0 = t1;
-    while (n_active > 0 && lens[order[n_active - 1]] == t1) --n_active;
+  std::vector<uint32_t> last(n_lanes, ~0u);
+  bool hybrid = false;
+  for (const pssa::DevBlock& B : L->model->blocks) hybrid |= B.hybrid;
+  for (size_t l = 0; l < p.order.size(); ++l) {
+    const size_t i = p.order[l];
+    std::memcpy(&ids_h[p.row[l]], ids + offset[i], lens[i] * 4);
+    last[i] = (uint32_t)(p.row[l] + lens[i] - 1);
   }
-  PSSA_HIP_TRY(hipMemcpyAsync(L->ids.p, ids_h.data(), tokens * 4, hipMemcpyHostToDevice, st));
-  // Row i of every segment is lane order[i] (its penalty window).
-  std::vector<int> map_h(n_lanes);
-  for (size_t i = 0; i < n_lanes; ++i) map_h[i] = (int)order[i];
-  DevBuf dmap, lg;
-  PSSA_RETURN_IF(upload(dmap, map_h.data(), n_lanes * 4, st));
-  for (const Segment& sg : segs) {
-    pssa::TrainRows rows;
-    rows.ids = L->ids.as<uint32_t>() + sg.row;
-    rows.carry = work;
-    PSSA_RETURN_IF(pssa::run_prefill_segment(L, sg.n_active, sg.T, rows, dmap.as<int>()));
-  }
-  // Each lane's last logits sit in row (its place in length order); put
-  // carries and logits back in lane order.
-  if (!identity) {
-    PSSA_RETURN_IF(lg.alloc(n_lanes * V * 4));
-    for (size_t i = 0; i < n_lanes; ++i) {
-      if (lens[order[i]] == 0) continue;
-      PSSA_HIP_TRY(hipMemcpyAsync(carry + order[i] * cw, work + i * cw, cw * 4, hipMemcpyDeviceToDevice, st));
-      PSSA_HIP_TRY(hipMemcpyAsync(lg.as<float>() + order[i] * V, L->logits.as<float>() + i * V, V * 4,
-                                  hipMemcpyDeviceToDevice, st));
-    }
-    PSSA_HIP_TRY(hipMemcpyAsync(L->logits.p, lg.p, n_lanes * V * 4, hipMemcpyDeviceToDevice, st));
-  }
-  return sync(L->ctx);  // the staging vectors and buffers above are freed at return
+  p.meta.insert(p.meta.end(), last.begin(), last.end());
+  if (hybrid)
+    for (size_t l = 0; l < p.order.size(); ++l)
+      for (size_t t = 0; t < lens[p.order[l]]; ++t) p.meta.push_back((uint32_t)t);
+  PSSA_HIP_TRY(hipMemcpyAsync(L->ids.p, ids_h.data(), tokens * 4, hipMemcpyHostToDevice, L->ctx->stream));
+  PSSA_RETURN_IF(upload_plan(L, p, n_lanes, hybrid ? tokens : 0));
+  p.rows.ids = L->ids.as<uint32_t>();
+  PSSA_RETURN_IF(pssa::run_prefill_ragged(L, p.rows));
+  return sync(L->ctx);  // the staging vectors are freed at return
 }
 
 // Ids [n_lanes, T] after the reference's rule for invalid ids (src/pssa.rs:
@@ -1457,80 +1475,50 @@ int pssa_hip_batch_forward(pssa_hip_lanes* L, const pssa_hip_sequence* seqs, siz
     }
     L->logit_lanes = 0;  // lanes->logits no longer follows a prefill
 
-    // Packed token offsets in the given order; the device works in order of
-    // decreasing length so that the lanes still running are always a prefix.
-    std::vector<size_t> offset(n_seqs), order(n_seqs);
-    for (size_t i = 0, o = 0; i < n_seqs; o += seqs[i].len, ++i) offset[i] = o;
-    for (size_t i = 0; i < n_seqs; ++i) order[i] = i;
-    std::stable_sort(order.begin(), order.end(),
-                     [&](size_t a, size_t b) { return seqs[a].len > seqs[b].len; });
-    bool identity = true;
-    for (size_t i = 0; i < n_seqs; ++i) identity &= seqs[order[i]].lane == i;
-
+    std::vector<size_t> offset(n_seqs);  // packed token offsets in the given order
+    std::vector<uint64_t> lens(n_seqs), lane_of(n_seqs);
+    for (size_t i = 0, o = 0; i < n_seqs; o += seqs[i].len, ++i) {
+      offset[i] = o;
+      lens[i] = seqs[i].len;
+      lane_of[i] = seqs[i].lane;
+    }
+    // Carries to reset, runs of neighbouring lanes in one fill.
     float* carry = L->carry.as<float>();
-    for (size_t i = 0; i < n_seqs; ++i)
-      if (seqs[i].reset) PSSA_RETURN_IF(pssa::launch_fill_zero(st, carry + seqs[i].lane * cw, cw));
-    float* work = carry;
-    if (!identity) {
-      if (!L->carry_work.p) PSSA_RETURN_IF(L->carry_work.alloc(L->lanes * cw * 4));
-      work = L->carry_work.as<float>();
-      for (size_t i = 0; i < n_seqs; ++i)
-        PSSA_HIP_TRY(hipMemcpyAsync(work + i * cw, carry + seqs[order[i]].lane * cw, cw * 4,
-                                    hipMemcpyDeviceToDevice, st));
+    std::vector<char> reset(L->lanes, 0);
+    for (size_t i = 0; i < n_seqs; ++i) reset[seqs[i].lane] = seqs[i].reset != 0;
+    for (size_t a = 0; a < L->lanes; ++a) {
+      if (!reset[a]) continue;
+      size_t e = a + 1;
+      while (e < L->lanes && reset[e]) ++e;
+      PSSA_RETURN_IF(pssa::launch_fill_zero(st, carry + a * cw, (e - a) * cw));
+      a = e;
     }
 
-    // Segments: times [t0, t1) of the n_active longest sequences.
-    struct Segment {
-      size_t t0, t1, n_active, row;
-    };
-    std::vector<Segment> segs;
+    RaggedPlan p;
+    plan_ragged(L, lens, lane_of, p);
     std::vector<uint32_t> ids_h(tokens), meta_h(2 * tokens);
-    size_t n_active = n_seqs, t0 = 0, row = 0;
-    while (n_active > 0) {
-      const size_t t1 = seqs[order[n_active - 1]].len;
-      const size_t T = t1 - t0;
-      for (size_t i = 0; i < n_active; ++i) {
-        const pssa_hip_sequence& q = seqs[order[i]];
-        for (size_t t = 0; t < T; ++t) {
-          const size_t r = row + i * T + t;
-          ids_h[r] = q.inputs[t0 + t];
-          meta_h[r] = q.targets[t0 + t];
-          meta_h[tokens + r] = (uint32_t)(offset[order[i]] + t0 + t);
-        }
-      }
-      segs.push_back({t0, t1, n_active, row});
-      row += n_active * T;
-      t0 = t1;
-      while (n_active > 0 && seqs[order[n_active - 1]].len == t1) --n_active;
+    for (size_t l = 0; l < p.order.size(); ++l) {
+      const pssa_hip_sequence& q = seqs[p.order[l]];
+      std::memcpy(&ids_h[p.row[l]], q.inputs, q.len * 4);
+      std::memcpy(&meta_h[p.row[l]], q.targets, q.len * 4);
+      for (size_t t = 0; t < q.len; ++t) meta_h[tokens + p.row[l] + t] = (uint32_t)(offset[p.order[l]] + t);
     }
     PSSA_HIP_TRY(hipMemcpyAsync(L->ids.p, ids_h.data(), tokens * 4, hipMemcpyHostToDevice, st));
     PSSA_HIP_TRY(hipMemcpyAsync(L->tok_meta.p, meta_h.data(), 2 * tokens * 4, hipMemcpyHostToDevice, st));
-    const uint32_t* dmeta = L->tok_meta.as<uint32_t>();
-    for (const Segment& sg : segs) {
-      pssa::TrainRows tr;
-      tr.ids = L->ids.as<uint32_t>() + sg.row;
-      tr.targets = dmeta + sg.row;
-      tr.index = dmeta + tokens + sg.row;
-      tr.logits = L->tok_logits.as<float>() + sg.row * V;
-      tr.loss = L->tok_loss.as<float>();
-      tr.carry = work;
-      PSSA_RETURN_IF(pssa::run_train_segment(L, sg.n_active, sg.t1 - sg.t0, tr));
-    }
-    if (!identity)
-      for (size_t i = 0; i < n_seqs; ++i)
-        PSSA_HIP_TRY(hipMemcpyAsync(carry + seqs[order[i]].lane * cw, work + i * cw, cw * 4,
-                                    hipMemcpyDeviceToDevice, st));
+    PSSA_RETURN_IF(upload_plan(L, p, 0, 0));
+    p.rows.ids = L->ids.as<uint32_t>();
+    p.rows.targets = L->tok_meta.as<uint32_t>();
+    p.rows.index = L->tok_meta.as<uint32_t>() + tokens;
+    p.rows.logits = L->tok_logits.as<float>();
+    p.rows.loss = L->tok_loss.as<float>();
+    PSSA_RETURN_IF(pssa::run_train_forward(L, p.rows));
 
     std::vector<float> loss_h(tokens);
     PSSA_HIP_TRY(hipMemcpyAsync(loss_h.data(), L->tok_loss.p, tokens * 4, hipMemcpyDeviceToHost, st));
     if (logits)
-      for (const Segment& sg : segs) {
-        const size_t T = sg.t1 - sg.t0;
-        for (size_t i = 0; i < sg.n_active; ++i)
-          PSSA_HIP_TRY(hipMemcpyAsync(logits + (offset[order[i]] + sg.t0) * V,
-                                      L->tok_logits.as<float>() + (sg.row + i * T) * V, T * V * 4,
-                                      hipMemcpyDeviceToHost, st));
-      }
+      for (size_t l = 0; l < p.order.size(); ++l)
+        PSSA_HIP_TRY(hipMemcpyAsync(logits + offset[p.order[l]] * V, L->tok_logits.as<float>() + p.row[l] * V,
+                                    lens[p.order[l]] * V * 4, hipMemcpyDeviceToHost, st));
     PSSA_RETURN_IF(sync(L->ctx));
     // The token mean in packed order, summed left to right in f32
     // (stage_logits_loss, src/gpu_batch.rs:1246-1249).
@@ -1841,7 +1829,6 @@ int pssa_hip_lanes_set_loops(pssa_hip_lanes* L, size_t loops, char* err, size_t 
     L->graph = nullptr;
     L->graph_lanes = 0;
     L->logit_lanes = 0;
-    L->carry_work = DevBuf();
     return Status::Ok();
   };
   return pssa::finish(body(), err, err_len);

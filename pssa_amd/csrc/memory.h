@@ -31,13 +31,15 @@ struct RetrieveArgs {
   // set, live slot s weighs exp((min - d_s)/tau) * hgate[s] * decay_s,
   // decay_s = (float)exp(age_s * log_lam), age_s = hage[s] + age_base
   // (+ row % age_T + 1 when age_T > 0, the bumps of a T-token prefill's
-  // earlier tokens), saturating; a read whose live weights sum to zero falls
+  // earlier tokens; row_age[row] + 1 instead with row_age set, for rows of
+  // lanes of their own lengths), saturating; a read whose live weights sum to zero falls
   // back to the unweighted softmax.  hage may be null (ages 0).
   const float* hgate = nullptr;
   const unsigned long long* hage = nullptr;
   double log_lam = 0.0;
   unsigned long long age_base = 0;
   int age_T = 0;
+  const uint32_t* row_age = nullptr;
   // Fused query product (a decode step's few-query soft read, see
   // retrieve_fuses_query): with qw set the Euclidean query of row r is
   // qa[r] . qw^T + qaux[r], qa [n, ld_qa] bf16 rows, qw [dk, qk] bf16

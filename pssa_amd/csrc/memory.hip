@@ -105,7 +105,8 @@ constexpr double kMaxRadius = 1.0 - 8.0 * (double)FLT_EPSILON;  // src/memory.rs
 __device__ __forceinline__ float hybrid_decay(const RetrieveArgs& a, int s, int n) {
   unsigned long long age = a.hage ? a.hage[s] : 0ull;
   const unsigned long long add =
-      a.age_base + (a.age_T > 0 ? (unsigned long long)(n % a.age_T) + 1ull : 0ull);
+      a.age_base + (a.row_age ? (unsigned long long)a.row_age[n] + 1ull
+                              : a.age_T > 0 ? (unsigned long long)(n % a.age_T) + 1ull : 0ull);
   age = age > ~0ull - add ? ~0ull : age + add;
   return (float)exp((double)age * a.log_lam);
 }

@@ -96,10 +96,12 @@ struct pssa_hip_lanes {
   size_t tap_lanes = 0;      // lanes of the last plastic step whose taps the buffers hold
   // Batch training forward (allocated on its first call): the fp32 scaled
   // logits of every token row [max_tokens, V], each row's target id and
-  // packed token index [2, max_tokens], the per-token losses in packed order
-  // [max_tokens], and a carry workspace [lanes, depth, d*s] for sequences
-  // whose lanes are not 0..n-1 in length order.
-  pssa::DevBuf tok_logits, tok_meta, tok_loss, carry_work;
+  // packed token index [2, max_tokens], and the per-token losses in packed
+  // order [max_tokens].
+  pssa::DevBuf tok_logits, tok_meta, tok_loss;
+  // Spans, last rows and positions of a ragged call (RaggedRows), allocated
+  // on the first one: [4 * lanes + max_tokens] u32.
+  pssa::DevBuf row_meta;
   // Repetition-penalty window (sample(), src/inference.rs:113-121): per lane
   // a ring of the last kHist consumed ids (prompt and generated), its fill
   // count and next position; the penalty (1 = off) and a flag the greedy
@@ -173,30 +175,42 @@ namespace pssa {
 // (a decode step leaves that to the greedy choice, which appends the token
 // it consumed).
 Status run_prefill(pssa_hip_lanes* L, size_t n_lanes, size_t T, bool taps = false, bool append = true);
-// Rows of one segment of a ragged prefill or training forward: n_lanes
-// lanes of T tokens.  Every pointer addresses the segment's first row
-// (lane).  With `logits` null only each lane's last-token logits are
-// computed, into lanes->logits rows 0..n_lanes-1.
-struct TrainRows {
-  const uint32_t* ids = nullptr;      // [n_lanes * T] input ids
-  const uint32_t* targets = nullptr;  // [n_lanes * T] target ids
-  const uint32_t* index = nullptr;    // [n_lanes * T] packed token index of each row
-  float* logits = nullptr;            // [n_lanes * T, V] scaled logits
-  float* loss = nullptr;              // per-token losses, indexed by `index`
-  float* carry = nullptr;             // [n_lanes, depth, d*s] carries, advanced in place
+// Concurrent lane groups (1 or 2) of a prefill of these lanes.
+int prefill_lane_groups(const pssa_hip_lanes* L, size_t n_lanes, size_t max_len);
+// Lanes of their own lengths (a ragged prefill or training forward), packed
+// lane after lane into rows.  The lanes form one or two groups (concurrent
+// lane groups); group g's lanes are launch lanes lane0[g] .. and its rows
+// row0[g] .. .  Device pointers unless noted.
+struct RaggedRows {
+  int groups = 1;
+  size_t lane0[3] = {}, row0[3] = {};  // prefix sums over the groups (host)
+  size_t max_len = 0;                  // the longest lane (host)
+  const uint32_t* ids = nullptr;       // [rows] input ids
+  // Per launch lane: first row (within its group), length, lane of the carry.
+  const int* spans = nullptr;
+  const uint32_t* pos = nullptr;       // [rows] position in the lane (hybrid read only)
+  // Prefill: the last row of lane i for i < n_lanes, ~0u for a lane that
+  // does not run; its logits land in row i of lanes->logits.
+  const uint32_t* last = nullptr;
+  size_t n_lanes = 0;
+  // Training forward: targets, packed token index, scaled logits and
+  // losses (at the packed index) of every row.
+  const uint32_t* targets = nullptr;
+  const uint32_t* index = nullptr;
+  float* logits = nullptr;
+  float* loss = nullptr;
 };
+// A ragged prefill (last-token logits; hybrid ages and penalty windows
+// advance as in run_prefill, the ages by the longest lane).
+Status run_prefill_ragged(pssa_hip_lanes* L, const RaggedRows& rows);
 // The forward of stage_embed_norm .. stage_logits_loss (src/gpu_batch.rs:
-// 445-1250) over one segment: every row gets its scaled logits and its
-// cross-entropy loss.  The hybrid read is not supported here (the
-// reference's batched stages reject it).
-Status run_train_segment(pssa_hip_lanes* L, size_t n_lanes, size_t T, const TrainRows& tr);
-// One segment of a ragged prefill (last-token logits only; hybrid ages
-// advance T as in run_prefill).
-Status run_prefill_segment(pssa_hip_lanes* L, size_t n_lanes, size_t T, const TrainRows& rows,
-                           const int* lane_map);
-// Appends each row's last min(T, kHist) ids of ids [n_lanes, T] to the
-// window of lane lane_map[row] (lane_map null: lane = row).
-Status launch_hist_append(pssa_hip_lanes* L, const uint32_t* ids, size_t n_lanes, size_t T, const int* lane_map);
+// 445-1250): every row gets its scaled logits and its cross-entropy loss.
+// The hybrid read is not supported here (the reference's batched stages
+// reject it).
+Status run_train_forward(pssa_hip_lanes* L, const RaggedRows& rows);
+// Appends each lane's last min(length, kHist) ids to its window: lane i's
+// ids are rows i*T .. of ids [n_lanes, T], or those of its span.
+Status launch_hist_append(pssa_hip_lanes* L, const uint32_t* ids, size_t n_lanes, size_t T, const int* spans);
 // One greedy decode step for n_lanes lanes (ids in lanes->ids, replaced by
 // the chosen ids); plastic adds the lane-ordered protected bank writes and
 // the Hebbian adapter update.  Only kernel launches: safe to capture.

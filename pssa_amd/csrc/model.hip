@@ -335,10 +335,13 @@ __global__ void loop_combine_kernel(float* __restrict__ x, const float* __restri
 // recorded once layer 0's input projection has been issued.
 class PrefillView {
  public:
+  // With `rr` the view is group `group` of the ragged rows (lane0, n_lanes and
+  // T are then that group's and the longest lane).
   PrefillView(pssa_hip_lanes* L, hipStream_t st, size_t lane0, size_t n_lanes, size_t T, bool taps, bool timing,
-              hipEvent_t first_in_done, float* y_part, const TrainRows* tr, bool concurrent, size_t tap_rows = 0)
+              hipEvent_t first_in_done, float* y_part, const RaggedRows* rr, int group, bool concurrent,
+              size_t tap_rows = 0)
       : L_(L), M_(L->model), c_(L->model->cfg), st_(st), n_lanes_(n_lanes), T_(T), taps_(taps),
-        first_in_done_(first_in_done), y_part_(y_part), tr_(tr), concurrent_(concurrent),
+        first_in_done_(first_in_done), y_part_(y_part), rr_(rr), concurrent_(concurrent),
         tm_{timing ? L : nullptr, st} {
     d_ = (int)c_.d_latent;
     s_ = (int)c_.d_state;
@@ -347,8 +350,8 @@ class PrefillView {
     r_ = (int)c_.adapter_rank;
     V_ = (int)c_.d_vocab;
     n_in_ = (int)M_->n_in;
-    rows_ = n_lanes * T;
-    const size_t row0 = lane0 * T;
+    rows_ = rr ? rr->row0[group + 1] - rr->row0[group] : n_lanes * T;
+    const size_t row0 = rr ? rr->row0[group] : lane0 * T;
     m_ = (int)rows_;
     dt_ = M_->dtype;
     bf16_ = dt_ == PSSA_HIP_BF16;
@@ -369,8 +372,10 @@ class PrefillView {
     Wm_ = static_cast<char*>(L->Wm.p) + row0 * C * es;
     Mv_ = static_cast<char*>(L->Mval.p) + row0 * d * es;
     H1_ = static_cast<char*>(L->H1.p) + row0 * 2 * d * es;
-    ids_ = (tr ? tr->ids : L->ids.as<uint32_t>()) + row0;
-    carry_ = (tr ? tr->carry : L->carry.as<float>()) + lane0 * c_.depth * L->loops * (size_t)d * s_;
+    ids_ = (rr ? rr->ids : L->ids.as<uint32_t>()) + row0;
+    // Spans name each lane's carry themselves.
+    carry_ = L->carry.as<float>() + (rr ? 0 : lane0) * c_.depth * L->loops * (size_t)d * s_;
+    spans_ = rr ? rr->spans + 3 * lane0 : nullptr;
     logits_ = L->logits.as<float>() + lane0 * (size_t)V;
     row0_ = row0;
     // Taps are [layer][all rows of the step]; a lane group writes its rows.
@@ -413,7 +418,7 @@ class PrefillView {
     hipStream_t st = st_;
     // Column offsets inside the fused projection output P.
     const int o_b = d, o_c = d + s, o_qx = d + 2 * s, o_gate = d + 2 * s + k, o_act = 2 * d + 2 * s + k;
-    const bool step_y = ssm_step_writes_y((int)T, s);
+    const bool step_y = !rr_ && ssm_step_writes_y((int)T, s);
     // In a bf16 decode step the input product normalises its rows itself.
     const bool fold_norm = bf16 && step_y && gemm_norm_fits(d);
     PSSA_RETURN_IF(tm_.mark(ST_NORM));
@@ -471,6 +476,8 @@ class PrefillView {
     sa.d = d;
     sa.s = s;
     sa.lanes = (int)n_lanes_;
+    sa.spans = spans_;
+    sa.rows = rows;
     sa.y_part = y_part_;
     sa.concurrent = concurrent_ ? 1 : 0;
     if (bf16 && step_y) {
@@ -497,7 +504,10 @@ class PrefillView {
       ra.hgate = B.hgate.as<float>();
       ra.hage = B.hage.as<unsigned long long>();
       ra.log_lam = std::log((double)B.lam);
-      ra.age_T = (int)T;
+      if (rr_)
+        ra.row_age = rr_->pos + row0_;
+      else
+        ra.age_T = (int)T;
     }
     if (bf16)
       ra.weights16 = static_cast<uint16_t*>(Wm_);
@@ -602,13 +612,15 @@ class PrefillView {
     return launch_gemm(st, dt, H1_, 2 * d, B.mlp_w2.p, 2 * d, m, d, 2 * d, e_r);
   }
 
+  Status finish_timing() { return tm_.finish(); }
+
   Status head() {
     const int d = d_, V = V_, m = m_, dt = dt_;
     const size_t rows = rows_, T = T_;
     hipStream_t st = st_;
     const float logit_scale = 1.0f / sqrtf((float)d);
     PSSA_RETURN_IF(tm_.mark(ST_HEAD));
-    if (tr_ && tr_->logits) {
+    if (rr_) {
       // Every row: scaled logits, then its cross-entropy loss.
       const void* hin = X_;
       if (bf16_) {
@@ -618,11 +630,11 @@ class PrefillView {
       EpiParams e_h;
       e_h.kind = EPI_SCALE;
       e_h.scale = logit_scale;
-      e_h.out32 = tr_->logits + row0_ * (size_t)V;
+      e_h.out32 = rr_->logits + row0_ * (size_t)V;
       e_h.ld32 = V;
       PSSA_RETURN_IF(launch_gemm(st, dt, hin, d, M_->unembed.p, d, m, V, d, e_h));
-      token_ce_kernel<<<(unsigned)rows, 256, 0, st>>>(tr_->logits + row0_ * (size_t)V, V, tr_->targets + row0_,
-                                                     tr_->index + row0_, tr_->loss);
+      token_ce_kernel<<<(unsigned)rows, 256, 0, st>>>(rr_->logits + row0_ * (size_t)V, V, rr_->targets + row0_,
+                                                     rr_->index + row0_, rr_->loss);
       PSSA_LAUNCH_CHECK("token_ce");
       return tm_.finish();
     }
@@ -653,7 +665,7 @@ class PrefillView {
   bool taps_;
   hipEvent_t first_in_done_;
   float* y_part_;
-  const TrainRows* tr_;
+  const RaggedRows* rr_;
   bool concurrent_;
   Timer tm_;
   int d_ = 0, s_ = 0, k_ = 0, C_ = 0, r_ = 0, V_ = 0, n_in_ = 0, m_ = 0, dt_ = 0;
@@ -663,22 +675,55 @@ class PrefillView {
   uint16_t* XNh16_ = nullptr;
   void *XNh_ = nullptr, *Yh_ = nullptr, *Zrh_ = nullptr, *Wm_ = nullptr, *Mv_ = nullptr, *H1_ = nullptr;
   const uint32_t* ids_ = nullptr;
+  const int* spans_ = nullptr;
   float* carry_ = nullptr;
   float* logits_ = nullptr;
 };
 
-constexpr int kPrefillLaneGroups = 2;
-static_assert(kPrefillLaneGroups <= pssa_hip_lanes::kMaxGroups, "one stream per lane group");
+// Row last[i] of X for every lane i, as the head's operand (one wave a row;
+// zeros for a lane that does not run).
+__global__ __launch_bounds__(64) void gather_rows_kernel(const float* __restrict__ X, const uint32_t* __restrict__ last,
+                                                         int d, float* __restrict__ out, uint16_t* __restrict__ out16) {
+  const uint32_t r = last[blockIdx.x];
+  for (int i = threadIdx.x; i < d; i += 64) {
+    const float v = r == ~0u ? 0.0f : X[(size_t)r * d + i];
+    if (out16)
+      out16[(size_t)blockIdx.x * d + i] = bf16_of(v);
+    else
+      out[(size_t)blockIdx.x * d + i] = v;
+  }
+}
 
-static Status prefill_groups(pssa_hip_lanes* L, size_t n_lanes, size_t T, bool taps, const TrainRows* tr);
+// The head of a ragged prefill: every lane's last row, in lane order.
+static Status ragged_head(pssa_hip_lanes* L, const RaggedRows& rr) {
+  const pssa_hip_model* M = L->model;
+  const int d = (int)M->cfg.d_latent, V = (int)M->cfg.d_vocab, dt = M->dtype;
+  const hipStream_t st = L->ctx->stream;
+  uint16_t* h16 = dt == PSSA_HIP_BF16 ? L->XNh.as<uint16_t>() : nullptr;
+  gather_rows_kernel<<<(unsigned)rr.n_lanes, 64, 0, st>>>(L->X.as<float>(), rr.last, d, L->XN.as<float>(), h16);
+  PSSA_LAUNCH_CHECK("gather_rows");
+  EpiParams e_h;
+  e_h.kind = EPI_SCALE;
+  e_h.scale = 1.0f / sqrtf((float)d);
+  e_h.out32 = L->logits.as<float>();
+  e_h.ld32 = V;
+  return launch_gemm(st, dt, h16 ? (const void*)h16 : L->XN.p, d, M->unembed.p, d, (int)rr.n_lanes, V, d, e_h);
+}
+
+int prefill_lane_groups(const pssa_hip_lanes* L, size_t n_lanes, size_t max_len) {
+  const pssa_hip_config& c = L->model->cfg;
+  return n_lanes < 2 || max_len < 64 || L->timing || ssm_one_group((int)c.d_latent, (int)c.d_state, n_lanes, max_len) ? 1 : 2;
+}
+
+static Status prefill_groups(pssa_hip_lanes* L, size_t n_lanes, size_t T, bool taps, const RaggedRows* rr);
 static Status bump_hybrid_ages(pssa_hip_lanes* L, size_t T);
 
-Status run_prefill_segment(pssa_hip_lanes* L, size_t n_lanes, size_t T, const TrainRows& rows,
-                           const int* lane_map) {
-  if (rows.logits) return Status::Invalid("prefill segment: the all-token head belongs to the training forward");
-  PSSA_RETURN_IF(prefill_groups(L, n_lanes, T, false, &rows));
-  PSSA_RETURN_IF(launch_hist_append(L, rows.ids, n_lanes, T, lane_map));
-  return bump_hybrid_ages(L, T);
+Status run_prefill_ragged(pssa_hip_lanes* L, const RaggedRows& rr) {
+  PSSA_RETURN_IF(prefill_groups(L, rr.lane0[rr.groups], rr.max_len, false, &rr));
+  PSSA_RETURN_IF(ragged_head(L, rr));
+  for (int g = 0; g < rr.groups; ++g)
+    PSSA_RETURN_IF(launch_hist_append(L, rr.ids + rr.row0[g], rr.lane0[g + 1] - rr.lane0[g], 0, rr.spans + 3 * rr.lane0[g]));
+  return bump_hybrid_ages(L, rr.max_len);
 }
 
 Status run_prefill(pssa_hip_lanes* L, size_t n_lanes, size_t T, bool taps, bool append) {
@@ -690,13 +735,15 @@ Status run_prefill(pssa_hip_lanes* L, size_t n_lanes, size_t T, bool taps, bool 
 // One wave per row: the row's last min(T, 64) ids go into its lane's ring.
 __global__ __launch_bounds__(64) void hist_append_kernel(uint32_t* __restrict__ hist, int* __restrict__ hist_n,
                                                          int* __restrict__ hist_pos, const uint32_t* __restrict__ ids,
-                                                         int T, const int* __restrict__ lane_map) {
+                                                         int T, const int* __restrict__ spans) {
   constexpr int H = pssa_hip_lanes::kHist;
   const int row = blockIdx.x, j = threadIdx.x;
-  const int lane = lane_map ? lane_map[row] : row;
+  const int lane = spans ? spans[3 * row + 2] : row;
+  const size_t r0 = spans ? (size_t)spans[3 * row] : (size_t)row * T;
+  if (spans) T = spans[3 * row + 1];
   const int take = T < H ? T : H;
   const int pos = hist_pos[lane];
-  if (j < take) hist[(size_t)lane * H + (pos + j) % H] = ids[(size_t)row * T + (T - take) + j];
+  if (j < take) hist[(size_t)lane * H + (pos + j) % H] = ids[r0 + (T - take) + j];
   __syncthreads();
   if (j == 0) {
     hist_pos[lane] = (pos + take) % H;
@@ -705,9 +752,9 @@ __global__ __launch_bounds__(64) void hist_append_kernel(uint32_t* __restrict__ 
   }
 }
 
-Status launch_hist_append(pssa_hip_lanes* L, const uint32_t* ids, size_t n_lanes, size_t T, const int* lane_map) {
+Status launch_hist_append(pssa_hip_lanes* L, const uint32_t* ids, size_t n_lanes, size_t T, const int* spans) {
   hist_append_kernel<<<(unsigned)n_lanes, 64, 0, L->ctx->stream>>>(
-      L->hist.as<uint32_t>(), L->hist_n.as<int>(), L->hist_pos.as<int>(), ids, (int)T, lane_map);
+      L->hist.as<uint32_t>(), L->hist_n.as<int>(), L->hist_pos.as<int>(), ids, (int)T, spans);
   PSSA_LAUNCH_CHECK("hist_append");
   return Status::Ok();
 }
@@ -725,13 +772,13 @@ static Status bump_hybrid_ages(pssa_hip_lanes* L, size_t T) {
   return Status::Ok();
 }
 
-Status run_train_segment(pssa_hip_lanes* L, size_t n_lanes, size_t T, const TrainRows& tr) {
+Status run_train_forward(pssa_hip_lanes* L, const RaggedRows& rr) {
   for (const DevBlock& B : L->model->blocks)
     if (B.hybrid) return Status::Invalid("hybrid read currently requires the CPU backend");
-  return prefill_groups(L, n_lanes, T, false, &tr);
+  return prefill_groups(L, rr.lane0[rr.groups], rr.max_len, false, &rr);
 }
 
-static Status prefill_groups(pssa_hip_lanes* L, size_t n_lanes, size_t T, bool taps, const TrainRows* tr) {
+static Status prefill_groups(pssa_hip_lanes* L, size_t n_lanes, size_t T, bool taps, const RaggedRows* rr) {
   const hipStream_t st = L->ctx->stream;
   if (L->loops > 1)
     for (const DevBlock& B : L->model->blocks)
@@ -757,19 +804,23 @@ static Status prefill_groups(pssa_hip_lanes* L, size_t n_lanes, size_t T, bool t
 #ifndef PSSA_DECODE_GROUPS
 #define PSSA_DECODE_GROUPS 3
 #endif
-  const bool step_groups = PSSA_DECODE_GROUPS >= 2 && T == 1 && n_lanes >= 64 && !L->timing;
-  const int G = (int)std::min<size_t>(step_groups ? PSSA_DECODE_GROUPS : kPrefillLaneGroups, n_lanes);
-  if ((!taps && !L->timing && G >= 2 && T >= 64) || (step_groups && G >= 2)) {
+  const bool step_groups = PSSA_DECODE_GROUPS >= 2 && !rr && T == 1 && n_lanes >= 64 && !L->timing;
+  const int G = rr            ? rr->groups
+                : step_groups ? (int)std::min<size_t>(PSSA_DECODE_GROUPS, n_lanes)
+                              : prefill_lane_groups(L, n_lanes, T);
+  // A ragged prefill's head runs once, after the groups.
+  const bool view_head = !rr || rr->logits;
+  if (G >= 2 && (!taps || step_groups)) {
     PSSA_HIP_TRY(hipEventRecord(L->ev_fork, st));
     std::vector<PrefillView> views;
     views.reserve(G);
     size_t lane0 = 0;
     for (int g = 0; g < G; ++g) {
-      const size_t ng = n_lanes / G + ((size_t)g < n_lanes % G ? 1 : 0);
+      const size_t ng = rr ? rr->lane0[g + 1] - rr->lane0[g] : n_lanes / G + ((size_t)g < n_lanes % G ? 1 : 0);
       const hipStream_t sg = g == 0 ? st : L->aux_stream[g - 1];
-      float* yp = ypart ? ypart + (size_t)nz * lane0 * T * c.d_latent : nullptr;
+      float* yp = ypart ? ypart + (size_t)nz * (rr ? rr->row0[g] : lane0 * T) * c.d_latent : nullptr;
       views.emplace_back(L, sg, lane0, ng, T, taps, false, g + 1 < G && !step_groups ? L->ev_first[g] : nullptr,
-                         yp, tr, true, n_lanes * T);
+                         yp, rr, g, true, n_lanes * T);
       lane0 += ng;
     }
     for (int g = 0; g < G; ++g) {
@@ -783,17 +834,17 @@ static Status prefill_groups(pssa_hip_lanes* L, size_t n_lanes, size_t T, bool t
     }
     for (size_t l = 1; l < c.depth; ++l)
       for (int g = 0; g < G; ++g) PSSA_RETURN_IF(views[g].layer(l));
-    for (int g = 0; g < G; ++g) PSSA_RETURN_IF(views[g].head());
+    for (int g = 0; g < G && view_head; ++g) PSSA_RETURN_IF(views[g].head());
     for (int g = 1; g < G; ++g) {
       PSSA_HIP_TRY(hipEventRecord(L->ev_join[g - 1], L->aux_stream[g - 1]));
       PSSA_HIP_TRY(hipStreamWaitEvent(st, L->ev_join[g - 1], 0));
     }
     return Status::Ok();
   }
-  PrefillView v(L, st, 0, n_lanes, T, taps, L->timing, nullptr, ypart, tr, false);
+  PrefillView v(L, st, 0, n_lanes, T, taps, L->timing, nullptr, ypart, rr, 0, false);
   PSSA_RETURN_IF(v.embed());
   for (size_t l = 0; l < c.depth; ++l) PSSA_RETURN_IF(v.layer(l));
-  return v.head();
+  return view_head ? v.head() : v.finish_timing();
 }
 
 }  // namespace pssa

@@ -45,6 +45,10 @@ struct SsmArgs {
   int ld_y = 0;
   int T = 0, d = 0, s = 0;
   int lanes = 0;
+  // Ragged lanes: launch lane b runs rows spans[3b] .. + spans[3b + 1] - 1
+  // (its length, 1 <= length <= T) with the carry of lane spans[3b + 2].
+  // Null: rows b*T .. b*T+T-1, carry b.  `rows` is then the caller's.
+  const int* spans = nullptr;
   // Optional materialisation (stage API): per lane b, bar_a/bar_b at
   // + b*T*d*s, states at + b*(T+1)*d*s.  All three or none.
   float* bar_a = nullptr;
@@ -53,7 +57,7 @@ struct SsmArgs {
   // Partial readouts [state blocks, lanes*T, d], required when
   // ssm_state_blocks(s) > 2 (the blocks are then summed in a fixed order).
   float* y_part = nullptr;
-  size_t rows = 0;  // set by launch_ssm_scan
+  size_t rows = 0;  // rows of the launch (set by launch_ssm_scan without spans)
   // Optional bf16 copy of y, written by the single-step kernel when
   // ssm_step_writes_y (other paths leave it untouched).
   uint16_t* y16 = nullptr;
@@ -64,7 +68,7 @@ struct SsmArgs {
   int concurrent = 0;
 };
 
-// Rows of lane b are b*T .. b*T+T-1.  The states of a channel are split into
+// Rows of lane b are b*T .. b*T+T-1 (or its span's).  The states of a channel are split into
 // ssm_state_blocks(s) workgroups.  With two blocks both add their partial
 // readouts into y, which the caller zero-fills first (ssm_needs_zeroed_y; two
 // addends onto zero give the same sum in either order); with more, the
@@ -75,6 +79,10 @@ bool ssm_needs_zeroed_y(int s);
 // y16) directly: no zero-fill of y is needed and y16 is written.
 bool ssm_step_writes_y(int T, int s);
 Status launch_ssm_scan(hipStream_t stream, const SsmArgs& a);
+// Whether a prefill of these lanes is faster as one lane group: the few-lane
+// scan of all of them then fills the CUs by itself, and two groups' scans
+// would only run beside each other.
+bool ssm_one_group(int d, int s, size_t lanes, size_t max_len);
 
 // rates2[i] = rates[i] * log2(e) (stage API receives -softplus(a_raw)).
 Status launch_scale(hipStream_t stream, const float* in, float* out, size_t n, float scale);

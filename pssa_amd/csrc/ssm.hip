@@ -257,7 +257,9 @@ __global__ __launch_bounds__(NB * 256) void ssm_step_kernel(SsmArgs a) {
 #endif
 constexpr int SSM_TC = PSSA_SSM_TC;
 
-template <int J, int NW, int WPE>
+// SPANS: the lanes have spans (of the full-batch prefill's scan, whose loop is
+// sensitive to every register, a build of its own: 0.5% of the pass).
+template <int J, int NW, int WPE, bool SPANS>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE))) void ssm_scan_kernel(SsmArgs a) {
   // Steps staged per chunk: with few states per lane a chunk's compute is
   // short, so 16 steps stand between a chunk's input loads and their use.
@@ -281,11 +283,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE))) 
   const int i = i0 + lane;
   const int jw = jb + wave * J;
   const bool ivalid = i < a.d;
-  const int T = a.T, d = a.d, s = a.s;
-  const size_t row0 = (size_t)b * T;
+  const int T = SPANS ? a.spans[3 * b + 1] : a.T, d = a.d, s = a.s;
+  const size_t row0 = SPANS ? (size_t)a.spans[3 * b] : (size_t)b * T;
 
   float h[J], r2[J];
-  float* carry = a.carry + (size_t)b * a.carry_stride;
+  float* carry = a.carry + (size_t)(SPANS ? a.spans[3 * b + 2] : b) * a.carry_stride;
   const CarryCol cc = carry_col(jw, i, d, s);
 #pragma unroll
   for (int q = 0; q < J; ++q) {
@@ -468,11 +470,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
   const int i0 = blockIdx.x * CH, b = blockIdx.y, jb = blockIdx.z * SB;
   const int i = i0 + ch, jw = jb + g * GS + p;
   const bool ivalid = i < a.d;
-  const int T = a.T, d = a.d, s = a.s;
-  const size_t row0 = (size_t)b * T;
+  const int d = a.d, s = a.s;
+  const int T = a.spans ? a.spans[3 * b + 1] : a.T;
+  const size_t row0 = a.spans ? (size_t)a.spans[3 * b] : (size_t)b * T;
 
   float h[M], r2[M];
-  float* carry = a.carry + (size_t)b * a.carry_stride;
+  float* carry = a.carry + (size_t)(a.spans ? a.spans[3 * b + 2] : b) * a.carry_stride;
 #pragma unroll
   for (int m = 0; m < M; ++m) {
     const int j = jw + 4 * m;
@@ -702,6 +705,18 @@ constexpr long kScanFullGrid = 768;
 constexpr int kQuadChannels = 8;
 constexpr long kQuadMax = 1536;
 
+// From four workgroups per CU up to where the few-lane scan ends.  105M
+// prefill, two groups / one: 4 lanes x 512 (768 workgroups) 2.65 / 2.73 ms, 8
+// x 512 4.48 / 4.29, 12 x 512 5.76 / 5.47, 16 x 512 (3072) 7.33 / 7.00, 24 x
+// 512 9.51 / 10.9; short prompts leave the scan less of the pass: 8 x 128 1.66
+// / 1.73, 16 x 128 2.69 / 2.80.  Nine ragged prompts of up to 1000 4.39 /
+// 4.19 ms.
+bool ssm_one_group(int d, int s, size_t lanes, size_t max_len) {
+  if (s < 128 || max_len < 256) return false;
+  const size_t wgs = (size_t)((d + kQuadChannels - 1) / kQuadChannels) * lanes * ((s + 127) / 128);
+  return wgs >= 1024 && wgs <= 2 * (size_t)kQuadMax;
+}
+
 // Lanes per decode-step workgroup (they share the rate loads).
 #ifndef PSSA_SSM_STEP_LPB
 #define PSSA_SSM_STEP_LPB 4
@@ -716,12 +731,27 @@ static long quad_workgroups(const SsmArgs& a, dim3& grid) {
   return (long)grid.x * grid.y * grid.z;
 }
 
+template <int J, bool SPANS>
+static void launch_scan(hipStream_t stream, const SsmArgs& a, dim3 grid) {
+  if constexpr (J == 32) {
+    if ((long)grid.x * grid.y * grid.z < kScanFullGrid && !a.concurrent)
+      ssm_scan_kernel<16, 8, 4, SPANS><<<grid, 512, 0, stream>>>(a);
+    else
+      ssm_scan_kernel<32, 4, 3, SPANS><<<grid, 256, 0, stream>>>(a);
+  } else {
+    // Few states per lane: a small model's grid of a few workgroups, each
+    // bound by its step chain, so occupancy gives nothing and the register
+    // budget of two waves per SIMD keeps the 16-step staging out of scratch.
+    ssm_scan_kernel<J, 4, 2, SPANS><<<grid, 256, 0, stream>>>(a);
+  }
+}
+
 template <int J>
 static void launch_j(hipStream_t stream, const SsmArgs& a, bool mat) {
   dim3 grid((a.d + 63) / 64, a.lanes, (a.s + 4 * J - 1) / (4 * J)), qgrid;
   if (mat) {
     ssm_materialize_kernel<J, true><<<grid, 256, 0, stream>>>(a);
-  } else if (a.T == 1) {
+  } else if (a.T == 1 && !a.spans) {
     // At most one lane per wave of the workgroup (the readout's waves).
     constexpr int LPB2 = PSSA_SSM_STEP_LPB < 8 ? PSSA_SSM_STEP_LPB : 8;
     constexpr int LPB1 = PSSA_SSM_STEP_LPB < 4 ? PSSA_SSM_STEP_LPB : 4;
@@ -733,7 +763,7 @@ static void launch_j(hipStream_t stream, const SsmArgs& a, bool mat) {
       grid.y = (a.lanes + LPB1 - 1) / LPB1;
       ssm_step_kernel<J, 1, LPB1><<<grid, 256, 0, stream>>>(a);
     }
-  } else if (a.T < SSM_TC) {
+  } else if (a.T < SSM_TC && !a.spans) {
     ssm_materialize_kernel<J, false><<<grid, 256, 0, stream>>>(a);
   } else if (J >= 8 && quad_workgroups<J>(a, qgrid) <= (J == 32 && !a.concurrent ? 2 : 1) * kQuadMax) {
     constexpr int M = J == 32 ? 4 : 2;
@@ -743,18 +773,10 @@ static void launch_j(hipStream_t stream, const SsmArgs& a, bool mat) {
       ssm_quad_kernel<M, kQuadChannels, true><<<qgrid, 256, 0, stream>>>(a);
     else
       ssm_quad_kernel<M, kQuadChannels, false><<<qgrid, 256, 0, stream>>>(a);
-  } else if constexpr (J == 32) {
-    if ((long)grid.x * grid.y * grid.z < kScanFullGrid && !a.concurrent)
-      ssm_scan_kernel<16, 8, 4><<<grid, 512, 0, stream>>>(a);
-    else
-      ssm_scan_kernel<32, 4, 3><<<grid, 256, 0, stream>>>(a);
-  } else if constexpr (J <= 8) {
-    // Few states per lane: a small model's grid of a few workgroups, each
-    // bound by its step chain, so occupancy gives nothing and the register
-    // budget of two waves per SIMD keeps the 16-step staging out of scratch.
-    ssm_scan_kernel<J, 4, 2><<<grid, 256, 0, stream>>>(a);
+  } else if (a.spans) {
+    launch_scan<J, true>(stream, a, grid);
   } else {
-    ssm_scan_kernel<J, 4, 3><<<grid, 256, 0, stream>>>(a);
+    launch_scan<J, false>(stream, a, grid);
   }
 }
 
@@ -763,7 +785,8 @@ Status launch_ssm_scan(hipStream_t stream, const SsmArgs& a_in) {
   if (a.T <= 0 || a.d <= 0 || a.s <= 0 || a.lanes <= 0) return Status::Invalid("ssm: empty shape");
   const bool mat = a.bar_a && a.bar_b && a.states;
   const int nz = ssm_state_blocks(a.s);
-  a.rows = (size_t)a.lanes * a.T;
+  if (!a.spans) a.rows = (size_t)a.lanes * a.T;
+  if (mat && a.spans) return Status::Invalid("ssm: the tape is written for lanes of one length");
   if (mat || nz <= 2) {
     a.y_part = nullptr;
   } else if (!a.y_part) {

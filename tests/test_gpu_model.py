@@ -354,6 +354,39 @@ def test_ragged_prefill_matches_oracle_and_single_lanes(hip):
     layer.close()
 
 
+@pytest.mark.parametrize("d_state,dtype,hybrid", [(16, "f32", False), (64, "bf16", True), (136, "f32", True),
+                                                  (300, "bf16", False)])
+def test_ragged_rows_equal_single_lanes_bitwise(hip, d_state, dtype, hybrid):
+    """The packed rows of lanes of many lengths (one token, the scans' chunk
+    edges, both lane groups and, in the short batch, one) against each lane's
+    own prefill: logits, carries and the greedy tokens after it under the
+    repetition penalty, with the hybrid read's ages too."""
+    cfg = PSSAConfig(depth=2, d_vocab=151, d_latent=72, d_state=d_state, d_mem_key=8, mem_capacity=30)
+    w = ModelWeights.init(cfg, 17, "baseline")
+    w.populate_banks(18, count=25)
+    if hybrid:
+        w.set_hybrid_read(True, 0.97)
+    rng = np.random.default_rng(d_state)
+    for lens in ([17, 1, 64, 100, 3, 65, 16, 33, 2], [5, 1, 31]):
+        say("ragged rows", d_state, dtype, hybrid, lens)
+        seqs = [rng.integers(0, cfg.d_vocab, n, dtype=np.uint32) for n in lens]
+        layer = PSSALayer(hip, w, lanes=len(lens), max_tokens=sum(lens), weight_dtype=dtype)
+        layer.set_repetition_penalty(1.25)
+        got, car = layer.prefill_ragged(seqs), layer.get_carry()
+        if hybrid:
+            assert int(layer.get_hybrid(1)[1][:25].min()) == max(lens)
+        ids = None if hybrid else layer.decode(3)  # the lanes' ages differ from a lane's own afterwards
+        layer.close()
+        for i, q in enumerate(seqs):
+            one = PSSALayer(hip, w, lanes=1, max_tokens=max(lens), weight_dtype=dtype)
+            one.set_repetition_penalty(1.25)
+            np.testing.assert_array_equal(one.prefill_inference(q[None])[0], got[i])
+            np.testing.assert_array_equal(one.get_carry()[0], car[i])
+            if ids is not None:
+                np.testing.assert_array_equal(one.decode(3)[:, 0], ids[:, i])
+            one.close()
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 def test_memory_top_k_model_matches_oracle(hip, dtype):
     """set_memory_top_k on the model (src/pssa.rs:2215-2226): prefill and
