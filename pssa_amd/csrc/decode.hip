@@ -56,6 +56,32 @@ struct GreedyWindow {
   int* nonfinite = nullptr;  // raised on any non-finite logit
 };
 
+// The window of row `row` into LDS by one wave (oldest id first; kHist is the
+// wave's width, so every entry is one load in flight), after the consumed id
+// is appended to the ring; n_out = its entries, 0 without a penalty.
+__device__ __forceinline__ void read_window(const GreedyWindow& gw, uint32_t consumed, int row, int lane, bool pen,
+                                            uint32_t* win, int& n_out) {
+  constexpr int H = pssa_hip_lanes::kHist;
+  static_assert(H == 64, "one window entry per wave lane");
+  int n = gw.hist_n[row], pos = gw.hist_pos[row];
+  const uint32_t at = gw.hist[(size_t)row * H + lane];  // ring slot `lane`
+  if (gw.append_row_id) {
+    if (lane == 0) gw.hist[(size_t)row * H + pos] = consumed;
+    pos = (pos + 1) % H;
+    n = n < H ? n + 1 : H;
+    if (lane == 0) {
+      gw.hist_pos[row] = pos;
+      gw.hist_n[row] = n;
+    }
+  }
+  if (pen) {
+    const int j = (lane - pos + n + H) % H;  // slot's place in the window: slot (pos - n + j) mod kHist
+    const bool appended = gw.append_row_id && lane == (pos + H - 1) % H;
+    if (j < n) win[j] = appended ? consumed : at;
+  }
+  if (lane == 0) n_out = pen ? n : 0;
+}
+
 // One workgroup per lane, one pass over the logits: greedy id over 1..V-1
 // in f32::total_cmp order (ties to the lower id) after the repetition
 // penalty, and the surprise logsumexp(logits) - logits[chosen] of the raw
@@ -81,18 +107,7 @@ __global__ __launch_bounds__(256) void greedy_kernel(const float* __restrict__ l
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const float* lg = logits + (size_t)row * V;
   const bool pen = gw.penalty > 1.0f && gw.hist != nullptr;
-  if (gw.hist && tid == 0) {
-    int n = gw.hist_n[row], pos = gw.hist_pos[row];
-    if (gw.append_row_id) {
-      gw.hist[(size_t)row * H + pos] = ids[row];
-      pos = (pos + 1) % H;
-      n = n < H ? n + 1 : H;
-      gw.hist_pos[row] = pos;
-      gw.hist_n[row] = n;
-    }
-    s_n = pen ? n : 0;
-    for (int j = 0; j < n && pen; ++j) s_win[j] = gw.hist[(size_t)row * H + (pos - n + j + H) % H];
-  }
+  if (gw.hist && wave == 0) read_window(gw, ids[row], row, lane, pen, s_win, s_n);
   __syncthreads();
   const int wn = s_n;
   if (wave == 0 && lane < wn) {
@@ -205,20 +220,15 @@ __device__ __forceinline__ bool ranks_before(float pa, int va, float pb, int vb)
   return pa > pb || (pa == pb && va < vb);
 }
 
-// Vocabularies up to this size keep the lane's probability row in LDS, where
-// the one-thread ordered sum reads it at LDS latency; larger ones use the
-// global scratch row.
-constexpr int kSampleLdsMaxV = 36 * 1024;
 constexpr int kWinBloomWords = 64;  // 2048-bit filter of the penalty window ids
 
-template <bool ROW_LDS>
+// The general kernel: any vocabulary, the row in global scratch.
 __global__ __launch_bounds__(256) void sample_kernel(const float* __restrict__ logits, int V,
                                                      uint32_t* __restrict__ ids,
                                                      uint32_t* __restrict__ gen_ids,
                                                      const int* __restrict__ gen_pos, int n_lanes,
                                                      float* __restrict__ surprise, GreedyWindow gw, SampleArgs sa) {
   constexpr int H = pssa_hip_lanes::kHist;
-  extern __shared__ __attribute__((aligned(16))) float s_row[];
   __shared__ uint32_t s_win[H];
   __shared__ float s_val[H];
   __shared__ uint32_t s_bloom[kWinBloomWords];
@@ -231,21 +241,10 @@ __global__ __launch_bounds__(256) void sample_kernel(const float* __restrict__ l
   __shared__ int s_selv[kMaxSampleTopK];
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const float* lg = logits + (size_t)row * V;
-  float* pr = ROW_LDS ? s_row : sa.probs + (size_t)row * V;
+  float* pr = sa.probs + (size_t)row * V;
   const bool pen = gw.penalty > 1.0f && gw.hist != nullptr;
   if (tid < kWinBloomWords) s_bloom[tid] = 0u;
-  if (gw.hist && tid == 0) {
-    int n = gw.hist_n[row], pos = gw.hist_pos[row];
-    if (gw.append_row_id) {
-      gw.hist[(size_t)row * H + pos] = ids[row];
-      pos = (pos + 1) % H;
-      n = n < H ? n + 1 : H;
-      gw.hist_pos[row] = pos;
-      gw.hist_n[row] = n;
-    }
-    s_n = pen ? n : 0;
-    for (int j = 0; j < n && pen; ++j) s_win[j] = gw.hist[(size_t)row * H + (pos - n + j + H) % H];
-  }
+  if (gw.hist && wave == 0) read_window(gw, ids[row], row, lane, pen, s_win, s_n);
   __syncthreads();
   const int wn = s_n;
   // Penalised logits of the window ids: each distinct id divided (positive) or
@@ -317,19 +316,8 @@ __global__ __launch_bounds__(256) void sample_kernel(const float* __restrict__ l
     pr[v] = v == 0 ? 0.0f : (float)exp((double)((plogit(v) - top) / temp));
   __syncthreads();
   if (tid == 0) {
-    // Adding probs[0] = 0 first leaves the sum +0, so the float4 reads can
-    // start at id 0; the adds stay one at a time in id order.
     float sum = 0.0f;
-    const int v4 = ROW_LDS ? V & ~3 : 0;
-#pragma unroll 8
-    for (int v = 0; v < v4; v += 4) {
-      const float4 q = *reinterpret_cast<const float4*>(pr + v);
-      sum += q.x;
-      sum += q.y;
-      sum += q.z;
-      sum += q.w;
-    }
-    for (int v = v4 > 1 ? v4 : 1; v < V; ++v) sum += pr[v];
+    for (int v = 1; v < V; ++v) sum += pr[v];
     s_sum = sum;
   }
   __syncthreads();
@@ -432,6 +420,395 @@ __global__ __launch_bounds__(256) void sample_kernel(const float* __restrict__ l
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same choice with the row in registers, for vocabularies of up to
+// 1024 * NE ids: a workgroup of 16 waves, thread t holding ids t*NE ..
+// t*NE + NE - 1.  One lane's choice is one workgroup's latency, and of the
+// general kernel's 944 us at 16384 ids and top_k 24 most was the one-thread sum
+// and the search for each of the top_k; this one takes 74 us (a sampled,
+// penalised lane of the 105M model: 1.66 -> 0.82 ms per step).
+//
+// The f32 sum in id order, exactly as one thread adding one id at a time:
+// while the sum S stays inside one power of two (every S a multiple of
+// u = ulp(S)), adding p adds p rounded to a multiple of u, which depends on S
+// only where p is halfway between two multiples, and there only on S's last
+// bit.  Each thread therefore forms what its ids add for either last bit
+// (integers in units of u), and these maps compose associatively: a scan over
+// the threads gives every prefix.  The first thread whose ids take S past
+// the power of two (or that holds an id large against S, where p in units of u
+// is not exact) adds its ids one by one from its exact prefix, and the scan
+// resumes behind it with the new u: about one round per doubling of S.
+//
+// The top_k: T = the top_k-th largest of the threads' largest probabilities
+// (bit search by one wave), so at least top_k ids reach T and every id of the
+// top_k does; those (about top_k) are ranked by (probability desc, id asc).
+// More than kSampleCand of them (equal logits): top_k rounds of a workgroup
+// arg-max.
+constexpr int kSampleThreads = 1024;
+constexpr int kSampleCand = 512;
+constexpr int kSampleNE = 16, kSampleWideNE = 36;
+
+// x shifted in from the lanes before, 0 where there are none (`CTRL`,
+// `ROWS`: the DPP control and row mask of a wave-wide scan step).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_from(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xF, false);
+}
+// What the ids before (b0, b1: by the last bit of the sum they start from)
+// and then these (a0, a1) add, saturated at 2^24.
+__device__ __forceinline__ void sum_compose(int b0, int b1, int& a0, int& a1) {
+  const int n0 = b0 + ((b0 & 1) ? a1 : a0);
+  const int n1 = b1 + ((b1 & 1) ? a0 : a1);
+  a0 = min(n0, 1 << 24);
+  a1 = min(n1, 1 << 24);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ void sum_scan_step(int& a0, int& a1) {
+  const int b0 = dpp_from<CTRL, ROWS>(a0), b1 = dpp_from<CTRL, ROWS>(a1);
+  sum_compose(b0, b1, a0, a1);
+}
+
+template <int NE>
+__global__ __launch_bounds__(kSampleThreads) void sample_row_kernel(const float* __restrict__ logits, int V,
+                                                                   uint32_t* __restrict__ ids,
+                                                                   uint32_t* __restrict__ gen_ids,
+                                                                   const int* __restrict__ gen_pos, int n_lanes,
+                                                                   float* __restrict__ surprise, GreedyWindow gw,
+                                                                   SampleArgs sa) {
+  constexpr int H = pssa_hip_lanes::kHist, NW = kSampleThreads / 64;
+  __shared__ uint32_t s_win[H];
+  __shared__ float s_val[H];
+  __shared__ int s_n, s_cnt, s_t0, s_key;
+  __shared__ float s_m[NW], s_l[NW], s_x[NW];
+  __shared__ int2 s_pair[NW];
+  __shared__ float s_S;
+  __shared__ __attribute__((aligned(16))) int s_best[kSampleThreads];
+  __shared__ float s_cp[kSampleCand];
+  __shared__ int s_cv[kSampleCand];
+  __shared__ float s_selp[kMaxSampleTopK];
+  __shared__ int s_selv[kMaxSampleTopK];
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const float* lg = logits + (size_t)row * V;
+  const int v0 = tid * NE;
+  const bool pen = gw.penalty > 1.0f && gw.hist != nullptr;
+
+  float x[NE];
+  if (V % 4 == 0) {  // rows are 16-byte aligned
+#pragma unroll
+    for (int k = 0; k < NE; k += 4) {
+      const float4 q = *reinterpret_cast<const float4*>(lg + min(v0 + k, V - 4));
+      x[k] = q.x, x[k + 1] = q.y, x[k + 2] = q.z, x[k + 3] = q.w;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < NE; ++k) x[k] = lg[min(v0 + k, V - 1)];
+  }
+  if (tid == 0) s_n = 0;
+  if (tid == 64) s_cnt = 0;
+  if (gw.hist && wave == 0) {
+    read_window(gw, ids[row], row, lane, pen, s_win, s_n);
+    // Penalised logits of the window ids: each distinct id divided (positive)
+    // or multiplied by the penalty once per occurrence.
+    const int wn = pen ? __builtin_amdgcn_readfirstlane(s_n) : 0;
+    const uint32_t id = lane < wn ? s_win[lane] : 0u;
+    int c = 0;
+    for (int j = 0; j < wn; ++j) c += (uint32_t)__builtin_amdgcn_readlane((int)id, j) == id;
+    if (lane < wn) {
+      float l = id < (uint32_t)V ? lg[id] : 0.0f;
+      for (int q = 0; q < c; ++q) l = l > 0.0f ? l / gw.penalty : l * gw.penalty;
+      s_val[lane] = l;
+    }
+  }
+  // Raw logits: finite?  and, where asked for, their logsumexp.
+  int bad = 0;
+  float m = -INFINITY, sacc = 0.0f;
+#pragma unroll
+  for (int k = 0; k < NE; ++k)
+    if (v0 + k < V) {
+      bad |= !isfinite(x[k]);
+      m = fmaxf(m, x[k]);
+    }
+  if (surprise && m != -INFINITY) {
+#pragma unroll
+    for (int k = 0; k < NE; ++k)
+      if (v0 + k < V) sacc += expf(x[k] - m);
+  }
+  bad = __syncthreads_or(bad);  // the window too
+  {
+    const int wn = s_n;
+    const int wid = lane < wn ? (int)s_win[lane] : 0;
+    const int wval = lane < wn ? __float_as_int(s_val[lane]) : 0;
+    for (int j = 0; j < wn; ++j) {
+      const uint32_t id = (uint32_t)__builtin_amdgcn_readlane(wid, j);
+      if (id / (64 * NE) != (uint32_t)wave || id >= (uint32_t)V) continue;  // uniform
+      const float pv = __int_as_float(__builtin_amdgcn_readlane(wval, j));
+      const bool own = id / NE == (uint32_t)tid;
+#pragma unroll
+      for (int k = 0; k < NE; ++k)
+        if (id % NE == (uint32_t)k) x[k] = own ? pv : x[k];
+    }
+  }
+  // Maximum of the penalised logits over 1..V-1.
+  float mx = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < NE; ++k)
+    if (v0 + k >= 1 && v0 + k < V) mx = fmaxf(mx, x[k]);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    if (surprise) lse_merge(m, sacc, __shfl_xor(m, off, 64), __shfl_xor(sacc, off, 64));
+  }
+  if (lane == 0) {
+    s_m[wave] = m;
+    s_l[wave] = sacc;
+    s_x[wave] = mx;
+  }
+  __syncthreads();
+  float top = s_x[0];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) top = fmaxf(top, s_x[w]);
+
+  // Subtract before dividing (src/inference.rs:139-142).
+  const float temp = sa.temperature;
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int v = v0 + k;
+    x[k] = v >= 1 && v < V ? (float)exp((double)((x[k] - top) / temp)) : 0.0f;
+  }
+
+  // The ordered sum (see above).
+  float S = 0.0f;
+  for (int t0 = 0; t0 < kSampleThreads;) {
+    const int eb = max(__float_as_int(S) >> 23, 1);  // biased exponent of S >= 0
+    // Below 2^-103 no scale reaches units of u: every nonzero id stops there.
+    const bool tiny = eb < 24;
+    const float inv_u = tiny ? INFINITY : __int_as_float((277 - eb) << 23);
+    const int s_units = tiny ? 0 : (int)(S * inv_u);
+    constexpr float kRound = 12582912.0f;  // 1.5 * 2^23: x + kRound - kRound rounds x to an integer, ties to even
+    float n = 0.0f;
+    bool stop = false, tie = false;
+#pragma unroll
+    for (int k = 0; k < NE; ++k) {
+      const float q = x[k] == 0.0f ? 0.0f : x[k] * inv_u;
+      const float r = (q + kRound) - kRound;
+      stop |= !(q < 4194304.0f);
+      tie |= fabsf(q - r) == 0.5f;
+      n += r;
+    }
+    int a0 = (int)fminf(n, 16777216.0f), a1 = a0;
+    if (tie && !stop) {
+      a0 = 0;
+      a1 = 1;
+      const int from1 = a1;
+#pragma unroll
+      for (int k = 0; k < NE; ++k) {
+        const float q = x[k] == 0.0f ? 0.0f : x[k] * inv_u;
+        const float f = floorf(q), d = q - f;
+        const int i = (int)f;
+        const int up = d > 0.5f ? 1 : 0, half = d == 0.5f ? 1 : 0;
+        a0 += i + (half ? ((a0 + i) & 1) : up);
+        a1 += i + (half ? ((a1 + i) & 1) : up);
+      }
+      a1 -= from1;
+      a0 = min(a0, 1 << 24);
+      a1 = min(a1, 1 << 24);
+    }
+    if (stop) a0 = a1 = 1 << 24;
+    if (tid < t0) a0 = a1 = 0;
+    sum_scan_step<0x111, 0xF>(a0, a1);  // row_shr 1, 2, 4, 8: inside rows of 16
+    sum_scan_step<0x112, 0xF>(a0, a1);
+    sum_scan_step<0x114, 0xF>(a0, a1);
+    sum_scan_step<0x118, 0xF>(a0, a1);
+    sum_scan_step<0x142, 0xA>(a0, a1);  // row_bcast 15 into rows 1 and 3
+    sum_scan_step<0x143, 0xC>(a0, a1);  // row_bcast 31 into rows 2 and 3
+    if (lane == 63) s_pair[wave] = make_int2(a0, a1);
+    __syncthreads();
+    int base = s_units, cross = NW;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const int2 pr = s_pair[w];
+      const int end = base + ((base & 1) ? pr.y : pr.x);
+      if (cross == NW) {
+        if (end >= 1 << 24)
+          cross = w;
+        else
+          base = end;
+      }
+    }
+    if (cross == NW) {  // no id takes S past its power of two
+      if (!tiny) S = (float)base * __int_as_float(max(eb - 23, 1) << 23);
+      break;
+    }
+    if (wave == cross) {
+      const int incl = base + ((base & 1) ? a1 : a0);
+      const unsigned long long over = __ballot(incl >= 1 << 24);
+      const int tl = __builtin_ctzll(over);
+      const int before = __shfl_up(incl, 1, 64);
+      if (lane == tl) {
+        float t = tiny ? S : (float)(lane == 0 ? base : before) * __int_as_float(max(eb - 23, 1) << 23);
+#pragma unroll
+        for (int k = 0; k < NE; ++k) t += x[k];
+        s_S = t;
+        s_t0 = tid + 1;
+      }
+    }
+    __syncthreads();
+    S = s_S;
+    t0 = s_t0;
+    if (!isfinite(S)) break;
+  }
+  const bool mass_ok = isfinite(S) && S > 0.0f;
+  const int K = mass_ok ? min(V - 1, min(sa.top_k, kMaxSampleTopK)) : 0;
+  int key = -1;  // bits of the thread's largest probability (non-negative, so ordered as integers)
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    x[k] = x[k] / S;
+    if (v0 + k >= 1 && v0 + k < V && mass_ok) key = max(key, __float_as_int(x[k]));
+  }
+  s_best[tid] = key;
+  __syncthreads();
+  if (wave == 0 && K > 0) {
+    int4 b[NW / 4];
+#pragma unroll
+    for (int i = 0; i < NW / 4; ++i) b[i] = reinterpret_cast<const int4*>(s_best)[i * 64 + lane];
+    int t = 0;
+    for (int bit = 29; bit >= 0; --bit) {  // a probability is at most 1: bits below 2^30
+      const int c = t | (1 << bit);
+      int n = 0;
+#pragma unroll
+      for (int i = 0; i < NW / 4; ++i)
+        n += __popcll(__ballot(b[i].x >= c)) + __popcll(__ballot(b[i].y >= c)) + __popcll(__ballot(b[i].z >= c)) +
+             __popcll(__ballot(b[i].w >= c));
+      if (n >= K) t = c;
+    }
+    if (lane == 0) s_key = t;
+  }
+  __syncthreads();
+  if (K > 0 && key >= s_key) {
+    const int t = s_key;
+#pragma unroll
+    for (int k = 0; k < NE; ++k)
+      if (v0 + k >= 1 && v0 + k < V && __float_as_int(x[k]) >= t) {
+        const int slot = atomicAdd(&s_cnt, 1);
+        if (slot < kSampleCand) {
+          s_cp[slot] = x[k];
+          s_cv[slot] = v0 + k;
+        }
+      }
+  }
+  __syncthreads();
+  const int nc = s_cnt;
+  if (nc <= kSampleCand) {
+    if (tid < nc) {
+      const float p = s_cp[tid];
+      const int v = s_cv[tid];
+      int rank = 0;
+      for (int j = 0; j < nc; ++j) rank += ranks_before(s_cp[j], s_cv[j], p, v);
+      if (rank < K) {
+        s_selp[rank] = p;
+        s_selv[rank] = v;
+      }
+    }
+  } else {
+    float lp = INFINITY;
+    int lv = -1;
+    for (int r = 0; r < K; ++r) {
+      float bp = -1.0f;
+      int bv = INT32_MAX;
+#pragma unroll
+      for (int k = 0; k < NE; ++k) {
+        const int v = v0 + k;
+        if (v >= 1 && v < V && ranks_before(lp, lv, x[k], v) && ranks_before(x[k], v, bp, bv)) {
+          bp = x[k];
+          bv = v;
+        }
+      }
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) {
+        const float op = __shfl_xor(bp, off, 64);
+        const int ov = __shfl_xor(bv, off, 64);
+        if (ranks_before(op, ov, bp, bv)) {
+          bp = op;
+          bv = ov;
+        }
+      }
+      if (lane == 0) {
+        s_cp[(r & 1) * NW + wave] = bp;  // two slots alternate by round: one barrier each
+        s_cv[(r & 1) * NW + wave] = bv;
+      }
+      __syncthreads();
+      lp = s_cp[(r & 1) * NW];
+      lv = s_cv[(r & 1) * NW];
+      for (int w = 1; w < NW; ++w)
+        if (ranks_before(s_cp[(r & 1) * NW + w], s_cv[(r & 1) * NW + w], lp, lv)) {
+          lp = s_cp[(r & 1) * NW + w];
+          lv = s_cv[(r & 1) * NW + w];
+        }
+      if (tid == 0) {
+        s_selp[r] = lp;
+        s_selv[r] = lv;
+      }
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    int best = 0;
+    if (!mass_ok) {
+      if (sa.bad_mass && lane == 0) sa.bad_mass[0] = 1;
+    } else {
+      // Lane i holds choice i; the sums run in order on broadcast values.
+      const int sp = __float_as_int(lane < K ? s_selp[lane] : 0.0f);
+      const int sv = lane < K ? s_selv[lane] : 0;
+      auto prob = [&](int i) { return __int_as_float(__builtin_amdgcn_readlane(sp, i)); };
+      int cutoff = K;
+      float cumulative = 0.0f;
+      for (int i = 0; i < K; ++i) {
+        cumulative += prob(i);
+        if (cumulative >= sa.top_p) {
+          cutoff = i + 1;
+          break;
+        }
+      }
+      const int nf = cutoff > 1 ? cutoff : 1;
+      float mass = 0.0f;
+      for (int i = 0; i < nf; ++i) mass += prob(i);
+      // SimpleRng::next_u32 (xorshift64*) and gen_range_f32(0, mass)
+      // (src/linalg.rs:13-27).
+      unsigned long long g = sa.rng[row];
+      g ^= g >> 12;
+      g ^= g << 25;
+      g ^= g >> 27;
+      if (lane == 0) sa.rng[row] = g;
+      const uint32_t u = (uint32_t)((g * 0x2545F4914F6CDD1DULL) >> 32);
+      const float norm = (float)u / (float)4294967295u;
+      const float draw = norm * mass;  // low + norm * (high - low) with low = 0
+      float running = 0.0f;
+      best = __builtin_amdgcn_readlane(sv, nf - 1);
+      for (int i = 0; i < nf; ++i) {
+        running += prob(i);
+        if (draw <= running) {
+          best = __builtin_amdgcn_readlane(sv, i);
+          break;
+        }
+      }
+    }
+    if (lane == 0) {
+      ids[row] = (uint32_t)best;
+      if (gen_ids) gen_ids[(size_t)gen_pos[0] * n_lanes + row] = (uint32_t)best;
+      if (surprise) {
+        for (int w = 0; w < NW; ++w)
+          if (w == 0)
+            m = s_m[0], sacc = s_l[0];
+          else
+            lse_merge(m, sacc, s_m[w], s_l[w]);
+        surprise[row] = (m + logf(sacc)) - lg[best];
+      }
+      if (bad && gw.nonfinite) gw.nonfinite[0] = 1;
+    }
+  }
+}
+
 // The lanes' choice from L->logits: greedy at temperature 0, sampled above.
 static Status launch_choice(pssa_hip_lanes* L, size_t n_lanes, const GreedyWindow& gw, uint32_t* gen_ids,
                             const int* gen_pos, float* surprise) {
@@ -445,12 +822,15 @@ static Status launch_choice(pssa_hip_lanes* L, size_t n_lanes, const GreedyWindo
     sa.rng = L->rng.as<unsigned long long>();
     sa.probs = L->probs.as<float>();
     sa.bad_mass = L->nonfinite.as<int>() + 2;
-    if (V <= kSampleLdsMaxV)
-      sample_kernel<true><<<(unsigned)n_lanes, 256, (size_t)V * 4, st>>>(
-          L->logits.as<float>(), V, L->ids.as<uint32_t>(), gen_ids, gen_pos, (int)n_lanes, surprise, gw, sa);
+    auto* k = V <= kSampleThreads * kSampleNE       ? &sample_row_kernel<kSampleNE>
+              : V <= kSampleThreads * kSampleWideNE ? &sample_row_kernel<kSampleWideNE>
+                                                    : nullptr;
+    if (k)
+      k<<<(unsigned)n_lanes, kSampleThreads, 0, st>>>(L->logits.as<float>(), V, L->ids.as<uint32_t>(), gen_ids,
+                                                      gen_pos, (int)n_lanes, surprise, gw, sa);
     else
-      sample_kernel<false><<<(unsigned)n_lanes, 256, 0, st>>>(L->logits.as<float>(), V, L->ids.as<uint32_t>(),
-                                                              gen_ids, gen_pos, (int)n_lanes, surprise, gw, sa);
+      sample_kernel<<<(unsigned)n_lanes, 256, 0, st>>>(L->logits.as<float>(), V, L->ids.as<uint32_t>(), gen_ids,
+                                                       gen_pos, (int)n_lanes, surprise, gw, sa);
     PSSA_LAUNCH_CHECK("sample");
   } else {
     greedy_kernel<<<(unsigned)n_lanes, 256, 0, st>>>(L->logits.as<float>(), V, L->ids.as<uint32_t>(), gen_ids,
@@ -741,8 +1121,6 @@ Status init_decode_attributes() {
                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
   PSSA_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&hebbian_kernel),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-  PSSA_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&sample_kernel<true>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, kSampleLdsMaxV * 4));
   return Status::Ok();
 }
 

@@ -561,6 +561,30 @@ def test_decode_sampling_wide_vocabulary_and_top_k(hip, vocab, penalty):
     layer.close()
 
 
+@pytest.mark.parametrize("vocab,equal", [(2, False), (1024, True), (16384, False), (16385, False), (16386, True),
+                                         (36864, False), (36865, False)])
+def test_decode_sampling_at_the_row_kernel_edges(hip, vocab, equal):
+    """The sampling kernels' vocabulary edges (16 and 36 ids per thread, then
+    the global row), aligned and odd rows; with equal logits every id ties for
+    the top-k, more than the candidate list holds.  The ids are the oracle's,
+    whose sum adds the probabilities one by one in id order; long prompts fill
+    the penalty window (64 ids) and wrap its ring."""
+    say("decode sampling, row kernel", vocab, equal)
+    cfg = PSSAConfig(depth=1, d_vocab=vocab, d_latent=64, d_state=32, d_mem_key=8, mem_capacity=16)
+    w = ModelWeights.init(cfg, 3, "baseline")
+    w.populate_banks(4, count=cfg.mem_capacity)
+    if equal:
+        w.unembed[:] = 0.0
+    ids = np.random.default_rng(2).integers(0, vocab, (2, 61), dtype=np.uint32)
+    ref = oracle_sampled_decode(w, ids, 8, 1.25, 0.9, 0.97, 64, seed=5)
+    layer = PSSALayer(hip, w, lanes=2, max_tokens=128)
+    layer.set_repetition_penalty(1.25)
+    layer.set_sampling(0.9, 0.97, 64, seed=5)
+    layer.prefill_inference(ids)
+    np.testing.assert_array_equal(layer.decode(8, graph=True), ref)
+    layer.close()
+
+
 def test_sampling_validation(hip):
     say("decode sampling validation")
     w = small_model(seed=2, depth=1)
