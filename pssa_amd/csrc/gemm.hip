@@ -1108,6 +1108,117 @@ static void launch_skinny_f32_kind(hipStream_t stream, int kind, dim3 grid, cons
 #undef PSSA_GEMM_SKF_CASE
 }
 
+// ---------------------------------------------------------------------------
+// fp32 GEMM of many tiles: 64 x 64 tiles, each of four waves one 32 x 32
+// block, operand slabs of 32 K (128-byte rows) by direct-to-LDS loads through
+// a ring of four slabs (16-byte chunk c of row r at c ^ (r & 7): conflict-free
+// fragment reads).  An fp32 MFMA takes 64 cycles for 32 x 32 x 2, so a small
+// tile already keeps the matrix cores fed from LDS (16 KB per 1024 cycles and
+// CU) and the many tiles fill the CUs evenly: a 128 x 128 tile is eight such
+// blocks in a row per wave, and one wave per 32 x 32 tile straight from
+// global memory reads each operand row once per tile.  Per output element the
+// MFMA sequence over K is theirs, so the bits are.  4001 x 768 x 400: 70 ->
+// 34.4 us (71 TFLOP/s of the 154 a large product reaches).
+constexpr int F32_T = 64, F32_BK = 32, F32_S = 4;
+constexpr int F32_SLAB = 2 * F32_T * F32_BK;  // floats: A's rows, then B's
+
+template <int KIND>
+__global__ __launch_bounds__(256) void gemm_f32_lds_kernel(const float* __restrict__ A, int lda,
+                                                           const float* __restrict__ B, int ldb, int M, int N, int K,
+                                                           int vec_epi, EpiParams ep) {
+  // Dynamic: for a static array the compiler waits out every direct load
+  // before any read of it.
+  extern __shared__ __attribute__((aligned(1024))) uint16_t gemm_f32_smem[];
+  typedef float f32x4_t __attribute__((ext_vector_type(4)));
+  const int tilesM = (M + F32_T - 1) / F32_T, tilesN = (N + F32_T - 1) / F32_T;
+  const int tile = xcd_tile(blockIdx.x, tilesM * tilesN);
+  const int m0 = (tile / tilesN) * F32_T, n0 = (tile % tilesN) * F32_T;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = lane >> 5, l32 = lane & 31, wm = wave & 1, wn = wave >> 1;
+
+  // Waves 0 and 1 load A's rows, 2 and 3 B's: eight rows per instruction,
+  // lane l the chunk of row l / 8 that belongs at position l % 8.
+  constexpr int PER = 2 * F32_T / 8 / 4;  // instructions per wave and slab
+  const int c4 = 4 * ((lane & 7) ^ (lane >> 3));
+  const float* src[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int r = (wave * PER + i) * 8 + (lane >> 3);
+    src[i] = r < F32_T ? A + (size_t)min(m0 + r, M - 1) * lda : B + (size_t)min(n0 + r - F32_T, N - 1) * ldb;
+  }
+  const int nk = (K + F32_BK - 1) / F32_BK;
+  auto issue = [&](int kt, int slot) {
+    const int k = min(min(kt, nk - 1) * F32_BK + c4, K - 4);  // chunks past K are not read below
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      __builtin_amdgcn_global_load_lds(
+          (const void*)(src[i] + k),
+          (__attribute__((address_space(3))) void*)(gemm_f32_smem + 2 * (slot * F32_SLAB + (wave * PER + i) * 8 * F32_BK)),
+          16, 0, 0);
+  };
+  f32x16_t acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+#pragma unroll
+  for (int kt = 0; kt < F32_S - 1; ++kt) issue(kt, kt);
+  const int ra = (wm * 32 + l32) * F32_BK, rb = (F32_T + wn * 32 + l32) * F32_BK, sw = l32 & 7;
+  for (int kt0 = 0; kt0 < nk; kt0 += F32_S) {
+#pragma unroll
+    for (int j = 0; j < F32_S; ++j) {
+      const int kt = kt0 + j;
+      if (kt >= nk) break;
+      __builtin_amdgcn_s_waitcnt(vmcnt_only((F32_S - 2) * PER));
+      __builtin_amdgcn_s_barrier();
+      issue(kt + F32_S - 1, (j + F32_S - 1) % F32_S);
+      const uint16_t* sl = gemm_f32_smem + 2 * j * F32_SLAB;
+      f32x4_t fa[4], fb[4];
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        const int c = 4 * ((2 * kk + half) ^ sw);
+        fa[kk] = *reinterpret_cast<const f32x4_t*>(sl + 2 * (ra + c));
+        fb[kk] = *reinterpret_cast<const f32x4_t*>(sl + 2 * (rb + c));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      auto step = [&](int kk) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[kk].x, fa[kk].x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[kk].y, fa[kk].y, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[kk].z, fa[kk].z, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[kk].w, fa[kk].w, acc, 0, 0, 0);
+      };
+      const int steps = (K - kt * F32_BK) / 8;
+      if (steps >= 4) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) step(kk);
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < 3; ++kk)
+          if (kk < steps) step(kk);
+      }
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(vmcnt_only(0));  // the reloads past the end
+  epilogue_32x32<float, KIND>(ep, acc, m0 + wm * 32 + l32, n0 + wn * 32, M, N, vec_epi, half, l32);
+}
+
+static void launch_f32_lds_kind(hipStream_t stream, int kind, unsigned grid, const float* A, int lda, const float* B,
+                                int ldb, int M, int N, int K, int ve, const EpiParams& ep) {
+#define PSSA_GEMM_F32_CASE(KD)                                                            \
+  case KD:                                                                                \
+    gemm_f32_lds_kernel<KD><<<grid, 256, F32_S * F32_SLAB * 4, stream>>>(A, lda, B, ldb, M, N, K, ve, ep); \
+    break;
+  switch (kind) {
+    PSSA_GEMM_F32_CASE(EPI_STORE)
+    PSSA_GEMM_F32_CASE(EPI_SEGMENTS)
+    PSSA_GEMM_F32_CASE(EPI_ADD_AUX)
+    PSSA_GEMM_F32_CASE(EPI_ZRAW)
+    PSSA_GEMM_F32_CASE(EPI_SILU)
+    PSSA_GEMM_F32_CASE(EPI_RESIDUAL)
+    PSSA_GEMM_F32_CASE(EPI_SCALE)
+    PSSA_GEMM_F32_CASE(EPI_SEGMENTS_TAP)
+  }
+#undef PSSA_GEMM_F32_CASE
+}
+
 template <typename T>
 static void launch_kind(hipStream_t stream, int kind, dim3 grid, const T* A, int lda, const T* B,
                         int ldb, int M, int N, int K, int vl, int ve, const EpiParams& ep) {
@@ -1387,6 +1498,20 @@ Status launch_gemm(hipStream_t stream, int dtype, const void* A, int lda, const 
     if (grid.y > 65535) return Status::Invalid("gemm: too many row groups");
     launch_skinny_kind<uint16_t, 1, 16>(stream, ep.kind, grid, a16, lda, b16, ldb, M, N, K, vec_epi, ep);
     PSSA_LAUNCH_CHECK("gemm_skinny");
+    return Status::Ok();
+  }
+  // fp32, 64 x 64 tiles through LDS from 96 tiles (below, their serial K
+  // chain is one tile's latency either way and the one-wave tiles straight
+  // from global memory start sooner: 512 x 512 x 128, 64 tiles, 6.6 us
+  // against 8.1), or where K is no multiple of 16, which the one-wave tiles
+  // need.  Old / new: 512 x 1056 x 128 9.4 / 8.8 us, 200 x 2096 x 768 29.4 /
+  // 22.5, 1000 x 1536 x 768 39.8 / 36.6, 4001 x 768 x 400 70.1 / 34.4, 16384 x
+  // 768 x 128 52.3 / 50.9, 77 x 1536 x 1544 234 / 38.7.
+  const long tiles64 = (long)((M + F32_T - 1) / F32_T) * ((N + F32_T - 1) / F32_T);
+  if (!bf16 && vec_load && K % 8 == 0 && (tiles64 >= 96 || K % 16 != 0) && tiles64 <= INT32_MAX) {
+    launch_f32_lds_kind(stream, ep.kind, (unsigned)tiles64, static_cast<const float*>(A), lda,
+                        static_cast<const float*>(B), ldb, M, N, K, vec_epi, ep);
+    PSSA_LAUNCH_CHECK("gemm_f32_lds");
     return Status::Ok();
   }
   if (!bf16 && vec_load && K % 16 == 0 && (long)((M + 127) / 128) * ((N + 127) / 128) < 128) {

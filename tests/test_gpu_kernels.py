@@ -49,6 +49,23 @@ def test_gemm_f32_few_rows_equal_tiled_rows_bitwise(hip, n):
     assert rel_err(big[:64], O.gemm_xwt(x[:64], w)) < 1e-5
 
 
+@pytest.mark.parametrize("m,n,k", [(385, 1030, 64), (1000, 640, 72), (70, 40, 24), (4100, 260, 8), (513, 769, 136)])
+def test_gemm_f32_lds_tiles_equal_few_rows_bitwise(hip, m, n, k):
+    """The 64 x 64-tile fp32 product (partial row, column and K tiles; K of one
+    and of several slabs) against the one-wave tiles (K % 16 == 0) or, where
+    those need another K, the same rows alone; and against f64."""
+    say("gemm f32 lds tiles", m, n, k)
+    rng = np.random.default_rng(m + n + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    w = rng.standard_normal((n, k)).astype(np.float32)
+    y = hip.try_dispatch_gemm(x, w, m, n, k).reshape(m, n)
+    for r0 in (0, m - 5):
+        np.testing.assert_array_equal(hip.try_dispatch_gemm(x[r0:r0 + 5], w, 5, n, k).reshape(5, n), y[r0:r0 + 5])
+    # k products and sums of fp32: k * 2^-24 of the terms' absolute sum.
+    bound = (k + 1) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T)
+    assert np.all(np.abs(y - x.astype(np.float64) @ w.astype(np.float64).T) <= bound)
+
+
 @pytest.mark.parametrize("n,k", [(768, 768), (1056, 768), (1000, 128), (736, 800), (1024, 800)])
 def test_gemm_bf16_few_rows_equal_tiled_rows_bitwise(hip, n, k):
     """bf16 weights: few token rows run one wave per 32 x 32 tile, with
@@ -375,6 +392,34 @@ def test_retrieve_full_soft_read(hip):
     np.testing.assert_array_equal(mn.view(np.uint32), r_min.view(np.uint32))
     assert not w[:, count:].any()
     np.testing.assert_allclose(w.sum(axis=1), 1.0, rtol=1e-5)
+
+
+@pytest.mark.parametrize("n_q,cap,count,dk,dv,k", [(1, 1, 1, 1, 1, 0), (5, 64, 63, 3, 5, 0), (6, 70, 60, 33, 33, 64),
+                                                   (2050, 128, 127, 32, 40, 0), (8200, 300, 257, 64, 36, 0),
+                                                   (37, 512, 512, 100, 768, 0), (9, 600, 512, 1024, 20, 0)])
+def test_full_soft_read_edges_match_oracle(hip, n_q, cap, count, dk, dv, k):
+    """Full reads over the slot, dimension and query edges: minima (and, with
+    k >= count, indices) bit for bit, weights and readout within 1e-5, the
+    gate of the hybrid read's, which a neutral read (gates 1, ages 0, lam 1)
+    reproduces bit for bit."""
+    say("retrieve full soft read", n_q, cap, count, dk, dv, k)
+    rng = np.random.default_rng(cap + dk)
+    keys, vals, q = ball(rng, count, dk), ball(rng, count, dv), ball(rng, n_q, dk)
+    q[0] = keys[count // 2]
+    K, N, V, cnt = bank(cap, keys, vals)
+    out, mn, idx, w = hip.retrieve(q, K, N, V, cnt, 0.1, top_k=k, want_weights=True)
+    r_out, r_mn, r_idx = O.retrieve_batch(K, N, V, cnt, q, 0.1, k, threads=8)
+    np.testing.assert_array_equal(mn, r_mn)
+    assert rel_err(out, r_out) < 1e-5
+    np.testing.assert_allclose(w[:, :cnt].sum(1), 1.0, atol=cnt * 2.0 ** -24)
+    assert not w[:, cnt:].any()
+    if k:
+        np.testing.assert_array_equal(idx[:, :cnt], np.broadcast_to(np.arange(cnt, dtype=np.uint32), (n_q, cnt)))
+        assert np.all(idx[:, cnt:] == 0xFFFFFFFF)
+    h = hip.retrieve_hybrid(q, K, N, V, cnt, 0.1, np.ones(cnt), np.zeros(cnt, np.uint64), 1.0, top_k=k,
+                            want_weights=True)
+    for x, y in zip((out, mn, w), (h[0], h[1], h[3])):
+        np.testing.assert_array_equal(x, y)
 
 
 def test_memory_forward_stage_matches_oracle(hip):
