@@ -40,6 +40,7 @@ struct RetrieveArgs {
   unsigned long long age_base = 0;
   int age_T = 0;
   const uint32_t* row_age = nullptr;
+  int row0 = 0;  // row of the call that row 0 here is (launch_retrieve's passes over parts of it)
   // Fused query product (a decode step's few-query soft read, see
   // retrieve_fuses_query): with qw set the Euclidean query of row r is
   // qa[r] . qw^T + qaux[r], qa [n, ld_qa] bf16 rows, qw [dk, qk] bf16

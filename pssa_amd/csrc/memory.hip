@@ -6,6 +6,7 @@
 // (sequential sums, no fused multiply-add, Rust's asinh formula), so the f32
 // distances, and with them the top-k indices, agree with the reference
 // (src/memory.rs:181-262).  The softmax weights and the value mix are fp32.
+#include "gemm.h"
 #include "memory.h"
 
 #include <algorithm>
@@ -655,6 +656,216 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(4))) v
       wave_sync();
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Full soft read with the reference's own distances, for banks of up to 512
+// slots: the reads retrieve_kernel would serve one query per pair of waves,
+// its lanes each walking a key row and one wave summing the readout (1.08 ms
+// for 4001 queries x 389 slots x 32, 768 wide, of which the readout most).
+// Here the keys pass through LDS transposed, 32 dimensions at a time, so lane
+// j reads slot j + 64q at consecutive addresses and one conversion to f64
+// serves QG queries; every squared difference, sum, distance, weight and sum
+// of weights is formed by the same operations in the same order as there, so
+// weights and minima carry the same bits, whichever kernel a call takes.
+// The readout is a product on the matrix cores (fp32): with it that read takes
+// 0.09 ms (50 us here, 34 us the product), against a floor of 16 us for the
+// product at the fp32 matrix rate.
+// Bound: f64 VALU issue (3 operations per query, slot and dimension, about
+// 200 for each distance's asinh).
+constexpr int SW_DC = 32;        // key dimensions per staged chunk
+constexpr int SW_WAVES = 4;
+constexpr int SW_SLOTS = 512;
+constexpr int SW_MAX_DK = 1024;
+
+static size_t soft_wide_lds(int dk, int spl, int qg) {
+  return ((size_t)(SW_DC * (64 * spl + 1) + 3) / 4 * 4 + (size_t)SW_WAVES * qg * ((dk + 3) & ~3)) * sizeof(float) +
+         (size_t)SW_WAVES * spl * 64 * sizeof(double);
+}
+
+// Readout operand: the weights again, [n, ldw] with zeros past the count.
+struct SoftReadout {
+  float* w = nullptr;
+  int ldw = 0;
+};
+
+template <int QG, int SPL>
+__global__ __launch_bounds__(64 * SW_WAVES) void soft_wide_kernel(RetrieveArgs a, SoftReadout ro) {
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  constexpr int KP = 64 * SPL + 1;
+  const int dk = a.dk, dk_pad = (dk + 3) & ~3;
+  const int cnt = a.count_dev ? a.count_dev[0] : a.count;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  float* keyT = smem;  // [SW_DC][KP]
+  double* sacc = reinterpret_cast<double*>(smem + (SW_DC * KP + 3) / 4 * 4) + wave * SPL * 64;  // [SPL][64]
+  float* rows = smem + (SW_DC * KP + 3) / 4 * 4 + 2 * SW_WAVES * SPL * 64 + wave * QG * dk_pad;  // [QG][dk_pad]
+  const int n0 = (blockIdx.x * SW_WAVES + wave) * QG;
+
+  // The wave's queries (rows past the last repeat it and write nothing).
+#pragma unroll
+  for (int g = 0; g < QG; ++g) {
+    const float* src = a.q + (size_t)min(n0 + g, a.n - 1) * a.ld_q;
+    for (int i = lane; i < dk; i += 64) rows[g * dk_pad + i] = src[i];
+  }
+  wave_sync();
+  float q_sq[QG];
+  {
+    // Lane g runs query g's sequential sums (diffeomorphic_project,
+    // src/memory.rs:194-211, then the ball's squared norm).
+    const float* mine = rows + min(lane, QG - 1) * dk_pad;
+    if (a.project) {
+      const double r = sqrt(sumsq_f64(mine, dk));
+      const double scale = r == 0.0 ? 1.0 : fmin(r / (1.0 + r), kMaxRadius) / r;
+      if (a.q_norm && lane < QG && n0 + lane < a.n) a.q_norm[n0 + lane] = (float)fmin(r, (double)FLT_MAX);
+      wave_sync();
+#pragma unroll
+      for (int g = 0; g < QG; ++g) {
+        const double sg = readlane_f64(scale, g);
+        for (int i = lane; i < dk; i += 64) rows[g * dk_pad + i] = (float)((double)rows[g * dk_pad + i] * sg);
+      }
+      wave_sync();
+    }
+    const float own = bank_norm_sq(mine, dk);
+#pragma unroll
+    for (int g = 0; g < QG; ++g) {
+      q_sq[g] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(own), g));
+      if (a.q_pnc && n0 + g < a.n)
+        for (int i = lane; i < dk; i += 64) a.q_pnc[(size_t)(n0 + g) * dk + i] = rows[g * dk_pad + i];
+    }
+  }
+
+  double sq[QG][SPL];
+#pragma unroll
+  for (int g = 0; g < QG; ++g)
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) sq[g][j] = 0.0;
+  const bool vec = dk % 4 == 0 && ((uintptr_t)a.keys & 15) == 0;
+  for (int c0 = 0; c0 < dk; c0 += SW_DC) {
+    const int dc = min(SW_DC, dk - c0);
+    __syncthreads();
+    if (vec) {
+      constexpr int PC = SW_DC / 4;  // 16-byte pieces of a slot's chunk
+      constexpr int U = 16;          // loads in flight per thread: a chunk of 512 slots in one round
+      for (int e0 = tid; e0 < cnt * PC; e0 += U * 64 * SW_WAVES) {
+        float4 v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int e = min(e0 + u * 64 * SW_WAVES, cnt * PC - 1);
+          v[u] = *reinterpret_cast<const float4*>(a.keys + (size_t)(e / PC) * dk + c0 + min(4 * (e % PC), dc - 4));
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int e = e0 + u * 64 * SW_WAVES, i = 4 * (e % PC);
+          if (e < cnt * PC && i < dc) {
+            float* k = keyT + i * KP + e / PC;
+            k[0] = v[u].x, k[KP] = v[u].y, k[2 * KP] = v[u].z, k[3 * KP] = v[u].w;
+          }
+        }
+      }
+    } else {
+      for (int e = tid; e < cnt * SW_DC; e += 64 * SW_WAVES) {
+        const int i = e % SW_DC;
+        if (i < dc) keyT[i * KP + e / SW_DC] = a.keys[(size_t)(e / SW_DC) * dk + c0 + i];
+      }
+    }
+    __syncthreads();
+    // Lane i keeps dimension c0 + i of each query, widened; the products
+    // take it as a wave-uniform operand.  Slots past the count read whatever
+    // that part of keyT holds; their results are dropped.
+    double qd[QG];
+#pragma unroll
+    for (int g = 0; g < QG; ++g) qd[g] = (double)rows[g * dk_pad + min(c0 + (lane & (SW_DC - 1)), dk - 1)];
+    for (int i = 0; i < dc; ++i) {
+#pragma clang fp contract(off)
+      const float* kr = keyT + i * KP + lane;
+      double kv[SPL];
+#pragma unroll
+      for (int j = 0; j < SPL; ++j) kv[j] = (double)kr[64 * j];
+#pragma unroll
+      for (int g = 0; g < QG; ++g) {
+        const double qv = readlane_f64(qd[g], i);
+#pragma unroll
+        for (int j = 0; j < SPL; ++j) {
+          const double t = qv - kv[j];
+          sq[g][j] = sq[g][j] + t * t;
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < QG; ++g) {
+    const int n = n0 + g;
+    if (n >= a.n) break;
+    // The distances, one asinh in the code: the sums pass through the lane's
+    // own LDS cells so the loop over them need not be unrolled.
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) sacc[j * 64 + lane] = sq[g][j];
+    float local_min = FLT_MAX;
+    for (int j = 0; j < SPL; ++j) {
+      const int s = lane + 64 * j;
+      if (s < cnt) {
+#pragma clang fp contract(off)
+        const double den = (1.0 - (double)q_sq[g]) * (1.0 - (double)a.norm_sq[s]);
+        const float d = (float)(2.0 * rust_asinh(sqrt(sacc[s] / den)));
+        sacc[s] = (double)d;
+        local_min = fminf(local_min, d);
+      }
+    }
+    const float min_dist = cnt > 0 ? wave_min(local_min) : 0.0f;
+    if (a.out_min && lane == 0) a.out_min[n] = min_dist;
+    float e[SPL], part = 0.0f;
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) {
+      const int s = lane + 64 * j;
+      e[j] = 0.0f;
+      if (s < cnt) {
+        e[j] = expf((min_dist - (float)sacc[s]) / a.tau);
+        part += e[j];
+      }
+    }
+    float sum = wave_sum(part);
+    if (a.hgate) {  // hybrid: (e * gate) * decay, unless every such weight is zero
+      float part_h = 0.0f;
+      for (int j = 0; j < SPL; ++j) {
+        const int s = lane + 64 * j;
+        if (s < cnt) {
+          const float eh = (expf((min_dist - (float)sacc[s]) / a.tau) * a.hgate[s]) * hybrid_decay(a, s, a.row0 + n);
+          sacc[s] = (double)eh;
+          part_h += eh;
+        }
+      }
+      const float sum_h = wave_sum(part_h);
+      if (sum_h != 0.0f) {
+        sum = sum_h;
+#pragma unroll
+        for (int j = 0; j < SPL; ++j) e[j] = lane + 64 * j < cnt ? (float)sacc[lane + 64 * j] : 0.0f;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) {
+      const int s = lane + 64 * j;
+      const float w = s < cnt ? e[j] / sum : 0.0f;
+      if (s < a.capacity) put_weight(a, n, s, w);
+      if (ro.w && s < ro.ldw) ro.w[(size_t)n * ro.ldw + s] = w;
+    }
+    for (int s = lane + 64 * SPL; s < a.capacity; s += 64) put_weight(a, n, s, 0.0f);
+    if (a.out_idx)
+      for (int r = lane; r < a.top_k; r += 64)
+        a.out_idx[(size_t)n * a.top_k + r] = r < cnt ? (uint32_t)r : 0xFFFFFFFFu;
+  }
+}
+
+// out[j, s] = values[s, j] for s < cnt, zeros for cnt <= s < ld: the readout
+// product's operand.
+__global__ __launch_bounds__(256) void soft_values_kernel(const float* __restrict__ values, int cnt, int dv,
+                                                          float* __restrict__ out, int ld) {
+  __shared__ float tile[32][33];
+  const int s0 = blockIdx.x * 32, j0 = blockIdx.y * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  for (int r = ty; r < 32; r += 8)
+    tile[r][tx] = s0 + r < cnt && j0 + tx < dv ? values[(size_t)(s0 + r) * dv + j0 + tx] : 0.0f;
+  __syncthreads();
+  for (int r = ty; r < 32; r += 8)
+    if (j0 + r < dv && s0 + tx < ld) out[(size_t)(j0 + r) * ld + s0 + tx] = tile[tx][r];
 }
 
 // ---------------------------------------------------------------------------
@@ -1347,8 +1558,33 @@ static bool ranked_read_fits(const RetrieveArgs& a) {
          ((uintptr_t)a.q & 15) == 0 && ((uintptr_t)a.keys & 15) == 0;
 }
 
+static bool soft_read_fits(const RetrieveArgs& a);
+
+// The wide soft read: full reads (no ranking) of banks of up to 512 slots.
+// Without a readout (a model's read, which multiplies the weights itself) from
+// 1024 queries: fewer leave most CUs without a workgroup while each stages
+// the whole bank (128-wide keys, two layers: 512 queries 66 us general / 78
+// wide, 1024 95 / 82, 8192 707 / 319).
+constexpr int SW_MIN_WEIGHTS = 1024;
+static bool soft_wide_fits(const RetrieveArgs& a) {
+  return (a.top_k == 0 || (!a.count_dev && a.top_k >= a.count)) && a.count > 0 && a.count <= SW_SLOTS &&
+         a.dk <= SW_MAX_DK && !(a.out_val && a.count_dev) && !soft_read_fits(a) &&
+         (a.out_val || a.n >= SW_MIN_WEIGHTS);
+}
+// Readout width (the count in whole 16-wide K steps) and queries per pass.
+static int soft_wide_ld(const RetrieveArgs& a) { return (a.count + 15) & ~15; }
+static int soft_wide_chunk(const RetrieveArgs& a) { return std::min(a.n, a.chunk > 0 ? a.chunk : 32768); }
+static size_t soft_wide_scratch(const RetrieveArgs& a) {
+  return (size_t)soft_wide_ld(a) * ((size_t)soft_wide_chunk(a) + a.dv) * sizeof(float);
+}
+
 size_t retrieve_scratch_bytes(const RetrieveArgs& a) {
-  return ranked_read_fits(a) ? ranked_scratch_bytes(a.dk, ranked_chunk(a)) : 0;
+  if (ranked_read_fits(a)) return ranked_scratch_bytes(a.dk, ranked_chunk(a));
+  if (!a.out_val || !soft_wide_fits(a)) return 0;
+  // The allocation-free call's scratch is a fixed size: reads that need more
+  // keep the general kernel.
+  const size_t bytes = soft_wide_scratch(a);
+  return a.chunk > 0 && bytes > kNoallocScratchBytes ? 0 : bytes;
 }
 
 Status noalloc_scratch_address(void** out) {
@@ -1399,6 +1635,16 @@ static Status allow_large_lds() {
       PSSA_SOFT_QP_FN(1) PSSA_SOFT_QP_FN(2) PSSA_SOFT_QP_FN(4) PSSA_SOFT_QP_FN(8)
 #undef PSSA_SOFT_QP_FN
   };
+  const void* wide[] = {
+#define PSSA_SOFT_WIDE_FN(SPL)                                       \
+  reinterpret_cast<const void*>(&soft_wide_kernel<1, SPL>),          \
+      reinterpret_cast<const void*>(&soft_wide_kernel<2, SPL>),      \
+      reinterpret_cast<const void*>(&soft_wide_kernel<4, SPL>),
+      PSSA_SOFT_WIDE_FN(1) PSSA_SOFT_WIDE_FN(2) PSSA_SOFT_WIDE_FN(4) PSSA_SOFT_WIDE_FN(8)
+#undef PSSA_SOFT_WIDE_FN
+  };
+  for (const void* f : wide)
+    PSSA_HIP_TRY(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
   for (const void* f : soft)
     PSSA_HIP_TRY(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
   PSSA_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&ranked_dot_kernel),
@@ -1432,6 +1678,57 @@ bool retrieve_fuses_query(const RetrieveArgs& a) {
   return nwv == SOFT_WAVES_FEW && per == 1 && a.dk <= 32 && a.qk > 0 && a.qk % 128 == 0 &&
          a.ld_qa % 8 == 0 && ((uintptr_t)a.qa & 15) == 0 && ((uintptr_t)a.qw & 15) == 0 &&
          soft_read_lds(a.dk, a.capacity, 1, nwv) + soft_qp_lds(a.qk, nwv) <= 160 * 1024;
+}
+
+// Queries per wave: enough workgroups for two per CU before a wave takes more
+// queries per pass over the keys.
+static int soft_wide_qg(int n) {
+  const int wg1 = (n + SW_WAVES - 1) / SW_WAVES;
+  return wg1 >= 2048 ? 4 : wg1 >= 512 ? 2 : 1;
+}
+
+static Status launch_soft_wide(hipStream_t stream, const RetrieveArgs& a) {
+  PSSA_RETURN_IF(allow_large_lds());
+  const int spl = soft_spl(a.count), ld = soft_wide_ld(a);
+  const int chunk = a.out_val ? soft_wide_chunk(a) : a.n;
+  float* vt = nullptr;
+  SoftReadout ro;
+  if (a.out_val) {
+    vt = static_cast<float*>(a.scratch);
+    ro.w = vt + (size_t)ld * a.dv;
+    ro.ldw = ld;
+    soft_values_kernel<<<dim3((ld + 31) / 32, (a.dv + 31) / 32), 256, 0, stream>>>(a.values, a.count, a.dv, vt, ld);
+    PSSA_LAUNCH_CHECK("soft_values");
+  }
+  for (int q0 = 0; q0 < a.n; q0 += chunk) {
+    RetrieveArgs c = a;
+    c.n = std::min(chunk, a.n - q0);
+    c.q = a.q + (size_t)q0 * a.ld_q;
+    c.row0 = q0;
+    if (a.q_pnc) c.q_pnc = a.q_pnc + (size_t)q0 * a.dk;
+    if (a.q_norm) c.q_norm = a.q_norm + q0;
+    if (a.weights) c.weights = a.weights + (size_t)q0 * a.capacity;
+    if (a.weights16) c.weights16 = a.weights16 + (size_t)q0 * a.capacity;
+    if (a.out_min) c.out_min = a.out_min + q0;
+    if (a.out_idx) c.out_idx = a.out_idx + (size_t)q0 * a.top_k;
+    const int qg = soft_wide_qg(c.n);
+    const unsigned blocks = (unsigned)((c.n + SW_WAVES * qg - 1) / (SW_WAVES * qg));
+    const size_t lds = soft_wide_lds(a.dk, spl, qg);
+#define PSSA_SOFT_WIDE(QG, SPL) \
+  if (qg == QG && spl == SPL) soft_wide_kernel<QG, SPL><<<blocks, 64 * SW_WAVES, lds, stream>>>(c, ro);
+    PSSA_SOFT_WIDE(1, 1) PSSA_SOFT_WIDE(1, 2) PSSA_SOFT_WIDE(1, 4) PSSA_SOFT_WIDE(1, 8)
+    PSSA_SOFT_WIDE(2, 1) PSSA_SOFT_WIDE(2, 2) PSSA_SOFT_WIDE(2, 4) PSSA_SOFT_WIDE(2, 8)
+    PSSA_SOFT_WIDE(4, 1) PSSA_SOFT_WIDE(4, 2) PSSA_SOFT_WIDE(4, 4) PSSA_SOFT_WIDE(4, 8)
+#undef PSSA_SOFT_WIDE
+    PSSA_LAUNCH_CHECK("soft_wide");
+    if (a.out_val) {
+      EpiParams ep;
+      ep.out32 = a.out_val + (size_t)q0 * a.dv;
+      ep.ld32 = a.dv;
+      PSSA_RETURN_IF(launch_gemm(stream, PSSA_HIP_F32, ro.w, ld, vt, ld, c.n, a.dv, ld, ep));
+    }
+  }
+  return Status::Ok();
 }
 
 Status launch_retrieve(hipStream_t stream, const RetrieveArgs& a) {
@@ -1513,6 +1810,8 @@ Status launch_retrieve(hipStream_t stream, const RetrieveArgs& a) {
     }
     return Status::Ok();
   }
+  if (soft_wide_fits(a) && (!a.out_val || (a.scratch && retrieve_scratch_bytes(a) && a.scratch_bytes >= retrieve_scratch_bytes(a))))
+    return launch_soft_wide(stream, a);
   const int dk_pad = (a.dk + 3) & ~3;
   const size_t lds = (size_t)RETRIEVE_QPB * (dk_pad + a.capacity) * sizeof(float);
   if (lds > 128 * 1024) return Status::Invalid("retrieve: d_key + capacity too large for LDS");
