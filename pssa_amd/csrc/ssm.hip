@@ -702,8 +702,17 @@ constexpr long kScanFullGrid = 768;
 // 9.93; serialised scan stage, 16 lanes (3072) 4.71 / 4.20 ms, 18 lanes
 // 4.73 / 4.82.  Small model, scan stage: 64 lanes x 256 (1024) 0.120 / 0.098
 // ms, 128 x 128 (2048) 0.082 / 0.098.
+// Under 32 steps a workgroup's loading of its states is much of its work, and
+// only grids that are resident at once (three workgroups per CU) gain: whole
+// prefills of 6 lanes x 12 (1152) 0.974 / 1.035 ms, 10 x 24 (1920) 1.10 / 1.17,
+// but 3 x 33 (576) 1.10 / 1.01; up to 64 the line lies between 5 x 50 (960)
+// 1.22 / 1.15 and 16 x 60 (3072) 1.86 / 1.90.
 constexpr int kQuadChannels = 8;
 constexpr long kQuadMax = 1536;
+static long quad_limit(const SsmArgs& a, bool four_states) {
+  if (a.T < 32) return kQuadMax / 2;
+  return four_states && !a.concurrent && a.T >= 64 ? 2 * kQuadMax : kQuadMax;
+}
 
 // From four workgroups per CU up to where the few-lane scan ends.  105M
 // prefill, two groups / one: 4 lanes x 512 (768 workgroups) 2.65 / 2.73 ms, 8
@@ -765,7 +774,7 @@ static void launch_j(hipStream_t stream, const SsmArgs& a, bool mat) {
     }
   } else if (a.T < SSM_TC && !a.spans) {
     ssm_materialize_kernel<J, false><<<grid, 256, 0, stream>>>(a);
-  } else if (J >= 8 && quad_workgroups<J>(a, qgrid) <= (J == 32 && !a.concurrent ? 2 : 1) * kQuadMax) {
+  } else if (J >= 8 && quad_workgroups<J>(a, qgrid) <= quad_limit(a, J == 32)) {
     constexpr int M = J == 32 ? 4 : 2;
     const bool vec = a.s % 4 == 0 && a.ld_b % 4 == 0 && a.ld_c % 4 == 0 && ((uintptr_t)a.bproj & 15) == 0 &&
                      ((uintptr_t)a.cproj & 15) == 0;
