@@ -24,15 +24,22 @@ using pssa::Status;
 
 namespace {
 
-Status upload(DevBuf& dst, const void* src, size_t bytes, hipStream_t st) {
+// A temporary of one call (its block returns to the context's pool) holding
+// a host array.
+Status upload(pssa_hip_ctx* ctx, DevBuf& dst, const void* src, size_t bytes) {
+  PSSA_RETURN_IF(dst.alloc(bytes, &ctx->pool));
+  return ctx->stage.to_device(dst.p, src, bytes, ctx->stream);
+}
+// The same for a buffer that stays (model parameters, cached weights): moved
+// by the runtime, `src` must outlive the copy.
+Status upload_keep(pssa_hip_ctx* ctx, DevBuf& dst, const void* src, size_t bytes) {
   PSSA_RETURN_IF(dst.alloc(bytes));
-  if (bytes) PSSA_HIP_TRY(hipMemcpyAsync(dst.p, src, bytes, hipMemcpyHostToDevice, st));
+  if (bytes) PSSA_HIP_TRY(hipMemcpyAsync(dst.p, src, bytes, hipMemcpyHostToDevice, ctx->stream));
   return Status::Ok();
 }
 
-Status download(void* dst, const DevBuf& src, size_t bytes, hipStream_t st) {
-  if (bytes) PSSA_HIP_TRY(hipMemcpyAsync(dst, src.p, bytes, hipMemcpyDeviceToHost, st));
-  return Status::Ok();
+Status download(pssa_hip_ctx* ctx, void* dst, const DevBuf& src, size_t bytes) {
+  return ctx->stage.to_host(dst, src.p, bytes, ctx->stream);
 }
 
 uint16_t bf16_bits(float f) {
@@ -43,12 +50,12 @@ uint16_t bf16_bits(float f) {
 }
 
 // Weight upload in the model's storage type.
-Status upload_weight(DevBuf& dst, const float* src, size_t n, int dtype, hipStream_t st) {
-  if (dtype == PSSA_HIP_F32) return upload(dst, src, n * 4, st);
+Status upload_weight(pssa_hip_ctx* ctx, DevBuf& dst, const float* src, size_t n, int dtype) {
+  if (dtype == PSSA_HIP_F32) return upload_keep(ctx, dst, src, n * 4);
   std::vector<uint16_t> tmp(n);
   for (size_t i = 0; i < n; ++i) tmp[i] = bf16_bits(src[i]);
-  PSSA_RETURN_IF(upload(dst, tmp.data(), n * 2, st));
-  PSSA_HIP_TRY(hipStreamSynchronize(st));  // tmp must outlive the copy
+  PSSA_RETURN_IF(upload_keep(ctx, dst, tmp.data(), n * 2));
+  PSSA_HIP_TRY(hipStreamSynchronize(ctx->stream));  // tmp must outlive the copy
   return Status::Ok();
 }
 
@@ -106,7 +113,7 @@ Status cap_bank_values(pssa_hip_model* M, const std::vector<pssa::DevBlock*>& bl
                                            (size_t)d, caps, C, bad.as<int>()));
   }
   int flag = 0;
-  PSSA_RETURN_IF(download(&flag, bad, 4, st));
+  PSSA_RETURN_IF(download(M->ctx, &flag, bad, 4));
   PSSA_RETURN_IF(sync(M->ctx));
   if (flag) return Status::Invalid("capped memory value must be finite");
   if (M->dtype == PSSA_HIP_BF16) PSSA_RETURN_IF(tmp.alloc(bytes));
@@ -139,10 +146,10 @@ Status cached_weight(pssa_hip_ctx* ctx, const void* host, size_t n, int dtype, c
   auto it = ctx->weights.find(key);
   if (it == ctx->weights.end()) {
     pssa_hip_ctx::CachedWeight cw;
-    PSSA_RETURN_IF(upload(cw.buf, host, bytes, ctx->stream));
+    PSSA_RETURN_IF(upload_keep(ctx, cw.buf, host, bytes));
     it = ctx->weights.emplace(key, std::move(cw)).first;
   } else if (!it->second.current) {
-    PSSA_HIP_TRY(hipMemcpyAsync(it->second.buf.p, host, bytes, hipMemcpyHostToDevice, ctx->stream));
+    PSSA_RETURN_IF(ctx->stage.to_device(it->second.buf.p, host, bytes, ctx->stream));
     it->second.current = true;
   }
   *out = it->second.buf.p;
@@ -158,7 +165,7 @@ Status stage_ids_locked(pssa_hip_lanes* L, const uint32_t* ids, size_t n_lanes, 
   for (size_t i = 0; i < n_lanes * T; ++i)
     if (ids[i] >= V)
       return Status::Invalid("prompt ID " + std::to_string(ids[i]) + " outside model vocabulary");
-  PSSA_HIP_TRY(hipMemcpyAsync(L->ids.p, ids, n_lanes * T * 4, hipMemcpyHostToDevice, L->ctx->stream));
+  PSSA_RETURN_IF(L->ctx->stage.to_device(L->ids.p, ids, n_lanes * T * 4, L->ctx->stream));
   L->staged_lanes = n_lanes;
   L->staged_len = T;
   return Status::Ok();
@@ -192,6 +199,7 @@ int pssa_hip_init(int device, pssa_hip_ctx** out, char* err, size_t err_len) {
     ctx->name = prop.name;
     ctx->cu_count = prop.multiProcessorCount;
     PSSA_HIP_TRY(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
+    PSSA_RETURN_IF(ctx->stage.init());
     PSSA_RETURN_IF(pssa::init_gemm_attributes());
     PSSA_RETURN_IF(pssa::init_retrieve_attributes());
     PSSA_RETURN_IF(pssa::init_decode_attributes());
@@ -260,7 +268,12 @@ int pssa_hip_memcpy(pssa_hip_ctx* ctx, void* dst, const void* src, size_t bytes,
     const hipMemcpyKind k = kind == PSSA_HIP_H2D ? hipMemcpyHostToDevice
                             : kind == PSSA_HIP_D2H ? hipMemcpyDeviceToHost
                                                    : hipMemcpyDeviceToDevice;
-    PSSA_HIP_TRY(hipMemcpyAsync(dst, src, bytes, k, ctx->stream));
+    if (k == hipMemcpyHostToDevice)
+      PSSA_RETURN_IF(ctx->stage.to_device(dst, src, bytes, ctx->stream));
+    else if (k == hipMemcpyDeviceToHost)
+      PSSA_RETURN_IF(ctx->stage.to_host(dst, src, bytes, ctx->stream));
+    else
+      PSSA_HIP_TRY(hipMemcpyAsync(dst, src, bytes, k, ctx->stream));
     return sync(ctx);
   };
   return pssa::finish(body(), err, err_len);
@@ -299,14 +312,14 @@ int pssa_hip_gemm_xwt(pssa_hip_ctx* ctx, const float* x, size_t x_len, const voi
     std::lock_guard<std::mutex> g(ctx->mu);
     PSSA_HIP_TRY(hipSetDevice(ctx->device));
     DevBuf dx, dxh, dy;
-    PSSA_RETURN_IF(upload(dx, x, xin * 4, ctx->stream));
+    PSSA_RETURN_IF(upload(ctx, dx, x, xin * 4));
     const void* dw = nullptr;
     PSSA_RETURN_IF(cached_weight(ctx, w, win, w_dtype, &dw));
-    PSSA_RETURN_IF(dy.alloc(yout * 4));
+    PSSA_RETURN_IF(dy.alloc(yout * 4, &ctx->pool));
     const void* a = dx.p;
     if (w_dtype == PSSA_HIP_BF16) {
       // bf16 weights multiply bf16-rounded activations (fp32 accumulation).
-      PSSA_RETURN_IF(dxh.alloc(xin * 2));
+      PSSA_RETURN_IF(dxh.alloc(xin * 2, &ctx->pool));
       PSSA_RETURN_IF(pssa::launch_to_bf16(ctx->stream, dx.as<float>(), (int)k, dxh.as<uint16_t>(), (int)k, rows, (int)k));
       a = dxh.p;
     }
@@ -314,7 +327,7 @@ int pssa_hip_gemm_xwt(pssa_hip_ctx* ctx, const float* x, size_t x_len, const voi
     ep.out32 = dy.as<float>();
     ep.ld32 = (int)n;
     PSSA_RETURN_IF(pssa::launch_gemm(ctx->stream, w_dtype, a, (int)k, dw, (int)k, (int)rows, (int)n, (int)k, ep));
-    PSSA_RETURN_IF(download(y, dy, yout * 4, ctx->stream));
+    PSSA_RETURN_IF(download(ctx, y, dy, yout * 4));
     return sync(ctx);
   };
   return pssa::finish(body(), err, err_len);
@@ -330,32 +343,32 @@ static Status gemm_transposed(pssa_hip_ctx* ctx, const float* x, const float* w,
   PSSA_HIP_TRY(hipSetDevice(ctx->device));
   const hipStream_t st = ctx->stream;
   DevBuf dx, dw, dxt, dwt, dy, dacc;
-  PSSA_RETURN_IF(upload(dx, x, rows * k * 4, st));
-  PSSA_RETURN_IF(upload(dw, w, n * k * 4, st));
+  PSSA_RETURN_IF(upload(ctx, dx, x, rows * k * 4));
+  PSSA_RETURN_IF(upload(ctx, dw, w, n * k * 4));
   const float* xa = dx.as<float>();
   const float* wa = dw.as<float>();
   if (x_t) {  // [k, rows] -> [rows, k]
-    PSSA_RETURN_IF(dxt.alloc(rows * k * 4));
+    PSSA_RETURN_IF(dxt.alloc(rows * k * 4, &ctx->pool));
     PSSA_RETURN_IF(pssa::launch_transpose(st, xa, dxt.as<float>(), 1, (int)k, (int)rows, 1.0f));
     xa = dxt.as<float>();
   }
   if (w_t) {  // [k, n] -> [n, k]
-    PSSA_RETURN_IF(dwt.alloc(n * k * 4));
+    PSSA_RETURN_IF(dwt.alloc(n * k * 4, &ctx->pool));
     PSSA_RETURN_IF(pssa::launch_transpose(st, wa, dwt.as<float>(), 1, (int)k, (int)n, 1.0f));
     wa = dwt.as<float>();
   }
-  PSSA_RETURN_IF(dy.alloc(rows * n * 4));
+  PSSA_RETURN_IF(dy.alloc(rows * n * 4, &ctx->pool));
   pssa::EpiParams ep;
   ep.out32 = dy.as<float>();
   ep.ld32 = (int)n;
   if (accumulate) {
-    PSSA_RETURN_IF(upload(dacc, y, rows * n * 4, st));
+    PSSA_RETURN_IF(upload(ctx, dacc, y, rows * n * 4));
     ep.kind = pssa::EPI_ADD_AUX;
     ep.aux = dacc.as<float>();
     ep.ld_aux = (int)n;
   }
   PSSA_RETURN_IF(pssa::launch_gemm(st, PSSA_HIP_F32, xa, (int)k, wa, (int)k, (int)rows, (int)n, (int)k, ep));
-  PSSA_RETURN_IF(download(y, dy, rows * n * 4, st));
+  PSSA_RETURN_IF(download(ctx, y, dy, rows * n * 4));
   return sync(ctx);
 }
 
@@ -446,9 +459,9 @@ int pssa_hip_softplus_in_place(pssa_hip_ctx* ctx, float* values, size_t len, cha
     std::lock_guard<std::mutex> g(ctx->mu);
     PSSA_HIP_TRY(hipSetDevice(ctx->device));
     DevBuf dv;
-    PSSA_RETURN_IF(upload(dv, values, len * 4, ctx->stream));
+    PSSA_RETURN_IF(upload(ctx, dv, values, len * 4));
     PSSA_RETURN_IF(pssa::launch_softplus(ctx->stream, dv.as<float>(), len));
-    PSSA_RETURN_IF(download(values, dv, len * 4, ctx->stream));
+    PSSA_RETURN_IF(download(ctx, values, dv, len * 4));
     return sync(ctx);
   };
   return pssa::finish(body(), err, err_len);
@@ -488,17 +501,17 @@ static Status run_stage_ssm(pssa_hip_ctx* ctx, const float* delta, const float* 
   t.d = d_m;
   t.s = d_s;
   DevBuf dd, db, dx, dr, dc, dr2;
-  PSSA_RETURN_IF(upload(dd, delta, ld * 4, st));
-  PSSA_RETURN_IF(upload(db, b_proj, ls * 4, st));
-  PSSA_RETURN_IF(upload(dx, x_norm, ld * 4, st));
-  PSSA_RETURN_IF(upload(dr, rates, w * 4, st));
-  PSSA_RETURN_IF(upload(dc, c_proj, ls * 4, st));
-  PSSA_RETURN_IF(upload(t.carry_ds, initial, w * 4, st));
-  PSSA_RETURN_IF(t.y.alloc(ld * 4));
+  PSSA_RETURN_IF(upload(ctx, dd, delta, ld * 4));
+  PSSA_RETURN_IF(upload(ctx, db, b_proj, ls * 4));
+  PSSA_RETURN_IF(upload(ctx, dx, x_norm, ld * 4));
+  PSSA_RETURN_IF(upload(ctx, dr, rates, w * 4));
+  PSSA_RETURN_IF(upload(ctx, dc, c_proj, ls * 4));
+  PSSA_RETURN_IF(upload(ctx, t.carry_ds, initial, w * 4));
+  PSSA_RETURN_IF(t.y.alloc(ld * 4, &ctx->pool));
   // The scan keeps rates state-major ([s, d]) and states channel-blocked
   // (pssa::carry_at); the stage API speaks the reference's [d, s].
-  PSSA_RETURN_IF(dr2.alloc(w * 4));
-  PSSA_RETURN_IF(t.carry.alloc(w * 4));
+  PSSA_RETURN_IF(dr2.alloc(w * 4, &ctx->pool));
+  PSSA_RETURN_IF(t.carry.alloc(w * 4, &ctx->pool));
   PSSA_RETURN_IF(pssa::launch_transpose(st, dr.as<float>(), dr2.as<float>(), 1, (int)d_m, (int)d_s,
                                         1.4426950408889634f));
   PSSA_RETURN_IF(pssa::launch_carry_convert(st, t.carry_ds.as<float>(), t.carry.as<float>(), 1, (int)d_m, (int)d_s,
@@ -525,13 +538,13 @@ static Status run_stage_ssm(pssa_hip_ctx* ctx, const float* delta, const float* 
   DevBuf dpart;
   const int nz = pssa::ssm_state_blocks((int)d_s);
   if (!materialize && nz > 2) {
-    PSSA_RETURN_IF(dpart.alloc((size_t)nz * ld * 4));
+    PSSA_RETURN_IF(dpart.alloc((size_t)nz * ld * 4, &ctx->pool));
     a.y_part = dpart.as<float>();
   }
   if (materialize) {
-    PSSA_RETURN_IF(t.bar_a.alloc(seq_len * w * 4));
-    PSSA_RETURN_IF(t.bar_b.alloc(seq_len * w * 4));
-    PSSA_RETURN_IF(t.states.alloc((seq_len + 1) * w * 4));
+    PSSA_RETURN_IF(t.bar_a.alloc(seq_len * w * 4, &ctx->pool));
+    PSSA_RETURN_IF(t.bar_b.alloc(seq_len * w * 4, &ctx->pool));
+    PSSA_RETURN_IF(t.states.alloc((seq_len + 1) * w * 4, &ctx->pool));
     a.bar_a = t.bar_a.as<float>();
     a.bar_b = t.bar_b.as<float>();
     a.states = t.states.as<float>();
@@ -546,15 +559,15 @@ static Status download_ssm(pssa_hip_ctx* ctx, SsmTape& t, float* bar_a, float* b
                            float* final_state) {
   const hipStream_t st = ctx->stream;
   const size_t ld = t.L * t.d, w = t.d * t.s;
-  if (y_ssm) PSSA_RETURN_IF(download(y_ssm, t.y, ld * 4, st));
+  if (y_ssm) PSSA_RETURN_IF(download(ctx, y_ssm, t.y, ld * 4));
   if (final_state) {
     PSSA_RETURN_IF(pssa::launch_carry_convert(st, t.carry.as<float>(), t.carry_ds.as<float>(), 1, (int)t.d, (int)t.s,
                                               false));
-    PSSA_RETURN_IF(download(final_state, t.carry_ds, w * 4, st));
+    PSSA_RETURN_IF(download(ctx, final_state, t.carry_ds, w * 4));
   }
-  if (bar_a) PSSA_RETURN_IF(download(bar_a, t.bar_a, t.L * w * 4, st));
-  if (bar_b) PSSA_RETURN_IF(download(bar_b, t.bar_b, t.L * w * 4, st));
-  if (states) PSSA_RETURN_IF(download(states, t.states, (t.L + 1) * w * 4, st));
+  if (bar_a) PSSA_RETURN_IF(download(ctx, bar_a, t.bar_a, t.L * w * 4));
+  if (bar_b) PSSA_RETURN_IF(download(ctx, bar_b, t.bar_b, t.L * w * 4));
+  if (states) PSSA_RETURN_IF(download(ctx, states, t.states, (t.L + 1) * w * 4));
   return sync(ctx);
 }
 
@@ -629,22 +642,22 @@ static Status run_stage_memory(pssa_hip_ctx* ctx, const float* x_norm, const flo
   const hipStream_t st = ctx->stream;
   const int L = (int)seq_len, d = (int)d_m, k = (int)d_k, C = (int)capacity;
   DevBuf dx, dwqx, dwqh, dwg, dwp, dk_, dn, dv, dvt, qx, qe, qp, qn, wts, mv, gm, mp, mi;
-  PSSA_RETURN_IF(upload(dx, x_norm, (size_t)L * d * 4, st));
-  PSSA_RETURN_IF(upload(dwqx, w_qx, (size_t)k * d * 4, st));
-  PSSA_RETURN_IF(upload(dwqh, w_qh, (size_t)k * d * 4, st));
-  PSSA_RETURN_IF(upload(dwg, w_gate, (size_t)d * d * 4, st));
-  PSSA_RETURN_IF(upload(dwp, w_proj, (size_t)d * d * 4, st));
-  PSSA_RETURN_IF(upload(dk_, keys, (size_t)C * k * 4, st));
-  PSSA_RETURN_IF(upload(dn, norm_sq, (size_t)C * 4, st));
-  PSSA_RETURN_IF(upload(dv, values, (size_t)C * d * 4, st));
+  PSSA_RETURN_IF(upload(ctx, dx, x_norm, (size_t)L * d * 4));
+  PSSA_RETURN_IF(upload(ctx, dwqx, w_qx, (size_t)k * d * 4));
+  PSSA_RETURN_IF(upload(ctx, dwqh, w_qh, (size_t)k * d * 4));
+  PSSA_RETURN_IF(upload(ctx, dwg, w_gate, (size_t)d * d * 4));
+  PSSA_RETURN_IF(upload(ctx, dwp, w_proj, (size_t)d * d * 4));
+  PSSA_RETURN_IF(upload(ctx, dk_, keys, (size_t)C * k * 4));
+  PSSA_RETURN_IF(upload(ctx, dn, norm_sq, (size_t)C * 4));
+  PSSA_RETURN_IF(upload(ctx, dv, values, (size_t)C * d * 4));
   std::vector<float> vt((size_t)d * C);
   for (int s2 = 0; s2 < C; ++s2)
     for (int j = 0; j < d; ++j) vt[(size_t)j * C + s2] = values[(size_t)s2 * d + j];
-  PSSA_RETURN_IF(upload(dvt, vt.data(), vt.size() * 4, st));
-  for (DevBuf* b : {&qx, &qe, &qp}) PSSA_RETURN_IF(b->alloc((size_t)L * k * 4));
-  PSSA_RETURN_IF(qn.alloc((size_t)L * 4));
-  PSSA_RETURN_IF(wts.alloc((size_t)L * C * 4));
-  for (DevBuf* b : {&mv, &gm, &mp, &mi}) PSSA_RETURN_IF(b->alloc((size_t)L * d * 4));
+  PSSA_RETURN_IF(upload(ctx, dvt, vt.data(), vt.size() * 4));
+  for (DevBuf* b : {&qx, &qe, &qp}) PSSA_RETURN_IF(b->alloc((size_t)L * k * 4, &ctx->pool));
+  PSSA_RETURN_IF(qn.alloc((size_t)L * 4, &ctx->pool));
+  PSSA_RETURN_IF(wts.alloc((size_t)L * C * 4, &ctx->pool));
+  for (DevBuf* b : {&mv, &gm, &mp, &mi}) PSSA_RETURN_IF(b->alloc((size_t)L * d * 4, &ctx->pool));
   // q_euc = x W_qx^T + y W_qh^T, as dot(row_x, x) + dot(row_h, y) (src/pssa.rs:1147-1152).
   pssa::EpiParams ex;
   ex.out32 = qx.as<float>();
@@ -701,14 +714,14 @@ static Status run_stage_memory(pssa_hip_ctx* ctx, const float* x_norm, const flo
   ep2.ld32 = d;
   PSSA_RETURN_IF(pssa::launch_gemm(st, PSSA_HIP_F32, mv.p, d, dwp.p, d, L, d, d, ep2));
   PSSA_RETURN_IF(pssa::launch_mul(st, gm.as<float>(), mp.as<float>(), mi.as<float>(), (size_t)L * d));
-  if (q_euc) PSSA_RETURN_IF(download(q_euc, qe, (size_t)L * k * 4, st));
-  if (q_pnc) PSSA_RETURN_IF(download(q_pnc, qp, (size_t)L * k * 4, st));
-  if (q_norm) PSSA_RETURN_IF(download(q_norm, qn, (size_t)L * 4, st));
-  if (weights) PSSA_RETURN_IF(download(weights, wts, (size_t)L * C * 4, st));
-  if (m_val) PSSA_RETURN_IF(download(m_val, mv, (size_t)L * d * 4, st));
-  if (g_mem) PSSA_RETURN_IF(download(g_mem, gm, (size_t)L * d * 4, st));
-  if (m_proj) PSSA_RETURN_IF(download(m_proj, mp, (size_t)L * d * 4, st));
-  PSSA_RETURN_IF(download(m_inj, mi, (size_t)L * d * 4, st));
+  if (q_euc) PSSA_RETURN_IF(download(ctx, q_euc, qe, (size_t)L * k * 4));
+  if (q_pnc) PSSA_RETURN_IF(download(ctx, q_pnc, qp, (size_t)L * k * 4));
+  if (q_norm) PSSA_RETURN_IF(download(ctx, q_norm, qn, (size_t)L * 4));
+  if (weights) PSSA_RETURN_IF(download(ctx, weights, wts, (size_t)L * C * 4));
+  if (m_val) PSSA_RETURN_IF(download(ctx, m_val, mv, (size_t)L * d * 4));
+  if (g_mem) PSSA_RETURN_IF(download(ctx, g_mem, gm, (size_t)L * d * 4));
+  if (m_proj) PSSA_RETURN_IF(download(ctx, m_proj, mp, (size_t)L * d * 4));
+  PSSA_RETURN_IF(download(ctx, m_inj, mi, (size_t)L * d * 4));
   return sync(ctx);
 }
 
@@ -729,7 +742,7 @@ int pssa_hip_memory_forward(pssa_hip_ctx* ctx, const float* x_norm, const float*
     std::lock_guard<std::mutex> g(ctx->mu);
     PSSA_HIP_TRY(hipSetDevice(ctx->device));
     DevBuf dy;
-    PSSA_RETURN_IF(upload(dy, y_ssm, seq_len * d_m * 4, ctx->stream));
+    PSSA_RETURN_IF(upload(ctx, dy, y_ssm, seq_len * d_m * 4));
     return run_stage_memory(ctx, x_norm, dy.as<float>(), w_qx, w_qh, w_gate, w_proj, keys, norm_sq, values,
                             seq_len, d_m, d_k, capacity, count, tau, top_k, q_euc, q_pnc, q_norm, weights, m_val,
                             g_mem, m_proj, m_inj);
@@ -830,18 +843,18 @@ static int retrieve_host(pssa_hip_ctx* ctx, const float* q_pnc, size_t n_q, cons
     PSSA_HIP_TRY(hipSetDevice(ctx->device));
     const hipStream_t st = ctx->stream;
     DevBuf dq, dk_, dn, dv, dval, dmin, didx, dw, dg, da;
-    PSSA_RETURN_IF(upload(dq, q_pnc, n_q * d_key * 4, st));
-    PSSA_RETURN_IF(upload(dk_, keys, capacity * d_key * 4, st));
-    PSSA_RETURN_IF(upload(dn, norm_sq, capacity * 4, st));
-    PSSA_RETURN_IF(upload(dv, values, capacity * d_val * 4, st));
+    PSSA_RETURN_IF(upload(ctx, dq, q_pnc, n_q * d_key * 4));
+    PSSA_RETURN_IF(upload(ctx, dk_, keys, capacity * d_key * 4));
+    PSSA_RETURN_IF(upload(ctx, dn, norm_sq, capacity * 4));
+    PSSA_RETURN_IF(upload(ctx, dv, values, capacity * d_val * 4));
     if (hybrid && count > 0) {
-      PSSA_RETURN_IF(upload(dg, gate, count * 4, st));
-      PSSA_RETURN_IF(upload(da, age, count * 8, st));
+      PSSA_RETURN_IF(upload(ctx, dg, gate, count * 4));
+      PSSA_RETURN_IF(upload(ctx, da, age, count * 8));
     }
-    PSSA_RETURN_IF(dval.alloc(n_q * d_val * 4));
-    if (out_min) PSSA_RETURN_IF(dmin.alloc(n_q * 4));
-    if (out_idx) PSSA_RETURN_IF(didx.alloc(n_q * top_k * 4));
-    if (out_weights) PSSA_RETURN_IF(dw.alloc(n_q * capacity * 4));
+    PSSA_RETURN_IF(dval.alloc(n_q * d_val * 4, &ctx->pool));
+    if (out_min) PSSA_RETURN_IF(dmin.alloc(n_q * 4, &ctx->pool));
+    if (out_idx) PSSA_RETURN_IF(didx.alloc(n_q * top_k * 4, &ctx->pool));
+    if (out_weights) PSSA_RETURN_IF(dw.alloc(n_q * capacity * 4, &ctx->pool));
     pssa::RetrieveArgs ra;
     ra.q = dq.as<float>();
     ra.ld_q = (int)d_key;
@@ -867,10 +880,10 @@ static int retrieve_host(pssa_hip_ctx* ctx, const float* q_pnc, size_t n_q, cons
     }
     PSSA_RETURN_IF(bind_retrieve_scratch(ctx, ra));
     PSSA_RETURN_IF(pssa::launch_retrieve(st, ra));
-    PSSA_RETURN_IF(download(out_val, dval, n_q * d_val * 4, st));
-    if (out_min) PSSA_RETURN_IF(download(out_min, dmin, n_q * 4, st));
-    if (out_idx) PSSA_RETURN_IF(download(out_idx, didx, n_q * top_k * 4, st));
-    if (out_weights) PSSA_RETURN_IF(download(out_weights, dw, n_q * capacity * 4, st));
+    PSSA_RETURN_IF(download(ctx, out_val, dval, n_q * d_val * 4));
+    if (out_min) PSSA_RETURN_IF(download(ctx, out_min, dmin, n_q * 4));
+    if (out_idx) PSSA_RETURN_IF(download(ctx, out_idx, didx, n_q * top_k * 4));
+    if (out_weights) PSSA_RETURN_IF(download(ctx, out_weights, dw, n_q * capacity * 4));
     return sync(ctx);
   };
   return pssa::finish(body(), err, err_len);
@@ -1012,8 +1025,8 @@ int pssa_hip_model_load(pssa_hip_ctx* ctx, const pssa_hip_weights* w, int weight
     m->cfg = c;
     m->dtype = weight_dtype;
     m->n_in = 2 * d + 2 * s + k + r;
-    PSSA_RETURN_IF(upload(m->embed, w->embed, V * d * 4, st));
-    PSSA_RETURN_IF(upload_weight(m->unembed, w->unembed, V * d, weight_dtype, st));
+    PSSA_RETURN_IF(upload_keep(ctx, m->embed, w->embed, V * d * 4));
+    PSSA_RETURN_IF(upload_weight(ctx, m->unembed, w->unembed, V * d, weight_dtype));
     m->blocks.resize(c.depth);
     std::vector<float> tmp;
     for (size_t l = 0; l < c.depth; ++l) {
@@ -1032,11 +1045,11 @@ int pssa_hip_model_load(pssa_hip_ctx* ctx, const pssa_hip_weights* w, int weight
       put(b.w_qx, k);
       put(b.w_gate, d);
       put(b.adapter_down, r);
-      PSSA_RETURN_IF(upload_weight(B.w_in, tmp.data(), tmp.size(), weight_dtype, st));
-      PSSA_RETURN_IF(upload_weight(B.w_qh, b.w_qh, k * d, weight_dtype, st));
-      PSSA_RETURN_IF(upload_weight(B.w_proj, b.w_proj, d * d, weight_dtype, st));
-      PSSA_RETURN_IF(upload_weight(B.mlp_w1, b.mlp_w1, 2 * d * d, weight_dtype, st));
-      PSSA_RETURN_IF(upload_weight(B.mlp_w2, b.mlp_w2, d * 2 * d, weight_dtype, st));
+      PSSA_RETURN_IF(upload_weight(ctx, B.w_in, tmp.data(), tmp.size(), weight_dtype));
+      PSSA_RETURN_IF(upload_weight(ctx, B.w_qh, b.w_qh, k * d, weight_dtype));
+      PSSA_RETURN_IF(upload_weight(ctx, B.w_proj, b.w_proj, d * d, weight_dtype));
+      PSSA_RETURN_IF(upload_weight(ctx, B.mlp_w1, b.mlp_w1, 2 * d * d, weight_dtype));
+      PSSA_RETURN_IF(upload_weight(ctx, B.mlp_w2, b.mlp_w2, d * 2 * d, weight_dtype));
       std::vector<float> ueff(d * r), rates(d * s), vt(d * C);
       for (size_t i = 0; i < d * r; ++i) ueff[i] = b.adapter_up[i] + b.adapter_slow[i];
       // State-major [s, d] for the scan.
@@ -1044,9 +1057,9 @@ int pssa_hip_model_load(pssa_hip_ctx* ctx, const pssa_hip_weights* w, int weight
         for (size_t j = 0; j < s; ++j) rates[j * d + i] = -softplus_host(b.a_raw[i * s + j]) * 1.4426950408889634f;
       for (size_t q = 0; q < C; ++q)
         for (size_t j = 0; j < d; ++j) vt[j * C + q] = b.mem_values[q * d + j];
-      PSSA_RETURN_IF(upload_weight(B.u_eff, ueff.data(), ueff.size(), weight_dtype, st));
-      PSSA_RETURN_IF(upload(B.u_fast, b.adapter_up, d * r * 4, st));
-      PSSA_RETURN_IF(upload(B.u_slow, b.adapter_slow, d * r * 4, st));
+      PSSA_RETURN_IF(upload_weight(ctx, B.u_eff, ueff.data(), ueff.size(), weight_dtype));
+      PSSA_RETURN_IF(upload_keep(ctx, B.u_fast, b.adapter_up, d * r * 4));
+      PSSA_RETURN_IF(upload_keep(ctx, B.u_slow, b.adapter_slow, d * r * 4));
       std::vector<float> conf(C, 1.0f);
       std::vector<unsigned long long> last(C, 0ull);
       if (b.mem_confidence) std::memcpy(conf.data(), b.mem_confidence, C * 4);
@@ -1062,24 +1075,24 @@ int pssa_hip_model_load(pssa_hip_ctx* ctx, const pssa_hip_weights* w, int weight
       B.lam = b.mem_hybrid_lam;
       B.top_k = (int)b.mem_top_k;
       B.value_cap = b.mem_value_cap;
-      PSSA_RETURN_IF(upload(B.hgate, hg.data(), C * 4, st));
-      PSSA_RETURN_IF(upload(B.hage, ha.data(), C * 8, st));
-      PSSA_RETURN_IF(upload(B.conf, conf.data(), C * 4, st));
-      PSSA_RETURN_IF(upload(B.last_seen, last.data(), C * 8, st));
-      PSSA_RETURN_IF(upload(B.meta, meta, sizeof(meta), st));
-      PSSA_RETURN_IF(upload(B.rates2, rates.data(), rates.size() * 4, st));
-      PSSA_RETURN_IF(upload(B.gamma, b.norm_gamma, d * 4, st));
-      PSSA_RETURN_IF(upload(B.beta, b.norm_beta, d * 4, st));
-      PSSA_RETURN_IF(upload(B.keys, b.mem_keys, C * k * 4, st));
-      PSSA_RETURN_IF(upload(B.norm_sq, b.mem_norm_sq, C * 4, st));
-      PSSA_RETURN_IF(upload(B.values, b.mem_values, C * d * 4, st));
-      PSSA_RETURN_IF(upload_weight(B.values_t, vt.data(), vt.size(), weight_dtype, st));
+      PSSA_RETURN_IF(upload_keep(ctx, B.hgate, hg.data(), C * 4));
+      PSSA_RETURN_IF(upload_keep(ctx, B.hage, ha.data(), C * 8));
+      PSSA_RETURN_IF(upload_keep(ctx, B.conf, conf.data(), C * 4));
+      PSSA_RETURN_IF(upload_keep(ctx, B.last_seen, last.data(), C * 8));
+      PSSA_RETURN_IF(upload_keep(ctx, B.meta, meta, sizeof(meta)));
+      PSSA_RETURN_IF(upload_keep(ctx, B.rates2, rates.data(), rates.size() * 4));
+      PSSA_RETURN_IF(upload_keep(ctx, B.gamma, b.norm_gamma, d * 4));
+      PSSA_RETURN_IF(upload_keep(ctx, B.beta, b.norm_beta, d * 4));
+      PSSA_RETURN_IF(upload_keep(ctx, B.keys, b.mem_keys, C * k * 4));
+      PSSA_RETURN_IF(upload_keep(ctx, B.norm_sq, b.mem_norm_sq, C * 4));
+      PSSA_RETURN_IF(upload_keep(ctx, B.values, b.mem_values, C * d * 4));
+      PSSA_RETURN_IF(upload_weight(ctx, B.values_t, vt.data(), vt.size(), weight_dtype));
       PSSA_RETURN_IF(sync(ctx));  // host staging vectors are reused
       // Values of a capped bank are capped (a no-op for values that were).
       if (B.value_cap > 0.0f) PSSA_RETURN_IF(cap_bank_values(m.get(), {&B}, B.value_cap));
     }
     const unsigned long long step0 = 0;
-    PSSA_RETURN_IF(upload(m->step, &step0, 8, st));
+    PSSA_RETURN_IF(upload_keep(ctx, m->step, &step0, 8));
     PSSA_RETURN_IF(sync(ctx));
     *out = m.release();
     return Status::Ok();
@@ -1187,9 +1200,9 @@ int pssa_hip_lanes_get_carry(pssa_hip_lanes* L, float* out, size_t len, char* er
     std::lock_guard<std::mutex> g(L->ctx->mu);
     PSSA_HIP_TRY(hipSetDevice(L->ctx->device));
     DevBuf tmp;
-    PSSA_RETURN_IF(tmp.alloc(n * 4));
+    PSSA_RETURN_IF(tmp.alloc(n * 4, &L->ctx->pool));
     PSSA_RETURN_IF(carry_layout(L, L->carry.as<float>(), tmp.as<float>(), false));
-    PSSA_RETURN_IF(download(out, tmp, n * 4, L->ctx->stream));
+    PSSA_RETURN_IF(download(L->ctx, out, tmp, n * 4));
     return sync(L->ctx);
   };
   return pssa::finish(body(), err, err_len);
@@ -1204,7 +1217,7 @@ int pssa_hip_lanes_set_carry(pssa_hip_lanes* L, const float* in, size_t len, cha
     std::lock_guard<std::mutex> g(L->ctx->mu);
     PSSA_HIP_TRY(hipSetDevice(L->ctx->device));
     DevBuf tmp;
-    PSSA_RETURN_IF(upload(tmp, in, n * 4, L->ctx->stream));
+    PSSA_RETURN_IF(upload(L->ctx, tmp, in, n * 4));
     PSSA_RETURN_IF(carry_layout(L, tmp.as<float>(), L->carry.as<float>(), true));
     // The prefill logits belong to the replaced carries.
     L->logit_lanes = 0;
@@ -1231,7 +1244,7 @@ int pssa_hip_prefill(pssa_hip_lanes* L, const uint32_t* ids, size_t n_lanes, siz
     PSSA_RETURN_IF(stage_ids_locked(L, ids, n_lanes, seq_len));
     PSSA_RETURN_IF(pssa::run_prefill(L, n_lanes, seq_len));
     L->logit_lanes = n_lanes;
-    if (logits_last) PSSA_RETURN_IF(download(logits_last, L->logits, n_lanes * V * 4, L->ctx->stream));
+    if (logits_last) PSSA_RETURN_IF(download(L->ctx, logits_last, L->logits, n_lanes * V * 4));
     return sync(L->ctx);
   };
   return pssa::finish(body(), err, err_len);
@@ -1288,7 +1301,7 @@ static void plan_ragged(const pssa_hip_lanes* L, const std::vector<uint64_t>& le
 static Status upload_plan(pssa_hip_lanes* L, RaggedPlan& p, size_t n_last, size_t n_pos) {
   if (!L->row_meta.p) PSSA_RETURN_IF(L->row_meta.alloc((4 * L->lanes + L->max_tokens) * 4));
   const size_t n_span = 3 * p.order.size();
-  PSSA_HIP_TRY(hipMemcpyAsync(L->row_meta.p, p.meta.data(), p.meta.size() * 4, hipMemcpyHostToDevice, L->ctx->stream));
+  PSSA_RETURN_IF(L->ctx->stage.to_device(L->row_meta.p, p.meta.data(), p.meta.size() * 4, L->ctx->stream));
   p.rows.spans = L->row_meta.as<int>();
   if (n_last) p.rows.last = L->row_meta.as<uint32_t>() + n_span;
   if (n_pos) p.rows.pos = L->row_meta.as<uint32_t>() + n_span + n_last;
@@ -1324,7 +1337,7 @@ static Status ragged_locked(pssa_hip_lanes* L, const uint32_t* ids, const uint64
   if (hybrid)
     for (size_t l = 0; l < p.order.size(); ++l)
       for (size_t t = 0; t < lens[p.order[l]]; ++t) p.meta.push_back((uint32_t)t);
-  PSSA_HIP_TRY(hipMemcpyAsync(L->ids.p, ids_h.data(), tokens * 4, hipMemcpyHostToDevice, L->ctx->stream));
+  PSSA_RETURN_IF(L->ctx->stage.to_device(L->ids.p, ids_h.data(), tokens * 4, L->ctx->stream));
   PSSA_RETURN_IF(upload_plan(L, p, n_lanes, hybrid ? tokens : 0));
   p.rows.ids = L->ids.as<uint32_t>();
   PSSA_RETURN_IF(pssa::run_prefill_ragged(L, p.rows));
@@ -1378,7 +1391,7 @@ int pssa_hip_prefill_ragged(pssa_hip_lanes* L, const uint32_t* ids, const uint64
     PSSA_RETURN_IF(ragged_locked(L, ids, lens, n_lanes));
     L->staged_lanes = L->staged_len = 0;  // `ids` holds the packed prompts
     L->logit_lanes = n_lanes;             // decode may continue from these logits
-    if (logits_last) PSSA_RETURN_IF(download(logits_last, L->logits, n_lanes * V * 4, L->ctx->stream));
+    if (logits_last) PSSA_RETURN_IF(download(L->ctx, logits_last, L->logits, n_lanes * V * 4));
     return sync(L->ctx);
   };
   return pssa::finish(body(), err, err_len);
@@ -1414,14 +1427,14 @@ int pssa_hip_prefill_cancellable(pssa_hip_lanes* L, const uint32_t* ids, size_t 
       for (size_t i = 0; i < n_lanes; ++i)
         std::memcpy(&part[i * T], ids + i * seq_len + t0, T * 4);
       PSSA_RETURN_IF(invalid_prefix_locked(L, part.data(), n_lanes, T));
-      PSSA_HIP_TRY(hipMemcpyAsync(L->ids.p, part.data(), n_lanes * T * 4, hipMemcpyHostToDevice, L->ctx->stream));
+      PSSA_RETURN_IF(L->ctx->stage.to_device(L->ids.p, part.data(), n_lanes * T * 4, L->ctx->stream));
       PSSA_RETURN_IF(pssa::run_prefill(L, n_lanes, T));
       PSSA_RETURN_IF(sync(L->ctx));  // `part` is refilled next
       if (processed) *processed = t0 + T;
     }
     L->staged_lanes = L->staged_len = 0;  // `ids` holds the last chunk
     L->logit_lanes = n_lanes;
-    if (logits_last) PSSA_RETURN_IF(download(logits_last, L->logits, n_lanes * V * 4, L->ctx->stream));
+    if (logits_last) PSSA_RETURN_IF(download(L->ctx, logits_last, L->logits, n_lanes * V * 4));
     return sync(L->ctx);
   };
   const int rc = pssa::finish(body(), err, err_len);
@@ -1503,8 +1516,8 @@ int pssa_hip_batch_forward(pssa_hip_lanes* L, const pssa_hip_sequence* seqs, siz
       std::memcpy(&meta_h[p.row[l]], q.targets, q.len * 4);
       for (size_t t = 0; t < q.len; ++t) meta_h[tokens + p.row[l] + t] = (uint32_t)(offset[p.order[l]] + t);
     }
-    PSSA_HIP_TRY(hipMemcpyAsync(L->ids.p, ids_h.data(), tokens * 4, hipMemcpyHostToDevice, st));
-    PSSA_HIP_TRY(hipMemcpyAsync(L->tok_meta.p, meta_h.data(), 2 * tokens * 4, hipMemcpyHostToDevice, st));
+    PSSA_RETURN_IF(L->ctx->stage.to_device(L->ids.p, ids_h.data(), tokens * 4, L->ctx->stream));
+    PSSA_RETURN_IF(L->ctx->stage.to_device(L->tok_meta.p, meta_h.data(), 2 * tokens * 4, L->ctx->stream));
     PSSA_RETURN_IF(upload_plan(L, p, 0, 0));
     p.rows.ids = L->ids.as<uint32_t>();
     p.rows.targets = L->tok_meta.as<uint32_t>();
@@ -1514,11 +1527,11 @@ int pssa_hip_batch_forward(pssa_hip_lanes* L, const pssa_hip_sequence* seqs, siz
     PSSA_RETURN_IF(pssa::run_train_forward(L, p.rows));
 
     std::vector<float> loss_h(tokens);
-    PSSA_HIP_TRY(hipMemcpyAsync(loss_h.data(), L->tok_loss.p, tokens * 4, hipMemcpyDeviceToHost, st));
+    PSSA_RETURN_IF(download(L->ctx, loss_h.data(), L->tok_loss, tokens * 4));
     if (logits)
       for (size_t l = 0; l < p.order.size(); ++l)
-        PSSA_HIP_TRY(hipMemcpyAsync(logits + offset[p.order[l]] * V, L->tok_logits.as<float>() + p.row[l] * V,
-                                    lens[p.order[l]] * V * 4, hipMemcpyDeviceToHost, st));
+        PSSA_RETURN_IF(L->ctx->stage.to_host(logits + offset[p.order[l]] * V,
+                                             L->tok_logits.as<float>() + p.row[l] * V, lens[p.order[l]] * V * 4, st));
     PSSA_RETURN_IF(sync(L->ctx));
     // The token mean in packed order, summed left to right in f32
     // (stage_logits_loss, src/gpu_batch.rs:1246-1249).
@@ -1566,7 +1579,7 @@ int pssa_hip_lanes_read_logits(pssa_hip_lanes* L, float* out, size_t len, char* 
     PSSA_RETURN_IF(need(len == n, "logits length must be the last prefill's lanes*d_vocab"));
     std::lock_guard<std::mutex> g(L->ctx->mu);
     PSSA_HIP_TRY(hipSetDevice(L->ctx->device));
-    PSSA_RETURN_IF(download(out, L->logits, n * 4, L->ctx->stream));
+    PSSA_RETURN_IF(download(L->ctx, out, L->logits, n * 4));
     return sync(L->ctx);
   };
   return pssa::finish(body(), err, err_len);
@@ -1597,17 +1610,17 @@ int pssa_hip_model_get_plastic(pssa_hip_model* M, size_t layer, float* adapter_u
     const hipStream_t st = M->ctx->stream;
     const pssa::DevBlock& B = M->blocks[layer];
     const size_t d = c.d_latent, k = c.d_mem_key, C = c.mem_capacity, r = c.adapter_rank;
-    if (adapter_up) PSSA_RETURN_IF(download(adapter_up, B.u_fast, d * r * 4, st));
-    if (keys) PSSA_RETURN_IF(download(keys, B.keys, C * k * 4, st));
-    if (values) PSSA_RETURN_IF(download(values, B.values, C * d * 4, st));
-    if (norm_sq) PSSA_RETURN_IF(download(norm_sq, B.norm_sq, C * 4, st));
-    if (confidence) PSSA_RETURN_IF(download(confidence, B.conf, C * 4, st));
+    if (adapter_up) PSSA_RETURN_IF(download(M->ctx, adapter_up, B.u_fast, d * r * 4));
+    if (keys) PSSA_RETURN_IF(download(M->ctx, keys, B.keys, C * k * 4));
+    if (values) PSSA_RETURN_IF(download(M->ctx, values, B.values, C * d * 4));
+    if (norm_sq) PSSA_RETURN_IF(download(M->ctx, norm_sq, B.norm_sq, C * 4));
+    if (confidence) PSSA_RETURN_IF(download(M->ctx, confidence, B.conf, C * 4));
     std::vector<unsigned long long> last(C);
-    if (last_seen) PSSA_RETURN_IF(download(last.data(), B.last_seen, C * 8, st));
+    if (last_seen) PSSA_RETURN_IF(download(M->ctx, last.data(), B.last_seen, C * 8));
     int meta[2] = {0, 0};
-    PSSA_RETURN_IF(download(meta, B.meta, sizeof(meta), st));
+    PSSA_RETURN_IF(download(M->ctx, meta, B.meta, sizeof(meta)));
     unsigned long long stp = 0;
-    PSSA_RETURN_IF(download(&stp, M->step, 8, st));
+    PSSA_RETURN_IF(download(M->ctx, &stp, M->step, 8));
     PSSA_RETURN_IF(sync(M->ctx));
     if (last_seen)
       for (size_t q = 0; q < C; ++q) last_seen[q] = last[q];
@@ -1672,9 +1685,9 @@ int pssa_hip_model_get_hybrid(pssa_hip_model* M, size_t layer, float* gate, uint
     const hipStream_t st = M->ctx->stream;
     const pssa::DevBlock& B = M->blocks[layer];
     const size_t C = M->cfg.mem_capacity;
-    if (gate) PSSA_RETURN_IF(download(gate, B.hgate, C * 4, st));
+    if (gate) PSSA_RETURN_IF(download(M->ctx, gate, B.hgate, C * 4));
     std::vector<unsigned long long> a(C);
-    if (age) PSSA_RETURN_IF(download(a.data(), B.hage, C * 8, st));
+    if (age) PSSA_RETURN_IF(download(M->ctx, a.data(), B.hage, C * 8));
     PSSA_RETURN_IF(sync(M->ctx));
     if (age)
       for (size_t q = 0; q < C; ++q) age[q] = a[q];
@@ -1775,7 +1788,7 @@ int pssa_hip_lanes_get_taps(pssa_hip_lanes* L, size_t layer, size_t n_lanes, flo
     const size_t n = n_lanes, d = c.d_latent, k = c.d_mem_key, r = c.adapter_rank;
     auto part = [&](float* dst, const DevBuf& src, size_t w) -> Status {
       if (!dst) return Status::Ok();
-      PSSA_HIP_TRY(hipMemcpyAsync(dst, src.as<float>() + layer * n * w, n * w * 4, hipMemcpyDeviceToHost, st));
+      PSSA_RETURN_IF(L->ctx->stage.to_host(dst, src.as<float>() + layer * n * w, n * w * 4, st));
       return Status::Ok();
     };
     PSSA_RETURN_IF(part(q_pnc, L->tap_q, k));
@@ -1852,7 +1865,7 @@ int pssa_hip_lanes_set_sampling(pssa_hip_lanes* L, float temperature, float top_
       if (!L->probs.p) PSSA_RETURN_IF(L->probs.alloc(L->lanes * L->model->cfg.d_vocab * 4));
       // SimpleRng::new (src/linalg.rs:7-11): every lane starts from `seed`.
       std::vector<uint64_t> st0(L->lanes, seed == 0 ? 0x853c49e6748fea9bULL : seed);
-      PSSA_HIP_TRY(hipMemcpyAsync(L->rng.p, st0.data(), L->lanes * 8, hipMemcpyHostToDevice, st));
+      PSSA_RETURN_IF(L->ctx->stage.to_device(L->rng.p, st0.data(), L->lanes * 8, L->ctx->stream));
       PSSA_RETURN_IF(sync(L->ctx));
     }
     L->temperature = temperature;
@@ -1900,13 +1913,13 @@ int pssa_hip_decode(pssa_hip_lanes* L, const uint32_t* first_ids, size_t n_lanes
     PSSA_RETURN_IF(ensure_decode_buffers(L, n_lanes, steps));
     PSSA_RETURN_IF(pssa::launch_fill_zero(st, static_cast<float*>(L->nonfinite.p), 3));
     const int zero = 0;
-    PSSA_HIP_TRY(hipMemcpyAsync(L->gen_pos.p, &zero, 4, hipMemcpyHostToDevice, st));
+    PSSA_RETURN_IF(L->ctx->stage.to_device(L->gen_pos.p, &zero, 4, L->ctx->stream));
     // After a prefill the first generated token is the choice from its logits
     // (src/inference.rs:367-379), and each later one costs a forward step of
     // the token before it; given first ids, every token costs a step.
     size_t fwd_steps = steps;
     if (first_ids) {
-      PSSA_HIP_TRY(hipMemcpyAsync(L->ids.p, first_ids, n_lanes * 4, hipMemcpyHostToDevice, st));
+      PSSA_RETURN_IF(L->ctx->stage.to_device(L->ids.p, first_ids, n_lanes * 4, L->ctx->stream));
     } else {
       PSSA_RETURN_IF(pssa::run_greedy_from_logits(L, n_lanes, true));
       fwd_steps = steps - 1;
@@ -1917,10 +1930,10 @@ int pssa_hip_decode(pssa_hip_lanes* L, const uint32_t* first_ids, size_t n_lanes
     } else {
       for (size_t t = 0; t < fwd_steps; ++t) PSSA_RETURN_IF(pssa::run_decode_step(L, n_lanes, plastic));
     }
-    PSSA_RETURN_IF(download(out_ids, L->gen_ids, steps * n_lanes * 4, st));
-    if (logits_last) PSSA_RETURN_IF(download(logits_last, L->logits, n_lanes * V * 4, st));
+    PSSA_RETURN_IF(download(L->ctx, out_ids, L->gen_ids, steps * n_lanes * 4));
+    if (logits_last) PSSA_RETURN_IF(download(L->ctx, logits_last, L->logits, n_lanes * V * 4));
     int nonfinite[3] = {0, 0, 0};
-    PSSA_RETURN_IF(download(nonfinite, L->nonfinite, 12, st));
+    PSSA_RETURN_IF(download(L->ctx, nonfinite, L->nonfinite, 12));
     // The last generated token has not been consumed: a continuation passes
     // it as first_ids.  `ids` now holds the step tokens.
     L->staged_lanes = L->staged_len = 0;
@@ -1951,15 +1964,15 @@ int pssa_hip_dense_scan(pssa_hip_ctx* ctx, const float* a, const float* b, const
     PSSA_HIP_TRY(hipSetDevice(ctx->device));
     const hipStream_t st = ctx->stream;
     DevBuf da, db, dh0, dh;
-    PSSA_RETURN_IF(upload(da, a, na * 4, st));
-    PSSA_RETURN_IF(upload(db, b, nb * 4, st));
-    if (h0) PSSA_RETURN_IF(upload(dh0, h0, batch * d_state * 4, st));
+    PSSA_RETURN_IF(upload(ctx, da, a, na * 4));
+    PSSA_RETURN_IF(upload(ctx, db, b, nb * 4));
+    if (h0) PSSA_RETURN_IF(upload(ctx, dh0, h0, batch * d_state * 4));
     PSSA_RETURN_IF(dh.alloc(nb * 4));
     PSSA_RETURN_IF(bind_dense_scan_scratch(ctx, (int)batch, (int)seq_len, (int)d_state));
     PSSA_RETURN_IF(pssa::launch_dense_scan(st, da.as<float>(), db.as<float>(), h0 ? dh0.as<float>() : nullptr,
                                            dh.as<float>(), (int)batch, (int)seq_len, (int)d_state, ctx->scratch,
                                            ctx->scratch_bytes));
-    PSSA_RETURN_IF(download(h, dh, nb * 4, st));
+    PSSA_RETURN_IF(download(ctx, h, dh, nb * 4));
     return sync(ctx);
   };
   return pssa::finish(body(), err, err_len);

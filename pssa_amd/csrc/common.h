@@ -77,14 +77,59 @@ inline Status checked_count(std::initializer_list<size_t> dims, size_t* out, con
   return Status::Ok();
 }
 
-// Device buffer owned by RAII.
+// Device blocks kept between calls for the temporaries of the host-array
+// entry points (each hipMalloc / hipFree pair costs about 20 us, and a call
+// takes up to fifteen).  Blocks are handed out again on the context's one
+// stream, so a block's next user runs after its last; at most kPoolBytes are
+// held, the rest is freed at once, and all of it with the context.
+class DevPool {
+ public:
+  static constexpr size_t kPoolBytes = (size_t)256 << 20;
+  ~DevPool() { clear(); }
+  // A held block of at least `n` bytes and not much more, or null.
+  void* take(size_t n, size_t* bytes) {
+    std::lock_guard<std::mutex> g(mu_);
+    const auto it = free_.lower_bound(n);
+    if (it == free_.end() || it->first > 2 * n + 4096) return nullptr;
+    void* p = it->second;
+    *bytes = it->first;
+    held_ -= it->first;
+    free_.erase(it);
+    return p;
+  }
+  void put(void* p, size_t bytes) {
+    {
+      std::lock_guard<std::mutex> g(mu_);
+      if (held_ + bytes <= kPoolBytes) {
+        free_.emplace(bytes, p);
+        held_ += bytes;
+        return;
+      }
+    }
+    (void)hipFree(p);
+  }
+  void clear() {
+    std::lock_guard<std::mutex> g(mu_);
+    for (auto& f : free_) (void)hipFree(f.second);
+    free_.clear();
+    held_ = 0;
+  }
+
+ private:
+  std::mutex mu_;
+  std::multimap<size_t, void*> free_;
+  size_t held_ = 0;
+};
+
+// Device buffer owned by RAII (returned to `pool` when it came from one).
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
+  DevPool* pool = nullptr;
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes) {
+  DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes), pool(o.pool) {
     o.p = nullptr;
     o.bytes = 0;
   }
@@ -93,6 +138,7 @@ struct DevBuf {
       release();
       p = o.p;
       bytes = o.bytes;
+      pool = o.pool;
       o.p = nullptr;
       o.bytes = 0;
     }
@@ -100,27 +146,114 @@ struct DevBuf {
   }
   ~DevBuf() { release(); }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p && pool)
+      pool->put(p, bytes);
+    else if (p)
+      (void)hipFree(p);
     p = nullptr;
     bytes = 0;
+    pool = nullptr;
   }
-  Status alloc(size_t n) {
+  Status alloc(size_t n, DevPool* from = nullptr) {
     release();
     n = (n + 255) & ~(size_t)255;  // whole 256-byte granules: fills may round up to a vector
     if (n == 0) n = 256;
+    if (from && (p = from->take(n, &bytes))) {
+      pool = from;
+      return Status::Ok();
+    }
     hipError_t e = hipMalloc(&p, n);
+    if (e != hipSuccess && from) {
+      (void)hipGetLastError();
+      from->clear();
+      e = hipMalloc(&p, n);
+    }
     if (e != hipSuccess) {
       p = nullptr;
       (void)hipGetLastError();
       return Status::NoMem("hipMalloc(" + std::to_string(n) + "): " + hipGetErrorString(e));
     }
     bytes = n;
+    pool = from;
     return Status::Ok();
   }
   template <class T>
   T* as() const {
     return static_cast<T*>(p);
   }
+};
+
+// Copies between host arrays and the device.  The runtime's copies of
+// pageable arrays cost 105 us for 256 KiB either way and 330-370 us down for 6
+// MB on the machine measured; a pinned transfer and a memcpy 13 + 9 us, and
+// with the host's copy of one piece beside the transfer of the next about 230
+// us.  Arrays from 32 KiB (uploads to 1 MiB, where the runtime's own pipeline
+// is as fast) therefore go through pinned slots of the context's; arrays
+// pinned by the caller move directly.  Used with the context's lock held, on
+// its stream.
+class HostStage {
+ public:
+  static constexpr size_t kSlot = (size_t)1 << 20, kMin = (size_t)32 << 10;
+  static constexpr int kSlots = 4;
+  ~HostStage() {
+    if (buf_) (void)hipHostFree(buf_);
+  }
+  Status init() {
+    PSSA_HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&buf_), kSlot * kSlots, 0));
+    return Status::Ok();
+  }
+  // A pageable source may be reused at return; the copy is ordered on the
+  // stream.
+  Status to_device(void* dst, const void* src, size_t n, hipStream_t st) {
+    if (!n) return Status::Ok();
+    if (n >= kMin && n < kSlot && !pinned(src)) {
+      if (used_ + n > kSlot * kSlots) PSSA_RETURN_IF(drain(st));
+      std::memcpy(buf_ + used_, src, n);
+      src = buf_ + used_;
+      used_ += (n + 255) & ~(size_t)255;
+    }
+    PSSA_HIP_TRY(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st));
+    return Status::Ok();
+  }
+  // The data is in `dst` at return (after all earlier work of the stream).
+  Status to_host(void* dst, const void* src, size_t n, hipStream_t st) {
+    if (!n) return Status::Ok();
+    if (n < kMin || pinned(dst)) {
+      PSSA_HIP_TRY(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st));
+      return drain(st);
+    }
+    PSSA_RETURN_IF(drain(st));
+    auto piece = [&](size_t off) { return n - off < kSlot ? n - off : kSlot; };
+    auto issue = [&](size_t off) {
+      return hipMemcpyAsync(buf_ + off / kSlot % 2 * kSlot, static_cast<const char*>(src) + off, piece(off),
+                            hipMemcpyDeviceToHost, st);
+    };
+    PSSA_HIP_TRY(issue(0));
+    for (size_t off = 0; off < n; off += kSlot) {
+      PSSA_HIP_TRY(hipStreamSynchronize(st));  // this piece is in its slot
+      if (off + kSlot < n) PSSA_HIP_TRY(issue(off + kSlot));
+      std::memcpy(static_cast<char*>(dst) + off, buf_ + off / kSlot % 2 * kSlot, piece(off));
+    }
+    return Status::Ok();
+  }
+
+ private:
+  // Every transfer out of or into the slots has ended.
+  Status drain(hipStream_t st) {
+    PSSA_HIP_TRY(hipStreamSynchronize(st));
+    used_ = 0;
+    return Status::Ok();
+  }
+  static bool pinned(const void* p) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    return at.type == hipMemoryTypeHost || at.type == hipMemoryTypeManaged;
+  }
+  char* buf_ = nullptr;
+  size_t used_ = 0;  // bytes of the slots that uploads may still be reading
 };
 
 // fp32 -> bf16 bits, rounded to nearest even, on gfx950's v_cvt_pk_bf16_f32
@@ -192,6 +325,8 @@ struct pssa_hip_ctx {
   std::string name;
   int cu_count = 0;
   std::mutex mu;
+  pssa::HostStage stage;
+  pssa::DevPool pool;  // before every member whose buffers return to it
   // Kernel scratch reused across calls (grown on demand, freed with the
   // context); calls on one context are serialised by `mu` on one stream.
   void* scratch = nullptr;
