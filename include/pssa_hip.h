@@ -325,7 +325,7 @@ int pssa_hip_retrieve_hybrid(pssa_hip_ctx* ctx, const float* q_pnc, size_t n_q, 
  * a [batch, L, s, s] row-major (h_t[r] = sum_c A_t[r][c] h_{t-1}[c] + b_t[r]),
  * b [batch, L, s], h0 [batch, s] (NULL = zeros), h [batch, L, s].
  * Accuracy: every h_t is an exact fp32 step (fused multiply-adds) from the
- * state before it.  With s = 64 and L >= 256 (16-byte aligned a and b) the
+ * state before it.  With s = 64, L >= 256 and batch <= 64 (16-byte aligned a and b) the
  * state entering each 32-step sub-chunk is carried through the composed
  * maps of the sub-chunks before it in its 128-step window, products of
  * bf16 hi/lo splits (about 2^-17 relative per factor); a composed map that

@@ -6,8 +6,8 @@
 //  - Time-sequential (dense_scan_ring_kernel, dense_scan_kernel): one
 //    workgroup walks one sequence in time order and reads every A_t once.
 //    With one workgroup per sequence only `batch` CUs stream, and a CU
-//    streams about 22 B/clk from HBM (3.3 TB/s with 64 CUs, measured), so
-//    this bounds long sequences of few lanes.
+//    streams at most about 22 B/clk from HBM (3.3 TB/s with 64 CUs,
+//    measured), so this bounds long sequences of few lanes.
 //
 //  - Chunked two-level (dense_twolevel_kernel, d_state 64): time is cut into
 //    windows of TL_SUB sub-chunks of TL_LC steps.  Level 1 composes each
@@ -22,66 +22,114 @@
 
 namespace pssa {
 
-template <int S, int DEPTH>
-__global__ __launch_bounds__(256) void dense_scan_kernel(const float* __restrict__ A,
-                                                         const float* __restrict__ Bv,
-                                                         const float* __restrict__ H0,
-                                                         float* __restrict__ H, int L, int s) {
-  constexpr int TPR = 256 / S;  // threads per row
+// Any d_state up to S: S * TPR threads, TPR neighbouring lanes a row.  Bound:
+// the chain of a step (h through LDS, CPT products in four sums, the row's
+// lanes by DPP).  States of up to 32 fit one wave, whose LDS operations are in
+// order, so a step needs no barrier.  The loads, DEPTH steps ahead, are
+// unguarded at clamped columns and masked at their use: under a guard per
+// element each closed its block with a full wait, a memory round trip a step.
+// 3 x 2011 steps of 48: 2.07 -> 0.48 ms; 64 x 2048 of 48 2.46 -> 0.54 (2.3
+// TB/s), of 16 0.575 -> 0.197; 30 x 1000 of 32 0.349 -> 0.161.
+template <int TPR>
+__device__ __forceinline__ float row_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));  // quad_perm 1,0,3,2
+  if constexpr (TPR == 4)
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));  // quad_perm 2,3,0,1
+  return v;
+}
+
+template <int S, int TPR, int DEPTH, bool VEC>
+__global__ __launch_bounds__(S * TPR) void dense_scan_kernel(const float* __restrict__ A,
+                                                             const float* __restrict__ Bv,
+                                                             const float* __restrict__ H0,
+                                                             float* __restrict__ H, int L, int s) {
+  static_assert(TPR == 2 || TPR == 4, "row_sum");
   constexpr int CPT = S / TPR;  // columns per thread
-  static_assert(CPT % 4 == 0 || CPT < 4, "column slice");
+  static_assert(CPT % 4 == 0, "column slice");
   __shared__ __attribute__((aligned(16))) float sh[2][S];
 
   const int tid = threadIdx.x;
-  const int row = tid / TPR, part = tid % TPR;
-  const int c0 = part * CPT;
-  const int seq = blockIdx.x;
-  const bool rvalid = row < s;
+  const int row = tid / TPR, part = tid % TPR, c0 = part * CPT;
+  const int seq = blockIdx.x, r = min(row, s - 1);
   const size_t ss = (size_t)s * s;
-  const float* Aseq = A + (size_t)seq * L * ss;
-  const float* bseq = Bv + (size_t)seq * L * s;
-  float* hseq = H + (size_t)seq * L * s;
+  const float* arow = A + (size_t)seq * L * ss + (size_t)r * s;
+  const float* brow = Bv + (size_t)seq * L * s + r;
+  float* hrow = H + (size_t)seq * L * s + r;
+  const bool writes = part == 0 && row < s;
+  const int nv = s - c0;  // columns of this thread in range
 
   if (tid < S) sh[0][tid] = (tid < s && H0) ? H0[(size_t)seq * s + tid] : 0.0f;
+  if (tid < S) sh[1][tid] = 0.0f;
 
   float ring[DEPTH][CPT];
   float bring[DEPTH];
-  auto fetch = [&](int t, int slot) {
-    const float* arow = Aseq + (size_t)t * ss + (size_t)row * s;
+  // The next step in order; past the last one it again, unused, so that the
+  // loop has no branch around its loads (the waits would not count past one).
+  int left = L;
+  auto fetch = [&](int slot) {
+    if constexpr (VEC) {
 #pragma unroll
-    for (int q = 0; q < CPT; ++q) {
-      const int col = c0 + q;
-      ring[slot][q] = (rvalid && col < s) ? __builtin_nontemporal_load(arow + col) : 0.0f;
+      for (int q = 0; q < CPT; q += 4) {
+        const float4 v = *reinterpret_cast<const float4*>(arow + min(c0 + q, s - 4));
+        ring[slot][q] = v.x, ring[slot][q + 1] = v.y, ring[slot][q + 2] = v.z, ring[slot][q + 3] = v.w;
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < CPT; ++q) ring[slot][q] = arow[min(c0 + q, s - 1)];
     }
-    bring[slot] = (rvalid && part == 0) ? bseq[(size_t)t * s + row] : 0.0f;
+    bring[slot] = *brow;
+    --left;
+    arow += left > 0 ? ss : 0;
+    brow += left > 0 ? s : 0;
+  };
+  // This wave's LDS writes are seen by its reads; with several waves a
+  // barrier that leaves the loads in flight.
+  auto meet = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if constexpr (S * TPR > 64) {
+      __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0x0 << 8) | (0xF) | (0x3 << 14));  // lgkmcnt(0)
+      asm volatile("s_barrier" ::: "memory");
+    } else {
+      __builtin_amdgcn_wave_barrier();
+    }
   };
 #pragma unroll
-  for (int q = 0; q < DEPTH; ++q)
-    if (q < L) fetch(q, q);
-  __syncthreads();
+  for (int q = 0; q < DEPTH; ++q) fetch(q);
+  meet();
 
   int cur = 0;
-  for (int t0 = 0; t0 < L; t0 += DEPTH) {
+  auto step = [&](int q) {
+    float p[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < CPT; c += 4) {
+      const float4 hv = *reinterpret_cast<const float4*>(&sh[cur][c0 + c]);
+      const float h4[4] = {hv.x, hv.y, hv.z, hv.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[e] = fmaf(c + e < nv ? ring[q][c + e] : 0.0f, h4[e], p[e]);
+    }
+    const float hv = row_sum<TPR>((p[0] + p[1]) + (p[2] + p[3])) + bring[q];
+    if (writes) {
+      sh[cur ^ 1][row] = hv;
+      *hrow = hv;
+    }
+    hrow += s;
+    cur ^= 1;
+  };
+  int t0 = 0;
+  for (; t0 + DEPTH <= L; t0 += DEPTH) {
 #pragma unroll
     for (int q = 0; q < DEPTH; ++q) {
-      const int t = t0 + q;
-      if (t < L) {
-        float acc = 0.0f;
-#pragma unroll
-        for (int c = 0; c < CPT; ++c) acc = fmaf(ring[q][c], sh[cur][c0 + c], acc);
-#pragma unroll
-        for (int off = TPR / 2; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
-        const float hv = acc + bring[q];
-        if (part == 0 && rvalid) {
-          sh[cur ^ 1][row] = hv;
-          hseq[(size_t)t * s + row] = hv;
-        }
-        if (t + DEPTH < L) fetch(t + DEPTH, q);
-        __syncthreads();
-        cur ^= 1;
-      }
+      step(q);
+      fetch(q);
+      meet();
     }
   }
+#pragma unroll
+  for (int q = 0; q < DEPTH; ++q)
+    if (t0 + q < L) {
+      step(q);
+      meet();
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -612,8 +660,15 @@ __global__ __launch_bounds__(TL_THREADS) void dense_twolevel_kernel(TwoLevelArgs
   if (nc > 0) compose_finish();
 }
 
+// Sequences the two-level schedule takes: TL_SUB workgroups each, one to a CU.
+// Past the 256 CUs every launch runs two rounds, and the sequential kernel's
+// one workgroup per sequence streams as fast: 80 x 1024 0.743 / 0.593 ms
+// (two-level / ring), 96 x 700 0.559 / 0.405, 256 x 512 0.854 / 0.442; 64 x
+// 2048 0.770 / 1.17.
+constexpr int TL_MAX_BATCH = 256 / TL_SUB;
+
 size_t dense_scan_scratch_bytes(int batch, int L, int s) {
-  if (s != DS_S || L < 2 * TL_W) return 0;
+  if (s != DS_S || L < 2 * TL_W || batch > TL_MAX_BATCH) return 0;
   return ((size_t)2 * batch * (TL_SUB - 1) * TL_AGG + (size_t)2 * batch * DS_S) * sizeof(float);
 }
 
@@ -622,6 +677,15 @@ static bool ring_fits(const float* A, const float* B, int s) {
 }
 
 Status init_dense_scan_attributes() { return Status::Ok(); }
+
+template <int S, int TPR, int DEPTH>
+static void launch_general(hipStream_t stream, const float* A, const float* B, const float* H0, float* H, int batch,
+                           int L, int s) {
+  if (s % 4 == 0 && ((uintptr_t)A & 15) == 0)
+    dense_scan_kernel<S, TPR, DEPTH, true><<<batch, S * TPR, 0, stream>>>(A, B, H0, H, L, s);
+  else
+    dense_scan_kernel<S, TPR, DEPTH, false><<<batch, S * TPR, 0, stream>>>(A, B, H0, H, L, s);
+}
 
 Status launch_dense_scan(hipStream_t stream, const float* A, const float* B, const float* H0, float* H,
                          int batch, int L, int s, void* scratch, size_t scratch_bytes) {
@@ -649,15 +713,18 @@ Status launch_dense_scan(hipStream_t stream, const float* A, const float* B, con
     }
     return Status::Ok();
   }
-  if (ring_fits(A, B, s)) {
+  // Few sequences leave the step chain the bound, which the general kernel's
+  // register ring keeps shorter (32 x 232: 0.098 ms against 0.121); with more
+  // the direct loads of the LDS ring carry more (256 x 512: 0.475 / 0.442).
+  if (ring_fits(A, B, s) && batch > TL_MAX_BATCH) {
     dense_scan_ring_kernel<<<batch, DS_THREADS, 0, stream>>>(A, B, H0, H, L);
-  } else if (s <= 16)
-    dense_scan_kernel<16, 16><<<batch, 256, 0, stream>>>(A, B, H0, H, L, s);
-  else if (s <= 32)
-    dense_scan_kernel<32, 16><<<batch, 256, 0, stream>>>(A, B, H0, H, L, s);
-  else if (s <= 64)
-    dense_scan_kernel<64, 8><<<batch, 256, 0, stream>>>(A, B, H0, H, L, s);
-  else
+  } else if (s <= 16) {
+    launch_general<16, 4, 16>(stream, A, B, H0, H, batch, L, s);
+  } else if (s <= 32) {
+    launch_general<32, 2, 8>(stream, A, B, H0, H, batch, L, s);
+  } else if (s <= 64) {
+    launch_general<64, 4, 8>(stream, A, B, H0, H, batch, L, s);
+  } else
     return Status{PSSA_HIP_EUNSUPPORTED, "dense scan: d_state above 64 is not supported"};
   PSSA_LAUNCH_CHECK("dense_scan");
   return Status::Ok();

@@ -493,6 +493,43 @@ def test_dense_scan_matches_oracle(hip, B, L, s):
     assert rel_err(h, ref) < 1e-4
 
 
+@pytest.mark.parametrize("s", [1, 4, 15, 16, 17, 31, 32, 33, 48, 63])
+def test_dense_scan_general_kernels_edges(hip, s):
+    """The general kernels (one wave up to 32 states, four above; aligned rows
+    and odd ones) around their prefetch depths, against the recurrence in f64:
+    each step's s products and sums of fp32 add at most (s + 1) * 2^-24 of the
+    state's size, and transitions of norm < 0.99 damp them (1 / (1 - 0.99))."""
+    for L in (1, 7, 8, 9, 15, 16, 17, 33, 70):
+        say("dense scan general", L, s)
+        rng = np.random.default_rng(L * 100 + s)
+        q, _ = np.linalg.qr(rng.standard_normal((3, L, s, s)))
+        a = (q * rng.uniform(0.8, 0.99, (3, L, 1, s))).astype(np.float32)
+        b = rng.standard_normal((3, L, s)).astype(np.float32)
+        h0 = rng.standard_normal((3, s)).astype(np.float32)
+        ref, h = np.empty((3, L, s)), h0.astype(np.float64)
+        for t in range(L):
+            h = np.einsum("bij,bj->bi", a[:, t].astype(np.float64), h) + b[:, t]
+            ref[:, t] = h
+        assert rel_err(hip.dense_scan(a, b, h0), ref) < 100 * (s + 1) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("B,L", [(1, 1), (1, 255), (64, 33), (64, 256), (65, 1), (65, 31), (65, 300)])
+def test_dense_scan_64_states_by_batch_and_length(hip, B, L):
+    """d_state 64 on both sides of the rules: below two windows or past 64
+    sequences the recurrence runs step by step (the bound of the test above);
+    64 x 256 is the two-level schedule, 2^-17 a factor of its four maps."""
+    say("dense scan 64 states", B, L)
+    rng = np.random.default_rng(B * 1000 + L)
+    a = (rng.standard_normal((B, L, 64, 64)) * (0.5 / 8.0)).astype(np.float32)
+    b = rng.standard_normal((B, L, 64)).astype(np.float32)
+    h0 = rng.standard_normal((B, 64)).astype(np.float32)
+    ref, h = np.empty((B, L, 64)), h0.astype(np.float64)
+    for t in range(L):
+        h = np.einsum("bij,bj->bi", a[:, t].astype(np.float64), h) + b[:, t]
+        ref[:, t] = h
+    assert rel_err(hip.dense_scan(a, b, h0), ref) < max(4 * 2.0 ** -17, 2 * 65 * 2.0 ** -24)
+
+
 @pytest.mark.parametrize("B,L", [(1, 256), (3, 300), (2, 513), (5, 1000)])
 def test_dense_scan_two_level_matches_oracle(hip, B, L):
     """d_state 64 and at least two windows of 128 steps take the chunked
