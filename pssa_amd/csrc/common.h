@@ -101,9 +101,12 @@ class DevPool {
     {
       std::lock_guard<std::mutex> g(mu_);
       if (held_ + bytes <= kPoolBytes) {
-        free_.emplace(bytes, p);
-        held_ += bytes;
-        return;
+        try {
+          free_.emplace(bytes, p);
+          held_ += bytes;
+          return;
+        } catch (...) {  // no host memory to hold it: freed (destructors call this)
+        }
       }
     }
     (void)hipFree(p);
