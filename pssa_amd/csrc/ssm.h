@@ -45,10 +45,6 @@ struct SsmArgs {
   int ld_y = 0;
   int T = 0, d = 0, s = 0;
   int lanes = 0;
-  // Ragged lanes: launch lane b runs rows spans[3b] .. + spans[3b + 1] - 1
-  // (its length, 1 <= length <= T) with the carry of lane spans[3b + 2].
-  // Null: rows b*T .. b*T+T-1, carry b.  `rows` is then the caller's.
-  const int* spans = nullptr;
   // Optional materialisation (stage API): per lane b, bar_a/bar_b at
   // + b*T*d*s, states at + b*(T+1)*d*s.  All three or none.
   float* bar_a = nullptr;
@@ -66,6 +62,10 @@ struct SsmArgs {
   // four-wave variant then runs at any grid size (the eight-wave one is the
   // faster scan alone on small grids, but leaves those kernels less room).
   int concurrent = 0;
+  // Ragged lanes: launch lane b runs rows spans[3b] .. + spans[3b + 1] - 1
+  // (its length, 1 <= length <= T) with the carry of lane spans[3b + 2].
+  // Null: rows b*T .. b*T+T-1, carry b.  `rows` is then the caller's.
+  const int* spans = nullptr;
 };
 
 // Rows of lane b are b*T .. b*T+T-1 (or its span's).  The states of a channel are split into
