@@ -297,9 +297,10 @@ int pssa_hip_retrieve_resident(pssa_hip_ctx* ctx, const float* d_q_pnc, size_t n
  * hipMalloc).  Results equal pssa_hip_retrieve_resident's bit for bit.  The
  * exact top-k path runs 8192 queries per pass in a static scratch array of
  * 19 MiB that each GPU the library runs on holds until the process ends;
- * a shape needing more scratch fails with PSSA_HIP_EINVAL.  Every call on
- * one GPU shares that GPU's array: calls that overlap on one GPU (from two
- * contexts, or two streams) race and must be serialised by the caller. */
+ * a shape needing more scratch fails with PSSA_HIP_EINVAL.  Every such call
+ * on one GPU shares that GPU's array: calls that overlap on one GPU (from two
+ * contexts, or two streams) race and must be serialised by the caller.  Full
+ * soft reads (top_k = 0) use no scratch. */
 int pssa_hip_retrieve_resident_noalloc(pssa_hip_ctx* ctx, const float* d_q_pnc, size_t n_q,
                                        const float* d_keys, const float* d_norm_sq, const float* d_values,
                                        size_t capacity, size_t count, size_t d_key, size_t d_val, float tau,

@@ -781,7 +781,7 @@ int pssa_hip_memory_forward_after_ssm(pssa_hip_ctx* ctx, const float* x_norm, co
 
 // Points ra.scratch at the context's scratch, grown to what the launch needs.
 // Called with ctx->mu held; the previous buffer is released only once the
-// stream has drained.
+// stream has drained.  A full soft read runs without where there is no memory.
 static Status bind_retrieve_scratch(pssa_hip_ctx* ctx, pssa::RetrieveArgs& ra) {
   const size_t need_bytes = pssa::retrieve_scratch_bytes(ra);
   if (!need_bytes) return Status::Ok();
@@ -790,7 +790,13 @@ static Status bind_retrieve_scratch(pssa_hip_ctx* ctx, pssa::RetrieveArgs& ra) {
     if (ctx->scratch) PSSA_HIP_TRY(hipFree(ctx->scratch));
     ctx->scratch = nullptr;
     ctx->scratch_bytes = 0;
-    PSSA_HIP_TRY(hipMalloc(&ctx->scratch, need_bytes));
+    const hipError_t e = hipMalloc(&ctx->scratch, need_bytes);
+    if (e != hipSuccess) {
+      ctx->scratch = nullptr;
+      (void)hipGetLastError();
+      if (!pssa::retrieve_needs_scratch(ra)) return Status::Ok();
+      return Status::Device("retrieve scratch (" + std::to_string(need_bytes) + " bytes): " + hipGetErrorString(e));
+    }
     ctx->scratch_bytes = need_bytes;
   }
   ra.scratch = ctx->scratch;

@@ -22,11 +22,14 @@ struct RetrieveArgs {
   float* out_val = nullptr;     // [n, dv] (top-k readout)
   float* out_min = nullptr;     // optional [n]
   uint32_t* out_idx = nullptr;  // optional [n, top_k], ascending slot order
-  // Device scratch for the ranked top-k path (retrieve_scratch_bytes); when
-  // absent or too small the general kernel runs instead.
+  // Device scratch (retrieve_scratch_bytes); when absent or too small the
+  // ranked top-k path gives way to the general kernel, and a full soft read
+  // forms its readout inside its own kernel.
   void* scratch = nullptr;
   size_t scratch_bytes = 0;
-  int chunk = 0;  // queries per ranked dot/pick pass (0: the default, 32768)
+  // Queries per ranked dot/pick pass (0: the default, 32768).  Set: the
+  // scratch is the allocation-free call's, which only the ranked path uses.
+  int chunk = 0;
   // Hybrid read (retrieve_hybrid_into, src/memory.rs:568-660): with hgate
   // set, live slot s weighs exp((min - d_s)/tau) * hgate[s] * decay_s,
   // decay_s = (float)exp(age_s * log_lam), age_s = hage[s] + age_base
@@ -62,8 +65,12 @@ struct RetrieveArgs {
 // per wave, d_key <= 32, qk % 128 == 0 and the panels within LDS.
 bool retrieve_fuses_query(const RetrieveArgs& a);
 
-// Scratch the ranked top-k path needs for these arguments (0: not taken).
+// Scratch the ranked top-k path, or a full soft read's readout by a product,
+// uses for these arguments (0: neither is taken).
 size_t retrieve_scratch_bytes(const RetrieveArgs& a);
+// Whether a launch without that scratch would give other bits (the ranked
+// path); a full soft read without it gives the same ones.
+bool retrieve_needs_scratch(const RetrieveArgs& a);
 
 // The allocation-free retrieval (pssa_hip_retrieve_resident_noalloc) runs
 // the ranked path kNoallocChunk queries per pass in a static per-device

@@ -661,45 +661,62 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(4))) v
 // ---------------------------------------------------------------------------
 // Full soft read with the reference's own distances, for banks of up to 512
 // slots: the reads retrieve_kernel would serve one query per pair of waves,
-// its lanes each walking a key row and one wave summing the readout (1.08 ms
-// for 4001 queries x 389 slots x 32, 768 wide, of which the readout most).
-// Here the keys pass through LDS transposed, 32 dimensions at a time, so lane
-// j reads slot j + 64q at consecutive addresses and one conversion to f64
-// serves QG queries; every squared difference, sum, distance, weight and sum
-// of weights is formed by the same operations in the same order as there, so
-// weights and minima carry the same bits, whichever kernel a call takes.
-// The readout is a product on the matrix cores (fp32): with it that read takes
-// 0.09 ms (50 us here, 34 us the product), against a floor of 16 us for the
-// product at the fp32 matrix rate.
+// its lanes each walking a key row and one wave summing the readout.  Here the
+// keys pass through LDS transposed, 32 dimensions at a time, so lane j reads
+// slot j + 64q at consecutive addresses and one conversion to f64 serves QG
+// queries; every squared difference, sum, distance, weight and sum of weights
+// is formed by the same operations in the same order as there, so weights and
+// minima carry the same bits, whichever kernel a call takes.
+// The readout is a product on the matrix cores (fp32): one of the whole call's
+// weights with the transposed values, through scratch, or (READ) inside the
+// kernel from the weights in LDS and the row-major bank, without scratch and with
+// the same bits.
 // Bound: f64 VALU issue (3 operations per query, slot and dimension, about
 // 200 for each distance's asinh).
 constexpr int SW_DC = 32;        // key dimensions per staged chunk
-constexpr int SW_WAVES = 4;
+constexpr int SW_WAVES = 4;      // weights only
+constexpr int SW_READ_WAVES = 8; // with the readout: 16 queries from two a wave
+constexpr int SW_RING = 4;       // readout: groups of 32 slots loaded ahead, and the one in use
 constexpr int SW_SLOTS = 512;
 constexpr int SW_MAX_DK = 1024;
 
-static size_t soft_wide_lds(int dk, int spl, int qg) {
-  return ((size_t)(SW_DC * (64 * spl + 1) + 3) / 4 * 4 + (size_t)SW_WAVES * qg * ((dk + 3) & ~3)) * sizeof(float) +
-         (size_t)SW_WAVES * spl * 64 * sizeof(double);
+// Floats of the transposed chunk, and of the readout's weights ([rows][pitch],
+// whole 16-query tiles).
+__host__ __device__ constexpr int sw_key_floats(int spl) { return (SW_DC * (64 * spl + 1) + 3) / 4 * 4; }
+__host__ __device__ constexpr int sw_weight_pitch(int spl) { return 64 * spl + 4; }
+__host__ __device__ constexpr int sw_weight_rows(int nw, int qg) { return (nw * qg + 15) / 16 * 16; }
+
+// The chunk of keys, each wave's f64 cells and its query rows; with a readout
+// the cells and the weights take the place of the keys and rows once the sums
+// are formed.
+static size_t soft_wide_lds(int dk, int spl, int nw, int qg, bool read) {
+  const size_t keys = (size_t)sw_key_floats(spl) * 4, cells = (size_t)nw * spl * 64 * 8;
+  const size_t rows = (size_t)nw * qg * ((dk + 3) & ~3) * 4;
+  if (!read) return keys + cells + rows;
+  return std::max(keys + rows, cells + (size_t)sw_weight_rows(nw, qg) * sw_weight_pitch(spl) * 4);
 }
 
-// Readout operand: the weights again, [n, ldw] with zeros past the count.
+// Operand of a readout by a product: the weights again, [n, ldw] with zeros past
+// the count.
 struct SoftReadout {
   float* w = nullptr;
   int ldw = 0;
 };
 
-template <int QG, int SPL>
-__global__ __launch_bounds__(64 * SW_WAVES) void soft_wide_kernel(RetrieveArgs a, SoftReadout ro) {
+template <int QG, int SPL, bool READ>
+__global__ __launch_bounds__(64 * (READ ? SW_READ_WAVES : SW_WAVES)) void soft_wide_kernel(RetrieveArgs a, SoftReadout ro) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  constexpr int KP = 64 * SPL + 1;
+  constexpr int KP = 64 * SPL + 1, NW = READ ? SW_READ_WAVES : SW_WAVES, NT = 64 * NW;
+  constexpr int KEYS = sw_key_floats(SPL), CELLS = 2 * NW * SPL * 64, WP = sw_weight_pitch(SPL);
   const int dk = a.dk, dk_pad = (dk + 3) & ~3;
   const int cnt = a.count_dev ? a.count_dev[0] : a.count;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   float* keyT = smem;  // [SW_DC][KP]
-  double* sacc = reinterpret_cast<double*>(smem + (SW_DC * KP + 3) / 4 * 4) + wave * SPL * 64;  // [SPL][64]
-  float* rows = smem + (SW_DC * KP + 3) / 4 * 4 + 2 * SW_WAVES * SPL * 64 + wave * QG * dk_pad;  // [QG][dk_pad]
-  const int n0 = (blockIdx.x * SW_WAVES + wave) * QG;
+  double* sacc = reinterpret_cast<double*>(smem + (READ ? 0 : KEYS)) + wave * SPL * 64;  // [SPL][64]
+  float* rows = smem + KEYS + (READ ? 0 : CELLS) + wave * QG * dk_pad;                   // [QG][dk_pad]
+  float* wts = smem + CELLS;                                                             // READ: [NW * QG][WP]
+  const int n0 = (blockIdx.x * NW + wave) * QG;
+  const bool first = !READ || blockIdx.y == 0;  // writes what is not the readout
 
   // The wave's queries (rows past the last repeat it and write nothing).
 #pragma unroll
@@ -716,7 +733,7 @@ __global__ __launch_bounds__(64 * SW_WAVES) void soft_wide_kernel(RetrieveArgs a
     if (a.project) {
       const double r = sqrt(sumsq_f64(mine, dk));
       const double scale = r == 0.0 ? 1.0 : fmin(r / (1.0 + r), kMaxRadius) / r;
-      if (a.q_norm && lane < QG && n0 + lane < a.n) a.q_norm[n0 + lane] = (float)fmin(r, (double)FLT_MAX);
+      if (a.q_norm && first && lane < QG && n0 + lane < a.n) a.q_norm[n0 + lane] = (float)fmin(r, (double)FLT_MAX);
       wave_sync();
 #pragma unroll
       for (int g = 0; g < QG; ++g) {
@@ -729,7 +746,7 @@ __global__ __launch_bounds__(64 * SW_WAVES) void soft_wide_kernel(RetrieveArgs a
 #pragma unroll
     for (int g = 0; g < QG; ++g) {
       q_sq[g] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(own), g));
-      if (a.q_pnc && n0 + g < a.n)
+      if (a.q_pnc && first && n0 + g < a.n)
         for (int i = lane; i < dk; i += 64) a.q_pnc[(size_t)(n0 + g) * dk + i] = rows[g * dk_pad + i];
     }
   }
@@ -746,16 +763,16 @@ __global__ __launch_bounds__(64 * SW_WAVES) void soft_wide_kernel(RetrieveArgs a
     if (vec) {
       constexpr int PC = SW_DC / 4;  // 16-byte pieces of a slot's chunk
       constexpr int U = 16;          // loads in flight per thread: a chunk of 512 slots in one round
-      for (int e0 = tid; e0 < cnt * PC; e0 += U * 64 * SW_WAVES) {
+      for (int e0 = tid; e0 < cnt * PC; e0 += U * NT) {
         float4 v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const int e = min(e0 + u * 64 * SW_WAVES, cnt * PC - 1);
+          const int e = min(e0 + u * NT, cnt * PC - 1);
           v[u] = *reinterpret_cast<const float4*>(a.keys + (size_t)(e / PC) * dk + c0 + min(4 * (e % PC), dc - 4));
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const int e = e0 + u * 64 * SW_WAVES, i = 4 * (e % PC);
+          const int e = e0 + u * NT, i = 4 * (e % PC);
           if (e < cnt * PC && i < dc) {
             float* k = keyT + i * KP + e / PC;
             k[0] = v[u].x, k[KP] = v[u].y, k[2 * KP] = v[u].z, k[3 * KP] = v[u].w;
@@ -763,7 +780,7 @@ __global__ __launch_bounds__(64 * SW_WAVES) void soft_wide_kernel(RetrieveArgs a
         }
       }
     } else {
-      for (int e = tid; e < cnt * SW_DC; e += 64 * SW_WAVES) {
+      for (int e = tid; e < cnt * SW_DC; e += NT) {
         const int i = e % SW_DC;
         if (i < dc) keyT[i * KP + e / SW_DC] = a.keys[(size_t)(e / SW_DC) * dk + c0 + i];
       }
@@ -792,6 +809,7 @@ __global__ __launch_bounds__(64 * SW_WAVES) void soft_wide_kernel(RetrieveArgs a
       }
     }
   }
+  if constexpr (READ) __syncthreads();  // the cells overlay the keys
 #pragma unroll
   for (int g = 0; g < QG; ++g) {
     const int n = n0 + g;
@@ -812,7 +830,7 @@ __global__ __launch_bounds__(64 * SW_WAVES) void soft_wide_kernel(RetrieveArgs a
       }
     }
     const float min_dist = cnt > 0 ? wave_min(local_min) : 0.0f;
-    if (a.out_min && lane == 0) a.out_min[n] = min_dist;
+    if (a.out_min && first && lane == 0) a.out_min[n] = min_dist;
     float e[SPL], part = 0.0f;
 #pragma unroll
     for (int j = 0; j < SPL; ++j) {
@@ -845,13 +863,100 @@ __global__ __launch_bounds__(64 * SW_WAVES) void soft_wide_kernel(RetrieveArgs a
     for (int j = 0; j < SPL; ++j) {
       const int s = lane + 64 * j;
       const float w = s < cnt ? e[j] / sum : 0.0f;
-      if (s < a.capacity) put_weight(a, n, s, w);
-      if (ro.w && s < ro.ldw) ro.w[(size_t)n * ro.ldw + s] = w;
+      if (first && s < a.capacity) put_weight(a, n, s, w);
+      if constexpr (READ)
+        wts[(wave * QG + g) * WP + s] = w;
+      else if (ro.w && s < ro.ldw)
+        ro.w[(size_t)n * ro.ldw + s] = w;
     }
+    if (!first) continue;
     for (int s = lane + 64 * SPL; s < a.capacity; s += 64) put_weight(a, n, s, 0.0f);
     if (a.out_idx)
       for (int r = lane; r < a.top_k; r += 64)
         a.out_idx[(size_t)n * a.top_k + r] = r < cnt ? (uint32_t)r : 0xFFFFFFFFu;
+  }
+  if constexpr (READ) {
+    // out[query, column] = sum over slots of weight * value.  MFMA 16 x 16 x 4:
+    // the columns' values are the rows of the product (lane l: columns 2i and
+    // 2i + 1, i = l % 16, of two tiles), the queries its columns; a lane ends
+    // with eight neighbouring columns of query l % 16.  Lane group l / 16 takes
+    // the slots of every eight that put the additions in the fp32 GEMM's order
+    // (slots 0, 4, 1, 5, 2, 6, 3, 7 of each eight): the bits are those of the
+    // product of launch_soft_wide.  Weights past the count are zero and the
+    // values there (the last slot's again) are masked.
+    typedef float f32x4_t __attribute__((ext_vector_type(4)));
+    constexpr int RT = sw_weight_rows(NW, QG) / 16;
+    __syncthreads();
+    const int dv = a.dv, i16 = lane & 15, kq = lane >> 4, ng = (cnt + 31) / 32;
+    const int s0 = 4 * (kq & 1) + (kq >> 1);
+    auto slot = [&](int u) { return s0 + 8 * (u >> 1) + 2 * (u & 1); };  // of 32, step u
+    const bool vec2 = dv % 2 == 0 && ((uintptr_t)a.values & 7) == 0;
+    const bool vec4 = dv % 4 == 0 && ((uintptr_t)a.out_val & 15) == 0;
+    // blockIdx.y: a share of the column tiles (soft_wide_split).
+    for (int c0 = 32 * (wave + NW * blockIdx.y); c0 < dv; c0 += 32 * NW * gridDim.y) {
+      const int ca = min(c0 + 2 * i16, vec2 ? dv - 2 : dv - 1), cb = min(c0 + 2 * i16 + 1, dv - 1);
+      auto load = [&](int grp, float2 (&v)[8]) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const float* row = a.values + (size_t)min(32 * grp + slot(u), cnt - 1) * dv;
+          if (vec2)
+            v[u] = *reinterpret_cast<const float2*>(row + ca);
+          else
+            v[u].x = row[ca], v[u].y = row[cb];
+        }
+      };
+      f32x4_t acc[RT][2];
+#pragma unroll
+      for (int t = 0; t < RT; ++t) acc[t][0] = acc[t][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      // A ring of SW_RING groups' values in flight: with one workgroup on a CU
+      // the loads' latency is what a group costs.
+      float2 v[SW_RING][8];
+#pragma unroll
+      for (int r = 0; r < SW_RING - 1; ++r) load(min(r, ng - 1), v[r]);
+      for (int g0 = 0; g0 < ng; g0 += SW_RING) {
+#pragma unroll
+        for (int r = 0; r < SW_RING; ++r) {
+          const int grp = g0 + r;
+          if (grp >= ng) break;
+          load(min(grp + SW_RING - 1, ng - 1), v[(r + SW_RING - 1) % SW_RING]);
+          float w[RT][8];
+#pragma unroll
+          for (int t = 0; t < RT; ++t) {
+            const float* pw = wts + (16 * t + i16) * WP + 32 * grp;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) w[t][u] = pw[slot(u)];
+          }
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const bool live = 32 * grp + slot(u) < cnt;
+            const float vx = live ? v[r][u].x : 0.0f, vy = live ? v[r][u].y : 0.0f;
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+              acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vx, w[t][u], acc[t][0], 0, 0, 0);
+              acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vy, w[t][u], acc[t][1], 0, 0, 0);
+            }
+          }
+        }
+      }
+      const int col = c0 + 8 * kq;
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        const int q = 16 * t + i16, n = blockIdx.x * NW * QG + q;
+        if (q >= NW * QG || n >= a.n) continue;
+        float* out = a.out_val + (size_t)n * dv + col;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const float o[4] = {acc[t][0][2 * h], acc[t][1][2 * h], acc[t][0][2 * h + 1], acc[t][1][2 * h + 1]};
+          if (vec4) {
+            if (col + 4 * h < dv) *reinterpret_cast<float4*>(out + 4 * h) = make_float4(o[0], o[1], o[2], o[3]);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (col + 4 * h + e < dv) out[4 * h + e] = o[e];
+          }
+        }
+      }
+    }
   }
 }
 
@@ -1571,21 +1676,28 @@ static bool soft_wide_fits(const RetrieveArgs& a) {
          a.dk <= SW_MAX_DK && !(a.out_val && a.count_dev) && !soft_read_fits(a) &&
          (a.out_val || a.n >= SW_MIN_WEIGHTS);
 }
-// Readout width (the count in whole 16-wide K steps) and queries per pass.
+// Readout width (the count in whole 16-wide K steps) and queries per pass of
+// the readout by a product.
 static int soft_wide_ld(const RetrieveArgs& a) { return (a.count + 15) & ~15; }
-static int soft_wide_chunk(const RetrieveArgs& a) { return std::min(a.n, a.chunk > 0 ? a.chunk : 32768); }
-static size_t soft_wide_scratch(const RetrieveArgs& a) {
-  return (size_t)soft_wide_ld(a) * ((size_t)soft_wide_chunk(a) + a.dv) * sizeof(float);
+static int soft_wide_chunk(const RetrieveArgs& a) { return std::min(a.n, 32768); }
+// Whether a readout is that product (the bits are the same either way).  Fused,
+// sixteen or 32 queries of a workgroup read the whole bank: less to launch, but
+// more L2 traffic and, of few queries, two waves to a SIMD in the distances.
+// Product / fused, us: 17 slots of 5, 7 wide, 1 query 13.1 / 6.6 and 4000 14.1
+// / 9.6; 256 wide, 300 slots of 64, 1000 queries 30.0 / 38.5, 1400 47.5 / 38.6,
+// 8192 108 / 84; 768 wide, 512 slots of 32, 1000 35.4 / 61.5, 4001 91 / 94,
+// 20000 364 / 427; 2000 wide, 5000 queries 204 / 300.
+static bool soft_wide_product(const RetrieveArgs& a) {
+  return a.out_val && a.chunk == 0 && a.count > 64 && (a.dv > 256 || a.n <= 1280);
 }
 
 size_t retrieve_scratch_bytes(const RetrieveArgs& a) {
   if (ranked_read_fits(a)) return ranked_scratch_bytes(a.dk, ranked_chunk(a));
-  if (!a.out_val || !soft_wide_fits(a)) return 0;
-  // The allocation-free call's scratch is a fixed size: reads that need more
-  // keep the general kernel.
-  const size_t bytes = soft_wide_scratch(a);
-  return a.chunk > 0 && bytes > kNoallocScratchBytes ? 0 : bytes;
+  if (!soft_wide_fits(a) || !soft_wide_product(a)) return 0;
+  return (size_t)soft_wide_ld(a) * ((size_t)soft_wide_chunk(a) + a.dv) * sizeof(float);
 }
+
+bool retrieve_needs_scratch(const RetrieveArgs& a) { return ranked_read_fits(a); }
 
 Status noalloc_scratch_address(void** out) {
   static std::mutex mu;
@@ -1636,10 +1748,13 @@ static Status allow_large_lds() {
 #undef PSSA_SOFT_QP_FN
   };
   const void* wide[] = {
-#define PSSA_SOFT_WIDE_FN(SPL)                                       \
-  reinterpret_cast<const void*>(&soft_wide_kernel<1, SPL>),          \
-      reinterpret_cast<const void*>(&soft_wide_kernel<2, SPL>),      \
-      reinterpret_cast<const void*>(&soft_wide_kernel<4, SPL>),
+#define PSSA_SOFT_WIDE_FN(SPL)                                        \
+  reinterpret_cast<const void*>(&soft_wide_kernel<1, SPL, false>),    \
+      reinterpret_cast<const void*>(&soft_wide_kernel<2, SPL, false>), \
+      reinterpret_cast<const void*>(&soft_wide_kernel<4, SPL, false>), \
+      reinterpret_cast<const void*>(&soft_wide_kernel<1, SPL, true>),  \
+      reinterpret_cast<const void*>(&soft_wide_kernel<2, SPL, true>),  \
+      reinterpret_cast<const void*>(&soft_wide_kernel<4, SPL, true>),
       PSSA_SOFT_WIDE_FN(1) PSSA_SOFT_WIDE_FN(2) PSSA_SOFT_WIDE_FN(4) PSSA_SOFT_WIDE_FN(8)
 #undef PSSA_SOFT_WIDE_FN
   };
@@ -1680,26 +1795,54 @@ bool retrieve_fuses_query(const RetrieveArgs& a) {
          soft_read_lds(a.dk, a.capacity, 1, nwv) + soft_qp_lds(a.qk, nwv) <= 160 * 1024;
 }
 
-// Queries per wave: enough workgroups for two per CU before a wave takes more
-// queries per pass over the keys.
-static int soft_wide_qg(int n) {
-  const int wg1 = (n + SW_WAVES - 1) / SW_WAVES;
-  return wg1 >= 2048 ? 4 : wg1 >= 512 ? 2 : 1;
+// Queries per wave: enough workgroups for two per CU (of four waves) before a
+// wave takes more queries per pass over the keys; fused, four from 256
+// workgroups of sixteen queries (5000 queries, 512 slots of 32, 768 wide: two
+// a wave 177 us, four 142; 4001: 94 / 115).
+static int soft_wide_qg(const RetrieveArgs& a, bool read) {
+  int qg = a.n > 4 * 2047 || (read && a.n > 4096) ? 4 : a.n > 4 * 511 ? 2 : 1;
+  while (read && qg > 1 && soft_wide_lds(a.dk, soft_spl(a.count), SW_READ_WAVES, qg, true) > 160 * 1024) qg /= 2;
+  return qg;
+}
+
+// Shares of the columns of a fused readout: with fewer workgroups than CUs each
+// query's distances are formed by several of them, each reading out its share
+// (not where one's readout may replace queries that another has yet to read).
+static unsigned soft_wide_split(const RetrieveArgs& a, unsigned blocks) {
+  const uintptr_t q = (uintptr_t)a.q, o = (uintptr_t)a.out_val;
+  if (q < o + (size_t)a.n * a.dv * 4 && o < q + (size_t)a.n * a.ld_q * 4) return 1;
+  const unsigned rounds = (unsigned)((a.dv + 32 * SW_READ_WAVES - 1) / (32 * SW_READ_WAVES));
+  return std::max(1u, std::min(rounds, 256 / blocks));
+}
+
+template <bool READ>
+static Status launch_soft_wide_kernel(hipStream_t stream, const RetrieveArgs& a, const SoftReadout& ro) {
+  const int spl = soft_spl(a.count), qg = soft_wide_qg(a, READ), nw = READ ? SW_READ_WAVES : SW_WAVES;
+  const unsigned blocks = (unsigned)((a.n + nw * qg - 1) / (nw * qg));
+  const dim3 grid(blocks, READ ? soft_wide_split(a, blocks) : 1);
+  const size_t lds = soft_wide_lds(a.dk, spl, nw, qg, READ);
+#define PSSA_SOFT_WIDE(QG, SPL) \
+  if (qg == QG && spl == SPL) soft_wide_kernel<QG, SPL, READ><<<grid, 64 * nw, lds, stream>>>(a, ro);
+  PSSA_SOFT_WIDE(1, 1) PSSA_SOFT_WIDE(1, 2) PSSA_SOFT_WIDE(1, 4) PSSA_SOFT_WIDE(1, 8)
+  PSSA_SOFT_WIDE(2, 1) PSSA_SOFT_WIDE(2, 2) PSSA_SOFT_WIDE(2, 4) PSSA_SOFT_WIDE(2, 8)
+  PSSA_SOFT_WIDE(4, 1) PSSA_SOFT_WIDE(4, 2) PSSA_SOFT_WIDE(4, 4) PSSA_SOFT_WIDE(4, 8)
+#undef PSSA_SOFT_WIDE
+  PSSA_LAUNCH_CHECK("soft_wide");
+  return Status::Ok();
 }
 
 static Status launch_soft_wide(hipStream_t stream, const RetrieveArgs& a) {
   PSSA_RETURN_IF(allow_large_lds());
-  const int spl = soft_spl(a.count), ld = soft_wide_ld(a);
-  const int chunk = a.out_val ? soft_wide_chunk(a) : a.n;
-  float* vt = nullptr;
+  if (!a.out_val) return launch_soft_wide_kernel<false>(stream, a, SoftReadout());
+  const size_t need = retrieve_scratch_bytes(a);
+  if (!need || !a.scratch || a.scratch_bytes < need) return launch_soft_wide_kernel<true>(stream, a, SoftReadout());
+  const int ld = soft_wide_ld(a), chunk = soft_wide_chunk(a);
+  float* vt = static_cast<float*>(a.scratch);
   SoftReadout ro;
-  if (a.out_val) {
-    vt = static_cast<float*>(a.scratch);
-    ro.w = vt + (size_t)ld * a.dv;
-    ro.ldw = ld;
-    soft_values_kernel<<<dim3((ld + 31) / 32, (a.dv + 31) / 32), 256, 0, stream>>>(a.values, a.count, a.dv, vt, ld);
-    PSSA_LAUNCH_CHECK("soft_values");
-  }
+  ro.w = vt + (size_t)ld * a.dv;
+  ro.ldw = ld;
+  soft_values_kernel<<<dim3((ld + 31) / 32, (a.dv + 31) / 32), 256, 0, stream>>>(a.values, a.count, a.dv, vt, ld);
+  PSSA_LAUNCH_CHECK("soft_values");
   for (int q0 = 0; q0 < a.n; q0 += chunk) {
     RetrieveArgs c = a;
     c.n = std::min(chunk, a.n - q0);
@@ -1711,22 +1854,11 @@ static Status launch_soft_wide(hipStream_t stream, const RetrieveArgs& a) {
     if (a.weights16) c.weights16 = a.weights16 + (size_t)q0 * a.capacity;
     if (a.out_min) c.out_min = a.out_min + q0;
     if (a.out_idx) c.out_idx = a.out_idx + (size_t)q0 * a.top_k;
-    const int qg = soft_wide_qg(c.n);
-    const unsigned blocks = (unsigned)((c.n + SW_WAVES * qg - 1) / (SW_WAVES * qg));
-    const size_t lds = soft_wide_lds(a.dk, spl, qg);
-#define PSSA_SOFT_WIDE(QG, SPL) \
-  if (qg == QG && spl == SPL) soft_wide_kernel<QG, SPL><<<blocks, 64 * SW_WAVES, lds, stream>>>(c, ro);
-    PSSA_SOFT_WIDE(1, 1) PSSA_SOFT_WIDE(1, 2) PSSA_SOFT_WIDE(1, 4) PSSA_SOFT_WIDE(1, 8)
-    PSSA_SOFT_WIDE(2, 1) PSSA_SOFT_WIDE(2, 2) PSSA_SOFT_WIDE(2, 4) PSSA_SOFT_WIDE(2, 8)
-    PSSA_SOFT_WIDE(4, 1) PSSA_SOFT_WIDE(4, 2) PSSA_SOFT_WIDE(4, 4) PSSA_SOFT_WIDE(4, 8)
-#undef PSSA_SOFT_WIDE
-    PSSA_LAUNCH_CHECK("soft_wide");
-    if (a.out_val) {
-      EpiParams ep;
-      ep.out32 = a.out_val + (size_t)q0 * a.dv;
-      ep.ld32 = a.dv;
-      PSSA_RETURN_IF(launch_gemm(stream, PSSA_HIP_F32, ro.w, ld, vt, ld, c.n, a.dv, ld, ep));
-    }
+    PSSA_RETURN_IF(launch_soft_wide_kernel<false>(stream, c, ro));
+    EpiParams ep;
+    ep.out32 = a.out_val + (size_t)q0 * a.dv;
+    ep.ld32 = a.dv;
+    PSSA_RETURN_IF(launch_gemm(stream, PSSA_HIP_F32, ro.w, ld, vt, ld, c.n, a.dv, ld, ep));
   }
   return Status::Ok();
 }
@@ -1810,8 +1942,7 @@ Status launch_retrieve(hipStream_t stream, const RetrieveArgs& a) {
     }
     return Status::Ok();
   }
-  if (soft_wide_fits(a) && (!a.out_val || (a.scratch && retrieve_scratch_bytes(a) && a.scratch_bytes >= retrieve_scratch_bytes(a))))
-    return launch_soft_wide(stream, a);
+  if (soft_wide_fits(a)) return launch_soft_wide(stream, a);
   const int dk_pad = (a.dk + 3) & ~3;
   const size_t lds = (size_t)RETRIEVE_QPB * (dk_pad + a.capacity) * sizeof(float);
   if (lds > 128 * 1024) return Status::Invalid("retrieve: d_key + capacity too large for LDS");

@@ -136,3 +136,81 @@ def test_noalloc_retrieval_allocates_nothing_on_a_fresh_context():
     say(f"device bytes in use: +{free0 - free1} (allocation-free), +{free1 - free2} (allocating)")
     assert abs(free0 - free1) < (1 << 20)
     assert free1 - free2 >= (16 << 20)
+
+
+def soft_read(dev, fn, q, bank, capacity, count):
+    n, dk = q.shape
+    dv = bank[2].shape[1]
+    bufs = [dev.upload(a) for a in (q, *bank)]
+    out, mn = dev.empty((n, dv), np.float32), dev.empty((n,), np.float32)
+    fn(bufs[0].ptr, n, bufs[1].ptr, bufs[2].ptr, bufs[3].ptr, capacity, count, dk, dv, 0.1, 0, out.ptr, mn.ptr, None)
+    dev.synchronize()
+    res = out.to_host(), mn.to_host()
+    for b in bufs + [out, mn]:
+        b.close()
+    return res
+
+
+@pytest.mark.parametrize("n,capacity,count,dk,dv", [(8200, 512, 512, 32, 1600), (20001, 512, 300, 64, 96),
+                                                    (2050, 600, 512, 1024, 33), (8200, 512, 500, 900, 6),
+                                                    (3, 64, 17, 5, 7), (4097, 130, 129, 128, 770)])
+def test_noalloc_full_soft_read_matches_the_allocating_entry_point(hip, n, capacity, count, dk, dv):
+    """top_k = 0 through both entry points, at shapes whose readout would not
+    fit the static scratch and at ones that would, and each query alone (or in
+    a short call) against its row of the whole one: the same bits, whether the
+    readout is a product of its own or part of the read."""
+    say(f"full soft read: {n} queries, d_key {dk}, d_val {dv}, {count} of {capacity} slots")
+    rng = np.random.default_rng(dv)
+    keys, vals, q = ball(rng, capacity, dk), ball(rng, capacity, dv), ball(rng, n, dk)
+    bank = (keys, squared_norms(keys), vals)
+    out, mn = soft_read(hip, hip.retrieve_resident, q, bank, capacity, count)
+    out_n, mn_n = soft_read(hip, hip.retrieve_resident_noalloc, q, bank, capacity, count)
+    np.testing.assert_array_equal(out_n.view(np.uint32), out.view(np.uint32))
+    np.testing.assert_array_equal(mn_n.view(np.uint32), mn.view(np.uint32))
+    for a, b in ((0, 1), (n - 1, n), (n // 2, min(n, n // 2 + 37))):
+        part, low = soft_read(hip, hip.retrieve_resident, q[a:b], bank, capacity, count)
+        np.testing.assert_array_equal(part.view(np.uint32), out[a:b].view(np.uint32))
+        np.testing.assert_array_equal(low.view(np.uint32), mn[a:b].view(np.uint32))
+
+
+def test_noalloc_full_soft_read_uses_neither_memory_nor_the_shared_scratch():
+    """On a context of its own a full soft read through the allocation-free
+    entry point leaves the device memory in use as it is.  It does not touch
+    the static scratch either, so full soft reads may overlap other calls:
+    two contexts run them at once, with ranked reads between, and every result
+    is the one of a call alone."""
+    from pssa_amd import HipDevice
+
+    rng = np.random.default_rng(12)
+    n, C1, dk, dv = 30000, 512, 32, 768
+    keys, vals, q = ball(rng, C1, dk), ball(rng, C1, dv), ball(rng, n, dk)
+    devs = [HipDevice(0), HipDevice(0)]
+    bufs = [devs[0].upload(a) for a in (q, keys, squared_norms(keys), vals)]
+    outs = [devs[0].empty((n, dv), np.float32) for _ in range(3)]
+    idx = devs[0].empty((n, 8), np.uint32)
+
+    def call(dev, out, n_q, k=0):
+        dev.retrieve_resident_noalloc(bufs[0].ptr, n_q, bufs[1].ptr, bufs[2].ptr, bufs[3].ptr, C1, C1, dk, dv, 0.1, k,
+                                      out.ptr, None, idx.ptr if k else None)
+
+    for d in devs:
+        call(d, outs[0], 64)
+        d.synchronize()
+    free0 = _free_device_bytes()
+    say("fresh context: full soft read of", n, "queries")
+    call(devs[0], outs[0], n)
+    devs[0].synchronize()
+    free1 = _free_device_bytes()
+    alone = outs[0].to_host()
+    say("two contexts at once, one with ranked reads")
+    for _ in range(3):
+        call(devs[0], outs[1], n)
+        call(devs[1], outs[2], n, k=8)
+    for d in devs:
+        d.synchronize()
+    np.testing.assert_array_equal(outs[1].to_host().view(np.uint32), alone.view(np.uint32))
+    for b in bufs + outs + [idx]:
+        b.close()
+    for d in devs:
+        d.close()
+    assert abs(free0 - free1) < (1 << 20)
