@@ -256,7 +256,8 @@ __global__ __launch_bounds__(256) void retrieve_kernel(RetrieveArgs a) {
             const float e = expf((min_dist - sdist[s]) / a.tau);
             sdist[s] = e;
             part += e;
-            if (a.hgate) part_h += (e * a.hgate[s]) * hybrid_decay(a, s, n);
+            // One rounding, written out: soft_wide_kernel's sum has the same bits.
+            if (a.hgate) part_h = fmaf(e * a.hgate[s], hybrid_decay(a, s, n), part_h);
           }
           const float sum_p = wave_sum(part);
           const float sum_h = a.hgate ? wave_sum(part_h) : 0.0f;
@@ -847,9 +848,10 @@ __global__ __launch_bounds__(64 * (READ ? SW_READ_WAVES : SW_WAVES)) void soft_w
       for (int j = 0; j < SPL; ++j) {
         const int s = lane + 64 * j;
         if (s < cnt) {
-          const float eh = (expf((min_dist - (float)sacc[s]) / a.tau) * a.hgate[s]) * hybrid_decay(a, s, a.row0 + n);
-          sacc[s] = (double)eh;
-          part_h += eh;
+          const float eg = expf((min_dist - (float)sacc[s]) / a.tau) * a.hgate[s];
+          const float decay = hybrid_decay(a, s, a.row0 + n);
+          sacc[s] = (double)(eg * decay);
+          part_h = fmaf(eg, decay, part_h);  // as retrieve_kernel's
         }
       }
       const float sum_h = wave_sum(part_h);

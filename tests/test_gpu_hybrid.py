@@ -217,3 +217,37 @@ def test_hybrid_toggle_recaptures_decode_graph(hip):
         layer.close()
     for x, y in zip(*res):
         np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("hybrid", [False, True])
+def test_wide_key_prefill_does_not_depend_on_its_row_count(hip, dtype, hybrid):
+    """Keys of 128 with a partly filled bank: a prompt of 1024 rows or more (per
+    lane group) reads the bank with the wide soft read, shorter ones with the
+    general kernel.  One prefill of one lane and of two (two groups), and the
+    same prompts in pieces below the line, give the same logits, carries and
+    ages bit for bit; the hybrid read with gates below 1, some 0, and decay."""
+    say("wide-key prefill by rows", dtype, hybrid)
+    cfg = PSSAConfig(depth=2, d_vocab=97, d_latent=64, d_state=16, d_mem_key=128, mem_capacity=300)
+    w = ModelWeights.init(cfg, 5, "baseline")
+    w.populate_banks(6, count=250)
+    if hybrid:
+        rng = np.random.default_rng(7)
+        for b in w.blocks:
+            b.mem_hybrid_gate[:250] = rng.uniform(0.05, 1.0, 250).astype(np.float32)
+            b.mem_hybrid_gate[::6] = 0.0
+            b.mem_hybrid_age[:250] = rng.integers(0, 60, 250).astype(np.uint64)
+        w.set_hybrid_read(True, 0.999)
+    for lanes, T in ((1, 1300), (2, 1030)):
+        ids = np.random.default_rng(lanes).integers(0, cfg.d_vocab, (lanes, T), dtype=np.uint32)
+        a = PSSALayer(hip, w, lanes=lanes, max_tokens=lanes * T, weight_dtype=dtype)
+        b = PSSALayer(hip, w, lanes=lanes, max_tokens=lanes * T, weight_dtype=dtype)
+        la = a.prefill_inference(ids)
+        for t in range(0, T, 470):
+            lb = b.prefill_inference(ids[:, t:t + 470])
+        np.testing.assert_array_equal(la.view(np.uint32), lb.view(np.uint32))
+        np.testing.assert_array_equal(a.get_carry().view(np.uint32), b.get_carry().view(np.uint32))
+        for l in range(cfg.depth):
+            np.testing.assert_array_equal(a.get_hybrid(l)[1], b.get_hybrid(l)[1])
+        a.close()
+        b.close()

@@ -153,12 +153,13 @@ def soft_read(dev, fn, q, bank, capacity, count):
 
 @pytest.mark.parametrize("n,capacity,count,dk,dv", [(8200, 512, 512, 32, 1600), (20001, 512, 300, 64, 96),
                                                     (2050, 600, 512, 1024, 33), (8200, 512, 500, 900, 6),
-                                                    (3, 64, 17, 5, 7), (4097, 130, 129, 128, 770)])
+                                                    (3, 64, 17, 5, 7), (4097, 130, 129, 128, 770),
+                                                    (40000, 512, 389, 32, 300)])
 def test_noalloc_full_soft_read_matches_the_allocating_entry_point(hip, n, capacity, count, dk, dv):
     """top_k = 0 through both entry points, at shapes whose readout would not
     fit the static scratch and at ones that would, and each query alone (or in
     a short call) against its row of the whole one: the same bits, whether the
-    readout is a product of its own or part of the read."""
+    readout is a product of its own (of up to 32768 queries) or part of the read."""
     say(f"full soft read: {n} queries, d_key {dk}, d_val {dv}, {count} of {capacity} slots")
     rng = np.random.default_rng(dv)
     keys, vals, q = ball(rng, capacity, dk), ball(rng, capacity, dv), ball(rng, n, dk)
