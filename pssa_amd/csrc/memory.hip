@@ -1688,9 +1688,12 @@ static int soft_wide_chunk(const RetrieveArgs& a) { return std::min(a.n, 32768);
 // Product / fused, us: 17 slots of 5, 7 wide, 1 query 13.1 / 6.6 and 4000 14.1
 // / 9.6; 256 wide, 300 slots of 64, 1000 queries 30.0 / 38.5, 1400 47.5 / 38.6,
 // 8192 108 / 84; 768 wide, 512 slots of 32, 1000 35.4 / 61.5, 4001 91 / 94,
-// 20000 364 / 427; 2000 wide, 5000 queries 204 / 300.
+// 20000 364 / 427; 2000 wide, 5000 queries 204 / 300; 64 slots of 32, 500 wide,
+// 1000 15.9 / 14.2, 768 wide 16.3 / 18.3, 4000 wide, 100 16.3 / 14.1, 1000 22.8 / 42.8.
 static bool soft_wide_product(const RetrieveArgs& a) {
-  return a.out_val && a.chunk == 0 && a.count > 64 && (a.dv > 256 || a.n <= 1280);
+  if (!a.out_val || a.chunk > 0) return false;
+  if (a.dv <= 256) return a.count > 64 && a.n <= 1280;
+  return a.count > 64 || (long)a.n * a.dv > (1 << 19);
 }
 
 size_t retrieve_scratch_bytes(const RetrieveArgs& a) {

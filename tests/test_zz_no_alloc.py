@@ -154,7 +154,7 @@ def soft_read(dev, fn, q, bank, capacity, count):
 @pytest.mark.parametrize("n,capacity,count,dk,dv", [(8200, 512, 512, 32, 1600), (20001, 512, 300, 64, 96),
                                                     (2050, 600, 512, 1024, 33), (8200, 512, 500, 900, 6),
                                                     (3, 64, 17, 5, 7), (4097, 130, 129, 128, 770),
-                                                    (40000, 512, 389, 32, 300)])
+                                                    (40000, 512, 389, 32, 300), (1000, 64, 64, 32, 768)])
 def test_noalloc_full_soft_read_matches_the_allocating_entry_point(hip, n, capacity, count, dk, dv):
     """top_k = 0 through both entry points, at shapes whose readout would not
     fit the static scratch and at ones that would, and each query alone (or in
