@@ -612,6 +612,8 @@ class PrefillView {
     return launch_gemm(st, dt, H1_, 2 * d, B.mlp_w2.p, 2 * d, m, d, 2 * d, e_r);
   }
 
+  // Times a head that is not the view's own.
+  Status begin_head_timing() { return tm_.mark(ST_HEAD); }
   Status finish_timing() { return tm_.finish(); }
 
   Status head() {
@@ -720,7 +722,6 @@ static Status bump_hybrid_ages(pssa_hip_lanes* L, size_t T);
 
 Status run_prefill_ragged(pssa_hip_lanes* L, const RaggedRows& rr) {
   PSSA_RETURN_IF(prefill_groups(L, rr.lane0[rr.groups], rr.max_len, false, &rr));
-  PSSA_RETURN_IF(ragged_head(L, rr));
   for (int g = 0; g < rr.groups; ++g)
     PSSA_RETURN_IF(launch_hist_append(L, rr.ids + rr.row0[g], rr.lane0[g + 1] - rr.lane0[g], 0, rr.spans + 3 * rr.lane0[g]));
   return bump_hybrid_ages(L, rr.max_len);
@@ -839,12 +840,15 @@ static Status prefill_groups(pssa_hip_lanes* L, size_t n_lanes, size_t T, bool t
       PSSA_HIP_TRY(hipEventRecord(L->ev_join[g - 1], L->aux_stream[g - 1]));
       PSSA_HIP_TRY(hipStreamWaitEvent(st, L->ev_join[g - 1], 0));
     }
-    return Status::Ok();
+    return view_head ? Status::Ok() : ragged_head(L, *rr);
   }
   PrefillView v(L, st, 0, n_lanes, T, taps, L->timing, nullptr, ypart, rr, 0, false);
   PSSA_RETURN_IF(v.embed());
   for (size_t l = 0; l < c.depth; ++l) PSSA_RETURN_IF(v.layer(l));
-  return view_head ? v.head() : v.finish_timing();
+  if (view_head) return v.head();
+  PSSA_RETURN_IF(v.begin_head_timing());
+  PSSA_RETURN_IF(ragged_head(L, *rr));
+  return v.finish_timing();
 }
 
 }  // namespace pssa

@@ -387,6 +387,31 @@ def test_ragged_rows_equal_single_lanes_bitwise(hip, d_state, dtype, hybrid):
             one.close()
 
 
+def test_ragged_stage_times_cover_every_stage(hip):
+    """Stage timing of a ragged prefill: each stage a prefill of one length
+    spends time in, the head among them, and the same logits as untimed."""
+    say("ragged stage times")
+    cfg = PSSAConfig(depth=2, d_vocab=151, d_latent=72, d_state=16, d_mem_key=8, mem_capacity=30)
+    w = ModelWeights.init(cfg, 17, "baseline")
+    w.populate_banks(18, count=25)
+    rng = np.random.default_rng(3)
+    seqs = [rng.integers(0, cfg.d_vocab, n, dtype=np.uint32) for n in (70, 1, 90)]
+    layer = PSSALayer(hip, w, lanes=3, max_tokens=210)
+    plain = layer.prefill_ragged(seqs)
+    layer.set_stage_timing(True)
+    layer.reset_recurrent_state()
+    layer.prefill_inference(np.stack([seqs[0]] * 3))
+    uniform = layer.stage_times()
+    layer.reset_recurrent_state()
+    timed = layer.prefill_ragged(seqs)
+    ragged = layer.stage_times()
+    np.testing.assert_array_equal(timed, plain)
+    for stage, ms in uniform.items():
+        assert (ragged[stage] > 0.0) == (ms > 0.0), (stage, ms, ragged[stage])
+    assert ragged["head"] > 0.0
+    layer.close()
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 def test_memory_top_k_model_matches_oracle(hip, dtype):
     """set_memory_top_k on the model (src/pssa.rs:2215-2226): prefill and
