@@ -237,11 +237,8 @@ int pssa_hip_device_alloc(pssa_hip_ctx* ctx, size_t bytes, void** out, char* err
     std::lock_guard<std::mutex> g(ctx->mu);
     PSSA_HIP_TRY(hipSetDevice(ctx->device));
     void* p = nullptr;
-    const hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      return Status::NoMem(std::string("hipMalloc: ") + hipGetErrorString(e));
-    }
+    const hipError_t e = pssa::device_malloc(&p, bytes);
+    if (e != hipSuccess) return Status::NoMem(std::string("hipMalloc: ") + hipGetErrorString(e));
     *out = p;
     return Status::Ok();
   };
@@ -790,10 +787,8 @@ static Status bind_retrieve_scratch(pssa_hip_ctx* ctx, pssa::RetrieveArgs& ra) {
     if (ctx->scratch) PSSA_HIP_TRY(hipFree(ctx->scratch));
     ctx->scratch = nullptr;
     ctx->scratch_bytes = 0;
-    const hipError_t e = hipMalloc(&ctx->scratch, need_bytes);
+    const hipError_t e = pssa::device_malloc(&ctx->scratch, need_bytes);
     if (e != hipSuccess) {
-      ctx->scratch = nullptr;
-      (void)hipGetLastError();
       if (!pssa::retrieve_needs_scratch(ra)) return Status::Ok();
       return Status::Device("retrieve scratch (" + std::to_string(need_bytes) + " bytes): " + hipGetErrorString(e));
     }
@@ -813,7 +808,7 @@ static Status bind_dense_scan_scratch(pssa_hip_ctx* ctx, int batch, int L, int s
   if (ctx->scratch) PSSA_HIP_TRY(hipFree(ctx->scratch));
   ctx->scratch = nullptr;
   ctx->scratch_bytes = 0;
-  PSSA_HIP_TRY(hipMalloc(&ctx->scratch, need_bytes));
+  PSSA_HIP_TRY(pssa::device_malloc(&ctx->scratch, need_bytes));
   ctx->scratch_bytes = need_bytes;
   return Status::Ok();
 }

@@ -81,11 +81,34 @@ inline Status checked_count(std::initializer_list<size_t> dims, size_t* out, con
 // entry points (each hipMalloc / hipFree pair costs about 20 us, and a call
 // takes up to fifteen).  Blocks are handed out again on the context's one
 // stream, so a block's next user runs after its last; at most kPoolBytes are
-// held, the rest is freed at once, and all of it with the context.
+// held, the rest is freed at once, and all of it with the context or when an
+// allocation of any context finds no memory (device_malloc).
 class DevPool {
  public:
   static constexpr size_t kPoolBytes = (size_t)256 << 20;
-  ~DevPool() { clear(); }
+  DevPool() {
+    std::lock_guard<std::mutex> g(pools().mu);
+    next_ = pools().first;
+    pools().first = this;
+  }
+  ~DevPool() {
+    {
+      std::lock_guard<std::mutex> g(pools().mu);
+      DevPool** at = &pools().first;
+      while (*at != this) at = &(*at)->next_;
+      *at = next_;
+    }
+    clear();
+  }
+  DevPool(const DevPool&) = delete;
+  DevPool& operator=(const DevPool&) = delete;
+  // Frees what every pool of the process holds; false if that was nothing.
+  static bool clear_all() {
+    std::lock_guard<std::mutex> g(pools().mu);
+    bool any = false;
+    for (DevPool* p = pools().first; p; p = p->next_) any |= p->clear();
+    return any;
+  }
   // A held block of at least `n` bytes and not much more, or null.
   void* take(size_t n, size_t* bytes) {
     std::lock_guard<std::mutex> g(mu_);
@@ -111,18 +134,41 @@ class DevPool {
     }
     (void)hipFree(p);
   }
-  void clear() {
+  bool clear() {
     std::lock_guard<std::mutex> g(mu_);
+    const bool any = !free_.empty();
     for (auto& f : free_) (void)hipFree(f.second);
     free_.clear();
     held_ = 0;
+    return any;
   }
 
  private:
+  struct All {
+    std::mutex mu;
+    DevPool* first = nullptr;
+  };
+  static All& pools() {
+    static All* all = new All;  // outlives every context
+    return *all;
+  }
+  DevPool* next_ = nullptr;
   std::mutex mu_;
   std::multimap<size_t, void*> free_;
   size_t held_ = 0;
 };
+
+// hipMalloc; with no memory left, again without the blocks that pools hold.
+inline hipError_t device_malloc(void** p, size_t n) {
+  hipError_t e = hipMalloc(p, n);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    if (DevPool::clear_all()) e = hipMalloc(p, n);
+    if (e != hipSuccess) (void)hipGetLastError();
+  }
+  if (e != hipSuccess) *p = nullptr;
+  return e;
+}
 
 // Device buffer owned by RAII (returned to `pool` when it came from one).
 struct DevBuf {
@@ -165,17 +211,8 @@ struct DevBuf {
       pool = from;
       return Status::Ok();
     }
-    hipError_t e = hipMalloc(&p, n);
-    if (e != hipSuccess && from) {
-      (void)hipGetLastError();
-      from->clear();
-      e = hipMalloc(&p, n);
-    }
-    if (e != hipSuccess) {
-      p = nullptr;
-      (void)hipGetLastError();
-      return Status::NoMem("hipMalloc(" + std::to_string(n) + "): " + hipGetErrorString(e));
-    }
+    const hipError_t e = device_malloc(&p, n);
+    if (e != hipSuccess) return Status::NoMem("hipMalloc(" + std::to_string(n) + "): " + hipGetErrorString(e));
     bytes = n;
     pool = from;
     return Status::Ok();
