@@ -229,7 +229,8 @@ struct DevBuf {
 // with the host's copy of one piece beside the transfer of the next about 230
 // us.  Arrays from 32 KiB (uploads to 1 MiB, where the runtime's own pipeline
 // is as fast) therefore go through pinned slots of the context's; arrays
-// pinned by the caller move directly.  Used with the context's lock held, on
+// pinned by the caller, and any other memory the runtime knows (a device array
+// in a host array's place), move directly.  Used with the context's lock held, on
 // its stream.
 class HostStage {
  public:
@@ -246,7 +247,7 @@ class HostStage {
   // stream.
   Status to_device(void* dst, const void* src, size_t n, hipStream_t st) {
     if (!n) return Status::Ok();
-    if (n >= kMin && n < kSlot && !pinned(src)) {
+    if (n >= kMin && n < kSlot && !known(src)) {
       if (used_ + n > kSlot * kSlots) PSSA_RETURN_IF(drain(st));
       std::memcpy(buf_ + used_, src, n);
       src = buf_ + used_;
@@ -258,7 +259,7 @@ class HostStage {
   // The data is in `dst` at return (after all earlier work of the stream).
   Status to_host(void* dst, const void* src, size_t n, hipStream_t st) {
     if (!n) return Status::Ok();
-    if (n < kMin || pinned(dst)) {
+    if (n < kMin || known(dst)) {
       PSSA_HIP_TRY(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st));
       return drain(st);
     }
@@ -284,13 +285,14 @@ class HostStage {
     used_ = 0;
     return Status::Ok();
   }
-  static bool pinned(const void* p) {
+  // Not plain pageable memory: the host may not be able to read or write it.
+  static bool known(const void* p) {
     hipPointerAttribute_t at;
     if (hipPointerGetAttributes(&at, p) != hipSuccess) {
       (void)hipGetLastError();
       return false;
     }
-    return at.type == hipMemoryTypeHost || at.type == hipMemoryTypeManaged;
+    return at.type != hipMemoryTypeUnregistered;
   }
   char* buf_ = nullptr;
   size_t used_ = 0;  // bytes of the slots that uploads may still be reading
