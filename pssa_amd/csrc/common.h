@@ -298,6 +298,12 @@ class HostStage {
   size_t used_ = 0;  // bytes of the slots that uploads may still be reading
 };
 
+// Orders this wave's LDS writes before its subsequent LDS reads.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // fp32 -> bf16 bits, rounded to nearest even, on gfx950's v_cvt_pk_bf16_f32
 // (one instruction per pair; the same bits as the integer rounding
 // u + 0x7FFF + lsb for every finite value).

@@ -508,6 +508,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_row_kernel(const float*
   if (tid == 64) s_cnt = 0;
   if (gw.hist && wave == 0) {
     read_window(gw, ids[row], row, lane, pen, s_win, s_n);
+    wave_sync();  // a lane's entry is another lane's write
     // Penalised logits of the window ids: each distinct id divided (positive)
     // or multiplied by the penalty once per occurrence.
     const int wn = pen ? __builtin_amdgcn_readfirstlane(s_n) : 0;

@@ -66,12 +66,6 @@ __device__ __forceinline__ float poincare_dist(const float* __restrict__ q, floa
   return (float)(2.0 * rust_asinh(sqrt(sq / den)));
 }
 
-// Orders this wave's LDS writes before its subsequent LDS reads.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 __device__ __forceinline__ float wave_min(float v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v = fminf(v, __shfl_xor(v, off, 64));
