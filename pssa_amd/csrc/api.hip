@@ -1863,7 +1863,8 @@ int pssa_hip_lanes_set_sampling(pssa_hip_lanes* L, float temperature, float top_
     const hipStream_t st = L->ctx->stream;
     if (temperature > 0.0f) {
       if (!L->rng.p) PSSA_RETURN_IF(L->rng.alloc(L->lanes * 8));
-      if (!L->probs.p) PSSA_RETURN_IF(L->probs.alloc(L->lanes * L->model->cfg.d_vocab * 4));
+      if (!L->probs.p && L->model->cfg.d_vocab > (size_t)pssa::kSampleRowMaxV)
+        PSSA_RETURN_IF(L->probs.alloc(L->lanes * L->model->cfg.d_vocab * 4));
       // SimpleRng::new (src/linalg.rs:7-11): every lane starts from `seed`.
       std::vector<uint64_t> st0(L->lanes, seed == 0 ? 0x853c49e6748fea9bULL : seed);
       PSSA_RETURN_IF(L->ctx->stage.to_device(L->rng.p, st0.data(), L->lanes * 8, L->ctx->stream));

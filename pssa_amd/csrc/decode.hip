@@ -193,16 +193,18 @@ __global__ __launch_bounds__(256) void greedy_kernel(const float* __restrict__ l
 // Sampling at temperature > 0 (sample(), src/inference.rs:128-178) for one
 // lane per workgroup, after the same penalty window as greedy_kernel:
 //  - the maximum over ids 1..V-1 of the penalised logits;
-//  - probs[v] = exp((logit - max) / T) into the lane's row (LDS, or a global
-//    scratch row for large vocabularies), the exponential in f64 rounded once
+//  - probs[v] = exp((logit - max) / T), the exponential in f64 rounded once
 //    to f32 (the correctly rounded f32 value; the reference's f32::exp is
 //    within half an ulp plus a hair of it);
-//  - their f32 sum in id order by one thread, as the reference adds them;
-//  - p = probs / sum in place, then the top_k candidates in (probability
-//    desc, id asc) order by top_k rounds of a workgroup arg-max over the
-//    threads' own best candidates;
+//  - their f32 sum in id order, as the reference adds them;
+//  - p = probs / sum, then the top_k candidates in (probability desc, id asc)
+//    order;
 //  - the top_p cut, the mass, one gen_range_f32(0, mass) draw from the lane's
-//    SimpleRng and the running-sum match, in one thread.
+//    SimpleRng and the running-sum match.
+// sample_row_kernel holds the row in registers, up to kSampleRowMaxV ids;
+// sample_kernel, for larger vocabularies, in global scratch, with the sum by
+// one thread and the top_k by rounds of a workgroup arg-max over the threads'
+// own best candidates.
 // The surprise is the raw logits' logsumexp minus the chosen one, computed as
 // greedy_kernel computes it.
 constexpr int kMaxSampleTopK = 64;
@@ -211,7 +213,7 @@ struct SampleArgs {
   float temperature = 0.0f, top_p = 1.0f;
   int top_k = 1;
   unsigned long long* rng = nullptr;  // [lanes] SimpleRng states
-  float* probs = nullptr;             // [lanes, V] scratch
+  float* probs = nullptr;             // [lanes, V] scratch (V > kSampleRowMaxV)
   int* bad_mass = nullptr;            // raised on an invalid probability mass
 };
 
@@ -222,7 +224,7 @@ __device__ __forceinline__ bool ranks_before(float pa, int va, float pb, int vb)
 
 constexpr int kWinBloomWords = 64;  // 2048-bit filter of the penalty window ids
 
-// The general kernel: any vocabulary, the row in global scratch.
+// The general kernel: the row in global scratch.
 __global__ __launch_bounds__(256) void sample_kernel(const float* __restrict__ logits, int V,
                                                      uint32_t* __restrict__ ids,
                                                      uint32_t* __restrict__ gen_ids,
@@ -447,6 +449,7 @@ __global__ __launch_bounds__(256) void sample_kernel(const float* __restrict__ l
 constexpr int kSampleThreads = 1024;
 constexpr int kSampleCand = 512;
 constexpr int kSampleNE = 16, kSampleWideNE = 36;
+static_assert(kSampleThreads * kSampleWideNE == kSampleRowMaxV, "the scratch row's rule");
 
 // x shifted in from the lanes before, 0 where there are none (`CTRL`,
 // `ROWS`: the DPP control and row mask of a wave-wide scan step).
@@ -824,7 +827,7 @@ static Status launch_choice(pssa_hip_lanes* L, size_t n_lanes, const GreedyWindo
     sa.probs = L->probs.as<float>();
     sa.bad_mass = L->nonfinite.as<int>() + 2;
     auto* k = V <= kSampleThreads * kSampleNE       ? &sample_row_kernel<kSampleNE>
-              : V <= kSampleThreads * kSampleWideNE ? &sample_row_kernel<kSampleWideNE>
+              : V <= kSampleRowMaxV                 ? &sample_row_kernel<kSampleWideNE>
                                                     : nullptr;
     if (k)
       k<<<(unsigned)n_lanes, kSampleThreads, 0, st>>>(L->logits.as<float>(), V, L->ids.as<uint32_t>(), gen_ids,

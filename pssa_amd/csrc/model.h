@@ -112,8 +112,8 @@ struct pssa_hip_lanes {
   float graph_penalty = 1.0f;
   // Sampling at temperature > 0 (sample(), src/inference.rs:128-178): the
   // settings (temperature 0: the greedy choice), each lane's SimpleRng state
-  // and the per-lane probability scratch [lanes, V]; the captured step
-  // records the settings it was built with.
+  // and, past kSampleRowMaxV ids, the per-lane probability scratch [lanes, V];
+  // the captured step records the settings it was built with.
   // Recurrent depth loops (set_loops, src/pssa.rs:2171-2184): passes per
   // block and token, each with its own carry ([lanes, depth, loops] matrices of d*s);
   // Xin keeps a looped layer's input rows.
@@ -175,6 +175,8 @@ namespace pssa {
 // (a decode step leaves that to the greedy choice, which appends the token
 // it consumed).
 Status run_prefill(pssa_hip_lanes* L, size_t n_lanes, size_t T, bool taps = false, bool append = true);
+// Vocabularies up to this size are sampled with the row in registers.
+constexpr int kSampleRowMaxV = 36 * 1024;
 // Concurrent lane groups (1 or 2) of a prefill of these lanes.
 int prefill_lane_groups(const pssa_hip_lanes* L, size_t n_lanes, size_t max_len);
 // Lanes of their own lengths (a ragged prefill or training forward), packed

@@ -585,6 +585,32 @@ def test_decode_sampling_at_the_row_kernel_edges(hip, vocab, equal):
     layer.close()
 
 
+@pytest.mark.parametrize("vocab,row", [(36864, False), (36865, True)])
+def test_sampling_takes_a_probability_row_only_past_the_row_kernel(hip, vocab, row):
+    """Device memory taken by set_sampling and a sampled step of 64 lanes: the
+    [lanes, vocab] scratch (9.4 MB) only where the kernel reads it."""
+    import ctypes as C
+
+    say("sampling scratch", vocab)
+    cfg = PSSAConfig(depth=1, d_vocab=vocab, d_latent=64, d_state=16, d_mem_key=8, mem_capacity=16)
+    layer = PSSALayer(hip, ModelWeights.init(cfg, 3, "baseline"), lanes=64, max_tokens=64)
+    ids = np.arange(64, dtype=np.uint32)
+    layer.decode(1, first_ids=ids)
+    rt = C.CDLL("libamdhip64.so")
+
+    def free():
+        f, t = C.c_size_t(0), C.c_size_t(0)
+        assert rt.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    before = free()
+    layer.set_sampling(0.9, 0.97, 24, seed=5)
+    layer.decode(1, first_ids=ids)
+    taken = before - free()
+    layer.close()
+    assert (taken >= 9 << 20) == row and taken < (16 << 20), taken
+
+
 def test_sampling_validation(hip):
     say("decode sampling validation")
     w = small_model(seed=2, depth=1)
