@@ -16,6 +16,8 @@
 // waves' partial sums over j meet in LDS and are added in a fixed order.
 #include "ssm.h"
 
+#include <algorithm>
+
 namespace pssa {
 
 // ---------------------------------------------------------------------------
@@ -707,8 +709,18 @@ constexpr long kScanFullGrid = 768;
 // prefills of 6 lanes x 12 (1152) 0.974 / 1.035 ms, 10 x 24 (1920) 1.10 / 1.17,
 // but 3 x 33 (576) 1.10 / 1.01; up to 64 the line lies between 5 x 50 (960)
 // 1.22 / 1.15 and 16 x 60 (3072) 1.86 / 1.90.
+// Lanes of their own lengths count as whole ones by their rows (each some 32
+// steps longer, its loading of the states): a lane that ends early leaves its
+// CUs to the others, and the longest one's chain is what the pass waits for.
+// Ragged prefills of the 105M model, by the lanes / by the rows: one of 1000
+// with 31 of 5 9.45 / 3.36 ms, with 20 of 100 10.1 / 4.35; 32 spread over 4 to
+// 1024 10.7 / 6.68; 32 over 100 to 700 9.49 / 8.90.
 constexpr int kQuadChannels = 8;
 constexpr long kQuadMax = 1536;
+static long whole_lanes(const SsmArgs& a) {
+  const size_t lane = (size_t)a.T + 32;
+  return (long)std::min<size_t>(a.lanes, (a.rows + 32 * (size_t)a.lanes + lane - 1) / lane);
+}
 static long quad_limit(const SsmArgs& a, bool four_states) {
   if (a.T < 32) return kQuadMax / 2;
   return four_states && !a.concurrent && a.T >= 64 ? 2 * kQuadMax : kQuadMax;
@@ -732,12 +744,12 @@ bool ssm_one_group(int d, int s, size_t lanes, size_t max_len) {
 #endif
 
 // The few-lane scan's grid: kQuadChannels channels and 128 (J = 32) or 64
-// (J = 8) states per workgroup.
+// (J = 8) states per workgroup.  Returns its workgroups for the rule above.
 template <int J>
 static long quad_workgroups(const SsmArgs& a, dim3& grid) {
   constexpr int SB = J == 32 ? 128 : 64;
   grid = dim3((a.d + kQuadChannels - 1) / kQuadChannels, a.lanes, (a.s + SB - 1) / SB);
-  return (long)grid.x * grid.y * grid.z;
+  return (long)grid.x * whole_lanes(a) * grid.z;
 }
 
 template <int J, bool SPANS>

@@ -387,6 +387,37 @@ def test_ragged_rows_equal_single_lanes_bitwise(hip, d_state, dtype, hybrid):
             one.close()
 
 
+@pytest.mark.parametrize("d_state,lens", [
+    (256, [64 + i for i in range(24)]),             # two groups of more rows than the few-lane scan takes
+    (256, [31, 29, 31, 30, 28, 31, 25, 31, 31, 7]),  # one group of short prompts: the eight-wave scan
+    (64, [40 + i % 9 for i in range(24)]),          # eight states a wave lane
+    (300, [50 + i for i in range(13)]),             # three state blocks, summed after the scan
+    (256, [200] + [3 + i for i in range(30)]),      # one long lane among short ones: the few-lane scan
+    (256, [90] * 20 + [1, 2, 3]),
+])
+def test_ragged_scan_kernels_equal_single_lanes_bitwise(hip, d_state, lens):
+    """Ragged batches on both sides of the scan's rules at d_latent 768, against
+    each lane's own prefill: logits and carries, bit for bit."""
+    say("ragged scans", d_state, lens)
+    cfg = PSSAConfig(depth=1, d_vocab=64, d_latent=768, d_state=d_state, d_mem_key=8, mem_capacity=16)
+    w = ModelWeights.init(cfg, 7, "baseline")
+    w.populate_banks(8, count=12)
+    rng = np.random.default_rng(d_state + len(lens))
+    seqs = [rng.integers(0, cfg.d_vocab, n, dtype=np.uint32) for n in lens]
+    layer = PSSALayer(hip, w, lanes=len(lens), max_tokens=sum(lens))
+    one = PSSALayer(hip, w, lanes=1, max_tokens=max(lens))
+    for again in range(2):  # the second time from the first one's carries
+        got, car = layer.prefill_ragged(seqs), layer.get_carry()
+        for i, q in enumerate(seqs):
+            one.reset_recurrent_state()
+            if again:
+                one.prefill_inference(q[None])
+            np.testing.assert_array_equal(one.prefill_inference(q[None])[0], got[i])
+            np.testing.assert_array_equal(one.get_carry()[0], car[i])
+    layer.close()
+    one.close()
+
+
 def test_ragged_stage_times_cover_every_stage(hip):
     """Stage timing of a ragged prefill: each stage a prefill of one length
     spends time in, the head among them, and the same logits as untimed."""
