@@ -29,7 +29,9 @@ namespace pssa {
 // unguarded at clamped columns and masked at their use: under a guard per
 // element each closed its block with a full wait, a memory round trip a step.
 // 3 x 2011 steps of 48: 2.07 -> 0.48 ms; 64 x 2048 of 48 2.46 -> 0.54 (2.3
-// TB/s), of 16 0.575 -> 0.197; 30 x 1000 of 32 0.349 -> 0.161.
+// TB/s), of 16 0.575 -> 0.197; 30 x 1000 of 32 0.349 -> 0.161.  Unaligned rows
+// of 33 states, 1 x 40 steps 27.8 -> 16.2 us (33.0 without SPREAD, whose loads
+// past the end cost what they took), 1 x 700 0.528 -> 0.224 ms.
 template <int TPR>
 __device__ __forceinline__ float row_sum(float v) {
   v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));  // quad_perm 1,0,3,2
@@ -56,9 +58,15 @@ __global__ __launch_bounds__(S * TPR) void dense_scan_kernel(const float* __rest
   const float* brow = Bv + (size_t)seq * L * s + r;
   float* hrow = H + (size_t)seq * L * s + r;
   const bool writes = part == 0 && row < s;
-  const int nv = s - c0;  // columns of this thread in range
+  // Elements of this thread's row slice: neighbouring columns (c0 + e), or
+  // with single loads of several waves every TPR-th one (part + TPR * e), so
+  // that the loads of neighbouring lanes are neighbours (a load instruction of
+  // 33 states touches 17 lines, not 64); h lies in LDS in the same order.
+  constexpr bool SPREAD = !VEC && S * TPR > 64;
+  const int nv = SPREAD ? (s - part + TPR - 1) / TPR : s - c0;  // elements in range
+  auto pos = [](int c) { return SPREAD ? c % TPR * CPT + c / TPR : c; };
 
-  if (tid < S) sh[0][tid] = (tid < s && H0) ? H0[(size_t)seq * s + tid] : 0.0f;
+  if (tid < S) sh[0][pos(tid)] = (tid < s && H0) ? H0[(size_t)seq * s + tid] : 0.0f;
   if (tid < S) sh[1][tid] = 0.0f;
 
   float ring[DEPTH][CPT];
@@ -75,7 +83,7 @@ __global__ __launch_bounds__(S * TPR) void dense_scan_kernel(const float* __rest
       }
     } else {
 #pragma unroll
-      for (int q = 0; q < CPT; ++q) ring[slot][q] = arow[min(c0 + q, s - 1)];
+      for (int q = 0; q < CPT; ++q) ring[slot][q] = arow[min(SPREAD ? part + TPR * q : c0 + q, s - 1)];
     }
     bring[slot] = *brow;
     --left;
@@ -109,7 +117,7 @@ __global__ __launch_bounds__(S * TPR) void dense_scan_kernel(const float* __rest
     }
     const float hv = row_sum<TPR>((p[0] + p[1]) + (p[2] + p[3])) + bring[q];
     if (writes) {
-      sh[cur ^ 1][row] = hv;
+      sh[cur ^ 1][pos(row)] = hv;
       *hrow = hv;
     }
     hrow += s;

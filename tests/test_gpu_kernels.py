@@ -513,6 +513,33 @@ def test_dense_scan_general_kernels_edges(hip, s):
         assert rel_err(hip.dense_scan(a, b, h0), ref) < 100 * (s + 1) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("s", [16, 36, 48, 64])
+def test_dense_scan_of_unaligned_arrays(hip, s):
+    """Device arrays 4 bytes past a 16-byte boundary: single loads, above 32
+    states spread over neighbouring lanes, against the recurrence in f64 (the
+    bound of the test above) and beside the aligned call's result."""
+    B, L = 3, 37
+    say("dense scan unaligned", s)
+    rng = np.random.default_rng(s)
+    q, _ = np.linalg.qr(rng.standard_normal((B, L, s, s)))
+    a = (q * rng.uniform(0.8, 0.99, (B, L, 1, s))).astype(np.float32)
+    b = rng.standard_normal((B, L, s)).astype(np.float32)
+    ref, h = np.empty((B, L, s)), np.zeros((B, s))
+    for t in range(L):
+        h = np.einsum("bij,bj->bi", a[:, t].astype(np.float64), h) + b[:, t]
+        ref[:, t] = h
+    bufs = [hip.empty((x.size + 1,), np.float32) for x in (a, b, b)]
+    for off in (0, 4):
+        bufs[0].write(a, off)
+        bufs[1].write(b, off)
+        hip.dense_scan_resident(bufs[0].ptr + off, bufs[1].ptr + off, None, B, L, s, bufs[2].ptr + off)
+        hip.synchronize()
+        got = bufs[2].to_host()[off // 4:][:b.size].reshape(B, L, s)
+        assert rel_err(got, ref) < 100 * (s + 1) * 2.0 ** -24
+    for x in bufs:
+        x.close()
+
+
 @pytest.mark.parametrize("B,L", [(1, 1), (1, 255), (64, 33), (64, 256), (65, 1), (65, 31), (65, 300)])
 def test_dense_scan_64_states_by_batch_and_length(hip, B, L):
     """d_state 64 on both sides of the rules: below two windows or past 64
