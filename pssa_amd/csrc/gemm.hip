@@ -1111,8 +1111,10 @@ static void launch_skinny_f32_kind(hipStream_t stream, int kind, dim3 grid, cons
 // ---------------------------------------------------------------------------
 // fp32 GEMM of many tiles: 64 x 64 tiles, each of four waves one 32 x 32
 // block, operand slabs of 32 K (128-byte rows) by direct-to-LDS loads through
-// a ring of four slabs (16-byte chunk c of row r at c ^ (r & 7): conflict-free
-// fragment reads).  An fp32 MFMA takes 64 cycles for 32 x 32 x 2, so a small
+// a ring of four slabs (16-byte chunk c of row r at c ^ (r & 7): eight rows'
+// fragments lie in distinct banks, and a read of sixteen takes two turns, half
+// its cycles by the bank-conflict counter; the matrix cores are busy 0.37 of
+// the time at 1000 x 1536 x 768).  An fp32 MFMA takes 64 cycles for 32 x 32 x 2, so a small
 // tile already keeps the matrix cores fed from LDS (16 KB per 1024 cycles and
 // CU) and the many tiles fill the CUs evenly: a 128 x 128 tile is eight such
 // blocks in a row per wave, and one wave per 32 x 32 tile straight from
@@ -1506,7 +1508,8 @@ Status launch_gemm(hipStream_t stream, int dtype, const void* A, int lda, const 
   // against 8.1), or where K is no multiple of 16, which the one-wave tiles
   // need.  Old / new: 512 x 1056 x 128 9.4 / 8.8 us, 200 x 2096 x 768 29.4 /
   // 22.5, 1000 x 1536 x 768 39.8 / 36.6, 4001 x 768 x 400 70.1 / 34.4, 16384 x
-  // 768 x 128 52.3 / 50.9, 77 x 1536 x 1544 234 / 38.7.
+  // 768 x 128 52.3 / 50.9, 77 x 1536 x 1544 234 / 38.7, 32768 x 2096 x 768 1188 /
+  // 1147, 32768 x 768 x 1536 969 / 815, 4096 x 4096 x 4096 1411 / 1423.
   const long tiles64 = (long)((M + F32_T - 1) / F32_T) * ((N + F32_T - 1) / F32_T);
   if (!bf16 && vec_load && K % 8 == 0 && (tiles64 >= 96 || K % 16 != 0) && tiles64 <= INT32_MAX) {
     launch_f32_lds_kind(stream, ep.kind, (unsigned)tiles64, static_cast<const float*>(A), lda,
