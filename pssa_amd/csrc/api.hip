@@ -776,24 +776,30 @@ int pssa_hip_memory_forward_after_ssm(pssa_hip_ctx* ctx, const float* x_norm, co
 
 }  // extern "C"
 
+// Grows the context's scratch to `bytes`.  Called with ctx->mu held; the
+// previous buffer is released only once the stream has drained.  Where the
+// caller can do without (`optional`) it stays when there is no memory.
+static Status grow_scratch(pssa_hip_ctx* ctx, size_t bytes, bool optional) {
+  if (ctx->scratch_bytes >= bytes) return Status::Ok();
+  PSSA_HIP_TRY(hipStreamSynchronize(ctx->stream));
+  void* p = nullptr;
+  if (optional && pssa::device_malloc(&p, bytes) != hipSuccess) return Status::Ok();
+  if (ctx->scratch) PSSA_HIP_TRY(hipFree(ctx->scratch));
+  ctx->scratch = nullptr;
+  ctx->scratch_bytes = 0;
+  if (!p) PSSA_HIP_TRY(pssa::device_malloc(&p, bytes));
+  ctx->scratch = p;
+  ctx->scratch_bytes = bytes;
+  return Status::Ok();
+}
+
 // Points ra.scratch at the context's scratch, grown to what the launch needs.
-// Called with ctx->mu held; the previous buffer is released only once the
-// stream has drained.  A full soft read runs without where there is no memory.
+// Called with ctx->mu held.  A full soft read runs without where there is no
+// memory.
 static Status bind_retrieve_scratch(pssa_hip_ctx* ctx, pssa::RetrieveArgs& ra) {
   const size_t need_bytes = pssa::retrieve_scratch_bytes(ra);
   if (!need_bytes) return Status::Ok();
-  if (ctx->scratch_bytes < need_bytes) {
-    PSSA_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (ctx->scratch) PSSA_HIP_TRY(hipFree(ctx->scratch));
-    ctx->scratch = nullptr;
-    ctx->scratch_bytes = 0;
-    const hipError_t e = pssa::device_malloc(&ctx->scratch, need_bytes);
-    if (e != hipSuccess) {
-      if (!pssa::retrieve_needs_scratch(ra)) return Status::Ok();
-      return Status::Device("retrieve scratch (" + std::to_string(need_bytes) + " bytes): " + hipGetErrorString(e));
-    }
-    ctx->scratch_bytes = need_bytes;
-  }
+  PSSA_RETURN_IF(grow_scratch(ctx, need_bytes, !pssa::retrieve_needs_scratch(ra)));
   ra.scratch = ctx->scratch;
   ra.scratch_bytes = ctx->scratch_bytes;
   return Status::Ok();
@@ -802,15 +808,7 @@ static Status bind_retrieve_scratch(pssa_hip_ctx* ctx, pssa::RetrieveArgs& ra) {
 // Grows the context's scratch to what the two-level dense scan needs.
 // Called with ctx->mu held.
 static Status bind_dense_scan_scratch(pssa_hip_ctx* ctx, int batch, int L, int s) {
-  const size_t need_bytes = pssa::dense_scan_scratch_bytes(batch, L, s);
-  if (!need_bytes || ctx->scratch_bytes >= need_bytes) return Status::Ok();
-  PSSA_HIP_TRY(hipStreamSynchronize(ctx->stream));
-  if (ctx->scratch) PSSA_HIP_TRY(hipFree(ctx->scratch));
-  ctx->scratch = nullptr;
-  ctx->scratch_bytes = 0;
-  PSSA_HIP_TRY(pssa::device_malloc(&ctx->scratch, need_bytes));
-  ctx->scratch_bytes = need_bytes;
-  return Status::Ok();
+  return grow_scratch(ctx, pssa::dense_scan_scratch_bytes(batch, L, s), false);
 }
 
 extern "C" {

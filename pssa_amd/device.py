@@ -265,8 +265,8 @@ class HipDevice:
                                   out_val_ptr: int, out_min_ptr: int | None = None,
                                   out_idx_ptr: int | None = None) -> None:
         """retrieve_resident with no device allocation: the exact top-k path's
-        scratch is the device's static array (shared by every call on the GPU;
-        overlapping calls race)."""
+        scratch is the device's static array (shared by every top-k call on
+        the GPU; overlapping ones race)."""
         vp = C.c_void_p
         _abi.call(self._lib.pssa_hip_retrieve_resident_noalloc, self.handle, vp(q_ptr), n_q, vp(keys_ptr),
                   vp(norm_sq_ptr), vp(values_ptr), capacity, count, d_key, d_val, tau, top_k, vp(out_val_ptr),
