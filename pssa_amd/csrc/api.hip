@@ -60,8 +60,7 @@ Status upload_weight(pssa_hip_ctx* ctx, DevBuf& dst, const float* src, size_t n,
 }
 
 Status sync(pssa_hip_ctx* ctx) {
-  PSSA_HIP_TRY(hipStreamSynchronize(ctx->stream));
-  return Status::Ok();
+  return ctx->stage.wait(ctx->stream);
 }
 
 Status need(bool cond, const char* msg) { return cond ? Status::Ok() : Status::Invalid(msg); }

@@ -78,11 +78,11 @@ inline Status checked_count(std::initializer_list<size_t> dims, size_t* out, con
 }
 
 // Device blocks kept between calls for the temporaries of the host-array
-// entry points (each hipMalloc / hipFree pair costs about 20 us, and a call
-// takes up to fifteen).  Blocks are handed out again on the context's one
-// stream, so a block's next user runs after its last; at most kPoolBytes are
-// held, the rest is freed at once, and all of it with the context or when an
-// allocation of any context finds no memory (device_malloc).
+// entry points (a call takes up to fifteen; a hipMalloc / hipFree pair of 6 MB
+// costs 23 us, of up to 1 MiB 1.3).  Blocks are handed out again on the
+// context's one stream, so a block's next user runs after its last; at most
+// kPoolBytes are held, the rest is freed at once, and all of it with the
+// context or when an allocation of any context finds no memory (device_malloc).
 class DevPool {
  public:
   static constexpr size_t kPoolBytes = (size_t)256 << 20;
@@ -248,7 +248,7 @@ class HostStage {
   Status to_device(void* dst, const void* src, size_t n, hipStream_t st) {
     if (!n) return Status::Ok();
     if (n >= kMin && n < kSlot && !known(src)) {
-      if (used_ + n > kSlot * kSlots) PSSA_RETURN_IF(drain(st));
+      if (used_ + n > kSlot * kSlots) PSSA_RETURN_IF(wait(st));
       std::memcpy(buf_ + used_, src, n);
       src = buf_ + used_;
       used_ += (n + 255) & ~(size_t)255;
@@ -256,14 +256,14 @@ class HostStage {
     PSSA_HIP_TRY(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st));
     return Status::Ok();
   }
-  // The data is in `dst` at return (after all earlier work of the stream).
+  // The data is in `dst` once the stream is waited for.
   Status to_host(void* dst, const void* src, size_t n, hipStream_t st) {
     if (!n) return Status::Ok();
     if (n < kMin || known(dst)) {
       PSSA_HIP_TRY(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st));
-      return drain(st);
+      return Status::Ok();  // no wait of its own: some microseconds of a small call
     }
-    PSSA_RETURN_IF(drain(st));
+    PSSA_RETURN_IF(wait(st));
     auto piece = [&](size_t off) { return n - off < kSlot ? n - off : kSlot; };
     auto issue = [&](size_t off) {
       return hipMemcpyAsync(buf_ + off / kSlot % 2 * kSlot, static_cast<const char*>(src) + off, piece(off),
@@ -277,14 +277,14 @@ class HostStage {
     }
     return Status::Ok();
   }
-
- private:
-  // Every transfer out of or into the slots has ended.
-  Status drain(hipStream_t st) {
+  // Waits for the stream; every transfer out of or into the slots has ended.
+  Status wait(hipStream_t st) {
     PSSA_HIP_TRY(hipStreamSynchronize(st));
     used_ = 0;
     return Status::Ok();
   }
+
+ private:
   // Not plain pageable memory: the host may not be able to read or write it.
   static bool known(const void* p) {
     hipPointerAttribute_t at;

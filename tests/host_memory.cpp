@@ -124,7 +124,7 @@ static void copies() {
       std::fill(src.begin(), src.end(), 0xEE);  // reused at once
     }
     std::vector<unsigned char> back(n);
-    check(st.to_host(back.data(), dst[8].data(), n, nullptr).ok(), "to_host");
+    check(st.to_host(back.data(), dst[8].data(), n, nullptr).ok() && st.wait(nullptr).ok(), "to_host");
     bool same = back == dst[8];
     for (size_t r = 0; r < dst.size(); ++r)
       for (size_t i = 0; i < n; ++i) same &= dst[r][i] == (unsigned char)(i * 7 + i / 251 + r);
@@ -134,7 +134,9 @@ static void copies() {
     std::vector<char> a(n, 1), b(n, 2);
     g_device = a.data();
     g_direct.clear();
-    check(st.to_device(b.data(), a.data(), n, nullptr).ok() && st.to_host(a.data(), b.data(), n, nullptr).ok(), "copies");
+    check(st.to_device(b.data(), a.data(), n, nullptr).ok() && st.to_host(a.data(), b.data(), n, nullptr).ok() &&
+              st.wait(nullptr).ok(),
+          "copies");
     check(g_direct.size() == 2 && std::get<1>(g_direct[0]) == a.data() && std::get<2>(g_direct[0]) == n &&
               std::get<0>(g_direct[1]) == a.data() && std::get<2>(g_direct[1]) == n,
           ("a device array of " + std::to_string(n) + " bytes is copied by the runtime alone").c_str());
